@@ -81,6 +81,8 @@ struct GemmArgs {
   // skinny kernel: write the partial product to ws even when K is not split
   // (the split-K entry points of one range, K <= 16)
   int to_ws;
+  // tiled split kernel: the two-piece form may be tried (set by the host)
+  int fast;
 };
 
 // the value stored at C[m][n] of batch b from the product's value v
@@ -415,39 +417,40 @@ __global__ __launch_bounds__(kGT) void gemm_f32_kernel(const GemmArgs g) {
 // v_mfma_f32_16x16x4_f32 (16 x 32 cycles): 2.7x the fp32 matrix rate.
 // Non-finite inputs give NaN (x - x0 is Inf - Inf).
 //
-// Tiling: 256 threads = 4 waves in a 2x2 grid, block tile 128 x 128 x 16,
-// wave tile 64 x 64 = 2 x 2 MFMA tiles of 32 x 32.  The next k-tile is
-// fetched into registers while the current one is multiplied out of LDS.
+//
+// Two fp16 pieces do the same in three products where the values' range
+// allows (h2 below), and this form stays as what those tiles fall back to and
+// for short products.
+//
 // An operand contiguous along k is staged as [piece][row][k] (rows of 16
 // bf16, the two 16-byte chunks swapped on rows 8..15 mod 16) and read with
 // ds_read_b128; an operand contiguous along its rows (m or n) as
-// [piece][k][row] (rows of 160 bf16) and read with gfx950's transposing
-// ds_read_b64_tr_b16, so staging never transposes in registers.  Both
-// layouts are free of LDS bank conflicts (SQ_LDS_BANK_CONFLICT = 0).  MFMA 32x32x16 operands: lane l holds row l%32 and
-// k = 8(l/32) + 0..7; accumulator element e of lane l is
-// C[8(e/4) + 4(l/32) + e%4][l%32].
+// [piece][k][row] (rows of R + pad bf16, a stride of 16 or 48 banks mod 64)
+// and read with gfx950's transposing ds_read_b64_tr_b16, so staging never
+// transposes in registers.  Both layouts are free of LDS bank conflicts.
+// MFMA 32x32x16 operands: lane l holds row l%32 and k = 8(l/32) + 0..7;
+// accumulator element e of lane l is C[8(e/4) + 4(l/32) + e%4][l%32].
 // ---------------------------------------------------------------------------
-#ifndef MTX_X3_XCD
-#define MTX_X3_XCD 1
-#endif
 namespace x3 {
-constexpr int T = 128;             // tile rows and columns
-constexpr int BK = 16;             // k-tile depth (one MFMA k step)
-constexpr int LDK = BK;            // row stride (bf16) of a k-contiguous plane
-constexpr int LDR = T + 32;        // row stride (bf16) of a row-contiguous plane
+constexpr int T = 128;  // tile rows and columns
+constexpr int BK = 16;  // k-tile depth (one MFMA k step)
 // k-contiguous rows hold two 16-byte chunks, swapped on rows 8..15 mod 16:
 // a fragment read's 16 rows then cover 16 distinct 16-byte bank groups and
 // a staging store's 8 rows x 4 quarters 32 distinct 8-byte ones
 __device__ __forceinline__ int kswz(int row) { return ((row >> 3) & 1) * 8; }
-constexpr int NV = T * BK / 4 / kGT;  // float4 per thread per operand tile
 }  // namespace x3
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
+// two bf16 values in a register; opaque to the compiler, which otherwise
+// converts the low one a second time to shift it out of the pair
 __device__ __forceinline__ uint32_t pk_bf16(float x, float y) {
   bf16x2 v = {(__bf16)x, (__bf16)y};
-  return __builtin_bit_cast(uint32_t, v);
+  uint32_t u = __builtin_bit_cast(uint32_t, v);
+  asm("" : "+v"(u));
+  return u;
 }
 
 // x = h + m + l (+ 2^-24 |x|), for four values, each plane as four bf16
@@ -466,47 +469,55 @@ __device__ __forceinline__ void split3(f32x4 v, uint2& h, uint2& m, uint2& l) {
   l.y = pk_bf16(r2, r3);
 }
 
-// One operand's 128 x 16 tile (rows = m for A, n for B).  KC: contiguous
-// along k in global memory (rows strided by srow); else contiguous along the
-// rows (k strided by sk).  Thread slot i covers, KC: row idx/4, k 4(idx%4)..+3;
-// else: k idx/32, rows 4(idx%32)..+3 (idx = tid + 256 i).
-template <bool KC>
+// One operand's R x 16 tile (rows = m for A, n for B).  KC: contiguous along
+// k in global memory (rows strided by srow); else contiguous along the rows
+// (k strided by sk).  The tile is R*4 float4 vectors; slot i of a thread is
+// vector idx = tid + 256 i: KC: row idx/4, k 4(idx%4)..+3; else: k idx/(R/4),
+// rows 4(idx%(R/4))..+3.  Where 256 does not divide R*4 the threads past the
+// end repeat the vector 128 before (the same values to the same place).
+template <bool KC, int R>
 struct X3Stage {
-  static constexpr int PS = KC ? x3::T * x3::LDK : x3::BK * x3::LDR;  // plane size (bf16)
-  const float* __restrict__ base;
+  static constexpr int NV = (R * 4 + kGT - 1) / kGT;  // float4 per thread
+  static constexpr int NVEC = R * 4;
+  static_assert(NVEC % kGT == 0 || NVEC % kGT == 128, "tile rows");
+  // k-plane row stride (bf16): 16 or 48 banks mod 64
+  static constexpr int LDR = (R / 2) % 64 == 16 || (R / 2) % 64 == 48 ? R : R + 32;
+  static_assert((LDR / 2) % 64 == 16 || (LDR / 2) % 64 == 48, "bank stride");
+  static constexpr int PS = KC ? R * x3::BK : x3::BK * LDR;  // plane size (bf16)
+  const float* __restrict__ base;  // the operand at (row r0, k 0)
   int64_t srow, sk;
   int rows, r0;
-  int64_t off[x3::NV];
-  f32x4 r[x3::NV];
+  int lput[NV];  // LDS offsets (bf16) of this thread's vectors
 
+  __device__ __forceinline__ int vec(int i, int tid) const {
+    const int idx = tid + i * kGT;
+    return idx < NVEC ? idx : idx - 128;
+  }
   __device__ __forceinline__ void init(const float* b, int64_t s_row, int64_t s_k, int nrows, int row0, int tid) {
-    base = b;
     srow = s_row;
     sk = s_k;
     rows = nrows;
     r0 = row0;
+    base = b + (int64_t)r0 * srow;
 #pragma unroll
-    for (int i = 0; i < x3::NV; ++i) {
-      const int idx = tid + i * kGT;
-      off[i] = KC ? (int64_t)(r0 + idx / 4) * srow + 4 * (idx % 4) : (int64_t)(idx / 32) * sk + r0 + 4 * (idx % 32);
+    for (int i = 0; i < NV; ++i) {
+      const int idx = vec(i, tid);
+      if constexpr (KC) {
+        lput[i] = (idx / 4) * x3::BK + ((4 * (idx % 4)) ^ x3::kswz(idx / 4));
+      } else {
+        lput[i] = (idx / (R / 4)) * LDR + 4 * (idx % (R / 4));
+      }
     }
   }
-  // every row of the tile and every k of [k0, k0+16) in range, float4
-  // loads aligned (checked by the caller)
-  __device__ __forceinline__ void fetch_fast(int k0) {
-#pragma unroll
-    for (int i = 0; i < x3::NV; ++i)
-      r[i] = *reinterpret_cast<const f32x4*>(base + off[i] + (int64_t)k0 * (KC ? 1 : sk));
-  }
   // rows past `rows` and k past kend read as zero; unaligned vectors by element
-  __device__ __forceinline__ void fetch_checked(int k0, int kend, int tid) {
+  __device__ __forceinline__ void fetch_checked(f32x4 (&r)[NV], int k0, int kend, int tid) const {
 #pragma unroll
-    for (int i = 0; i < x3::NV; ++i) {
-      const int idx = tid + i * kGT;
+    for (int i = 0; i < NV; ++i) {
+      const int idx = vec(i, tid);
       f32x4 v = {0.f, 0.f, 0.f, 0.f};
       if constexpr (KC) {
-        const int row = r0 + idx / 4, k = k0 + 4 * (idx % 4);
-        if (row < rows) {
+        const int row = idx / 4, k = k0 + 4 * (idx % 4);
+        if (r0 + row < rows) {
           const float* p = base + (int64_t)row * srow + k;
           if (k + 3 < kend && (((uintptr_t)p) & 15u) == 0) {
             v = *reinterpret_cast<const f32x4*>(p);
@@ -517,58 +528,55 @@ struct X3Stage {
           }
         }
       } else {
-        const int k = k0 + idx / 32, row = r0 + 4 * (idx % 32);
+        const int k = k0 + idx / (R / 4), row = 4 * (idx % (R / 4));
         if (k < kend) {
           const float* p = base + (int64_t)k * sk + row;
-          if (row + 3 < rows && (((uintptr_t)p) & 15u) == 0) {
+          if (r0 + row + 3 < rows && (((uintptr_t)p) & 15u) == 0) {
             v = *reinterpret_cast<const f32x4*>(p);
           } else {
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-              if (row + j < rows) v[j] = p[j];
+              if (r0 + row + j < rows) v[j] = p[j];
           }
         }
       }
       r[i] = v;
     }
   }
-  __device__ __forceinline__ void put(__bf16* __restrict__ lds, int tid) const {
+  __device__ __forceinline__ void put(__bf16* __restrict__ lds, const f32x4 (&r)[NV]) const {
 #pragma unroll
-    for (int i = 0; i < x3::NV; ++i) {
-      const int idx = tid + i * kGT;
-      const int o = KC ? (idx / 4) * x3::LDK + ((4 * (idx % 4)) ^ x3::kswz(idx / 4))
-                       : (idx / 32) * x3::LDR + 4 * (idx % 32);
+    for (int i = 0; i < NV; ++i) {
       uint2 h, m, l;
       split3(r[i], h, m, l);
-      *reinterpret_cast<uint2*>(lds + o) = h;
-      *reinterpret_cast<uint2*>(lds + PS + o) = m;
-      *reinterpret_cast<uint2*>(lds + 2 * PS + o) = l;
+      *reinterpret_cast<uint2*>(lds + lput[i]) = h;
+      *reinterpret_cast<uint2*>(lds + PS + lput[i]) = m;
+      *reinterpret_cast<uint2*>(lds + 2 * PS + lput[i]) = l;
     }
   }
   // piece p's MFMA operand for tile rows rb .. rb+31: lane l gets row
   // rb + l%32 and k = 8(l/32) + 0..7
-  __device__ __forceinline__ bf16x8 frag(const __bf16* __restrict__ lds, int p, int rb, int lane) const {
+  __device__ __forceinline__ static bf16x8 frag(const __bf16* __restrict__ lds, int p, int rb, int lane) {
     if constexpr (KC) {
       const int row = rb + (lane & 31);
-      return *reinterpret_cast<const bf16x8*>(lds + p * PS + row * x3::LDK + ((8 * (lane >> 5)) ^ x3::kswz(row)));
+      return *reinterpret_cast<const bf16x8*>(lds + p * PS + row * x3::BK + ((8 * (lane >> 5)) ^ x3::kswz(row)));
     } else {
       // transposing read: in each 16-lane group G, lane j = 4i + q addresses
       // k row 8(G/2) + i (+4 for the second half) at rows rb + 16(G%2) + 4q;
       // lane j then receives row rb + 16(G%2) + j at those four k
       const int G = lane >> 4, j = lane & 15;
-      const __bf16* p0 = lds + p * PS + (8 * (G >> 1) + (j >> 2)) * x3::LDR + rb + 16 * (G & 1) + 4 * (j & 3);
+      const __bf16* p0 = lds + p * PS + (8 * (G >> 1) + (j >> 2)) * LDR + rb + 16 * (G & 1) + 4 * (j & 3);
       const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p0);
-      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + 4 * x3::LDR));
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + 4 * LDR));
       const uint2 ul = __builtin_bit_cast(uint2, lo), uh = __builtin_bit_cast(uint2, hi);
       return __builtin_bit_cast(bf16x8, make_uint4(ul.x, ul.y, uh.x, uh.y));
     }
   }
   // ACT 3 column sums: this thread's share of the staged B values, by
   // column (KC: the 4 k of slot i belong to column idx/4; else slot i holds
-  // columns 4(idx%32)..+3, the same for every slot)
-  __device__ __forceinline__ void colsum_add(float (&cs)[4]) const {
+  // columns 4(idx%(R/4))..+3, the same for every slot; R = 128)
+  __device__ __forceinline__ static void colsum_add(float (&cs)[4], const f32x4 (&r)[NV]) {
 #pragma unroll
-    for (int i = 0; i < x3::NV; ++i) {
+    for (int i = 0; i < NV; ++i) {
       if constexpr (KC) {
         cs[i] += (r[i][0] + r[i][1]) + (r[i][2] + r[i][3]);
       } else {
@@ -579,159 +587,546 @@ struct X3Stage {
   }
 };
 
-template <bool AK, bool BN1, int ACT>
-__global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
-  using SA = X3Stage<AK>;
-  using SB = X3Stage<!BN1>;  // B^T: rows = n, contiguous along k iff !BN1
-  // the operand planes, reused by the epilogue for half the C tile (64 x 128 fp32)
-  constexpr int kAB = 3 * (SA::PS + SB::PS) * 2, kEp = 64 * x3::T * 4;
-  __shared__ __attribute__((aligned(16))) char smem[kAB > kEp ? kAB : kEp];
-  __bf16* As = reinterpret_cast<__bf16*>(smem);
-  __bf16* Bs = As + 3 * SA::PS;
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wid = tid >> 6;
-  const int wm = (wid >> 1) * 64, wn = (wid & 1) * 64;
-#if MTX_X3_XCD
-  // Workgroups are dealt round-robin over the 8 XCDs in dispatch order;
-  // give each XCD a contiguous run of row-major tiles, so the column tiles
-  // that share an A row panel read it through the same L2
-  int tx = blockIdx.x, ty = blockIdx.y, tz = blockIdx.z;
-  {
-    const int nt = gridDim.x * gridDim.y * gridDim.z;
-    if ((nt & 7) == 0) {
-      const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-      const int t = (lin & 7) * (nt >> 3) + (lin >> 3);
-      tx = t % gridDim.x;
-      ty = (t / gridDim.x) % gridDim.y;
-      tz = t / (gridDim.x * gridDim.y);
+// ---------------------------------------------------------------------------
+// fp32 products from two fp16 pieces of every value, three products each.
+//
+// A row of A (a column of B) is scaled by a power of two s, then every value
+// x is split while its tile is staged into LDS: h = fp16(s x) and
+// l = fp16(2^14 (s x - h)), both rounded to nearest, so that s x = h +
+// 2^-14 l with an error of at most 2^-23 |s x|, or 2^-39 where that is more.
+// C is (sum ah bh + 2^-14 sum (al bh + ah bl)) / (sa sb): the cross terms
+// have accumulators of their own, and the dropped al bl weighs at most
+// 2^-24 |ab|.  Three v_mfma_f32_32x32x16_f16 do the work of the three-piece
+// split's six bf16 ones, and the main accumulator is rounded once per k step
+// instead of six times, which is most of a long product's error: against
+// float64 the products of the 384-wide model's training step are off by
+// 0.5-0.6 of what the three-piece form gave (K = 384: 6.2e-8 against 1.1e-7
+// relative; K = 1536: 2.6e-7 against 6.0e-7).
+//
+// The scale comes from 32 of the row's values, spread evenly over its k range
+// (the beginning alone says too little: in the gradient of a packed q/k/v
+// projection a first token's row starts with the query's, which is 0 up to
+// rounding).  Their largest goes to [2^-4, 2^-3), so the error above is 2^-35
+// of it for small values, and other values may be 2^17 times larger before l
+// overflows (65504).  A row without a nonzero sample gets the largest scale,
+// which any value above 2^-99 overflows; a largest sample outside 2^-60 ..
+// 2^60 or not finite gives a scale of Inf.  An overflow leaves Inf or NaN in
+// the accumulators of its whole row or column, so one look at them after the
+// k loop finds it, and the workgroup then computes its tile again from three
+// bf16 pieces (X3Stage), whose range is fp32's.
+//
+// Tiling: 256 threads = 4 waves; a wave owns MI x NI MFMA tiles of 32 x 32
+// and the waves form a WM x WN grid, so the block tile is 32 MI WM x 32 NI
+// WN, and 32 deep.  Pipeline: two LDS buffers and one barrier per k step.
+// While the products of step t run out of one buffer, the wave splits the
+// values of step t + 1 (in registers since the step before) into the other
+// buffer and requests those of step t + 2 into the registers as they come
+// free: each MFMA occupies the matrix pipe for 32 cycles and the issue port
+// for 4, and the split's vector instructions are placed into the gaps
+// (sched_group_barrier).  4096^3: 793 -> 465 us (173 -> 295 TFLOP/s, the
+// three-piece kernel before); 16384 x 384 x 1536: 130 -> 94; its weight
+// gradient 137 -> 104; 16384 x 1152 x 384, where a tile's beginning and end
+// weigh as much as its 12 steps, 106 -> 104.
+// ---------------------------------------------------------------------------
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+namespace h2 {
+constexpr int BK = 32;  // k-tile depth: a row's 32 floats are one 128-byte line
+// From K = 256 on the error is no larger than the three-piece form's (of a
+// shorter product the split's own 6e-8 is most)
+constexpr int MINK = 256;
+
+// the scale times 2^14 of a row whose largest |sample| has these bits, and the reciprocal of the scale itself
+__device__ __forceinline__ float scale2(uint32_t amax) {
+  const int e = (int)(amax >> 23);
+  if (amax == 0) return __uint_as_float(254u << 23);
+  if (e < 127 - 60 || e > 127 + 60) return __uint_as_float(0x7f800000u);
+  return __uint_as_float((uint32_t)(127 + 127 + 14 - 4 - e) << 23);
+}
+__device__ __forceinline__ float unscale(uint32_t amax) {
+  const int e = (int)(amax >> 23);
+  if (amax == 0) return __uint_as_float(14u << 23);
+  return __uint_as_float((uint32_t)(e + 4) << 23);
+}
+// x2 = 2^14 s x of four values -> h and l, four fp16 each: two mixed-precision
+// multiply-adds a value (zero is a 0 that the compiler cannot see, and the
+// pairs are opaque to it: it would otherwise convert every h twice)
+__device__ __forceinline__ uint32_t pair_h(float x, float y, float zero) {
+  f16x2 h = {(_Float16)__builtin_fmaf(x, 0x1p-14f, zero), (_Float16)__builtin_fmaf(y, 0x1p-14f, zero)};
+  uint32_t u = __builtin_bit_cast(uint32_t, h);
+  asm("" : "+v"(u));
+  return u;
+}
+__device__ __forceinline__ uint32_t pair_l(uint32_t hu, float x, float y) {
+  const f16x2 h = __builtin_bit_cast(f16x2, hu);
+  f16x2 l = {(_Float16)__builtin_fmaf((float)h[0], -16384.f, x), (_Float16)__builtin_fmaf((float)h[1], -16384.f, y)};
+  return __builtin_bit_cast(uint32_t, l);
+}
+__device__ __forceinline__ void split(f32x4 x2, float zero, uint2& h, uint2& l) {
+  h.x = pair_h(x2[0], x2[1], zero);
+  h.y = pair_h(x2[2], x2[3], zero);
+  l.x = pair_l(h.x, x2[0], x2[1]);
+  l.y = pair_l(h.y, x2[2], x2[3]);
+}
+}  // namespace h2
+
+// One operand's R x 32 tile (rows = m for A, n for B), R = 96 or 128.  KC:
+// contiguous along k in global memory (rows strided by srow); else contiguous
+// along the rows (k strided by sk).  Slot i of a thread is the float4 vector
+// idx = tid + 256 i: KC: row idx/8, k 4(idx%8)..+3; else: k idx/(R/4), rows
+// 4(idx%(R/4))..+3.
+// LDS planes.  KC: [row][32 k], rows of 64 bytes, the four 16-byte chunks
+// permuted by (row/4)%4, so the 16 rows of a fragment read's quarter cover
+// all 64 banks.  Else [k][R rows]: the transposing read takes 32 bytes of
+// four consecutive k rows per 16 lanes; R = 96 (48 banks a row) spreads them
+// by itself, R = 128 permutes the four 64-byte blocks of a row by k%4.
+template <bool KC, int R>
+struct H2Stage {
+  static_assert(R == 96 || R == 128, "tile rows");
+  static constexpr int NV = R * h2::BK / 4 / kGT;    // float4 per thread
+  static constexpr int PS = R * h2::BK;              // plane size (fp16)
+  static constexpr int NSC = KC ? NV : R == 128 ? 4 : 4 * NV;  // scales a thread needs
+  const char* base;   // the operand at (row r0, k 0)
+  int64_t kstep;      // bytes per k
+  int64_t last;       // bytes from base to the operand's end
+  uint32_t voff[NV];  // this thread's byte offsets in a k-tile
+  int lput;           // LDS offset (fp16) of slot 0; slot i adds a constant
+  int lputs[R == 96 && !KC ? NV : 1];
+  float sc[NSC];
+
+  __device__ __forceinline__ void init(const float* b, int64_t srow, int64_t sk, int rows, int K, int r0, int tid) {
+    base = reinterpret_cast<const char*>(b + (int64_t)r0 * srow);
+    kstep = sk * 4;
+    last = ((int64_t)(rows - 1 - r0) * srow + (int64_t)(K - 1) * sk + 1) * 4;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + i * kGT;
+      if constexpr (KC) voff[i] = (uint32_t)(idx / 8) * (uint32_t)(srow * 4) + 16 * (idx % 8);
+      else voff[i] = (uint32_t)(idx / (R / 4)) * (uint32_t)(sk * 4) + 16 * (idx % (R / 4));
+    }
+    if constexpr (KC) {
+      const int row = tid / 8, c = (tid % 8) / 2;
+      lput = row * h2::BK + 8 * (c ^ ((row >> 2) & 3)) + 4 * (tid & 1);
+    } else if constexpr (R == 128) {
+      const int k = tid / 32, c = 4 * (tid % 32);
+      lput = k * R + (c ^ (32 * (k & 3)));
+    } else {
+#pragma unroll
+      for (int i = 0; i < NV; ++i) lputs[i] = (tid + i * kGT) * 4;
     }
   }
-  const int m0 = ty * x3::T, n0 = tx * x3::T;
-  const int zb = tz;
-#else
-  const int m0 = blockIdx.y * x3::T, n0 = blockIdx.x * x3::T;
-  const int zb = blockIdx.z;
-#endif
+  __device__ __forceinline__ int put_at(int i) const {
+    if constexpr (KC) return lput + i * 32 * h2::BK;      // 32 rows on: the same permutation
+    else if constexpr (R == 128) return lput + i * 8 * R;  // 8 k on
+    else return lputs[i];
+  }
+  // The k-tile at k0 through a buffer resource based at its first value and
+  // ending at the operand's last: no per-lane address arithmetic, and rows
+  // past the operand's end read as zeros.  (A vector reaching past a row's
+  // last value takes what follows it in memory, which the caller allows for
+  // rows only: their products land in rows or columns of C that are not
+  // stored.)
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile(int k0) const {
+    const int64_t off = (int64_t)k0 * kstep, left = last - off;
+    const unsigned bytes = left > 0x7ffffff0ll ? 0x7ffffff0u : left > 0 ? (unsigned)left : 0u;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base + off), (short)0, (int)bytes, 0x00020000);
+  }
+  __device__ __forceinline__ f32x4 fetch(__amdgpu_buffer_rsrc_t rs, int i) const {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)voff[i], 0, 0));
+  }
+  // the same by element where a vector may reach past the last row or kend
+  __device__ __forceinline__ f32x4 fetch_checked(int k0, int kend, int nrows, int64_t srow, int i, int tid) const {
+    const int idx = tid + i * kGT;
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    const float* p = reinterpret_cast<const float*>(base);
+    if constexpr (KC) {
+      const int row = idx / 8, k = k0 + 4 * (idx % 8);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (row < nrows && k + j < kend) v[j] = p[(int64_t)row * srow + k + j];
+    } else {
+      const int k = k0 + idx / (R / 4), row = 4 * (idx % (R / 4));
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (k < kend && row + j < nrows) v[j] = p[(int64_t)k * (kstep / 4) + row + j];
+    }
+    return v;
+  }
+  // 32 values of each row, spread evenly over the n k (n >= 256) from kbeg on:
+  // KC: 8 vectors n/8 apart; else k rows n/32 apart
+  __device__ __forceinline__ void sample(f32x4 (&r)[NV], int kbeg, int n, uint32_t sstep, int tid) const {
+    const __amdgpu_buffer_rsrc_t rs = tile(kbeg);
+    const uint32_t far = KC ? (uint32_t)(n / 32) * 16u : (uint32_t)(n / 32) * sstep;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + i * kGT;
+      const uint32_t off = KC ? (uint32_t)(idx / 8) * sstep + (uint32_t)(idx % 8) * far
+                              : (uint32_t)(idx / (R / 4)) * far + 16 * (idx % (R / 4));
+      r[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
+    }
+  }
+  // amax[row] = the largest of each row's samples (as bits); it is zero before
+  __device__ __forceinline__ void row_max(const f32x4 (&r)[NV], uint32_t* amax, int tid) const {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + i * kGT;
+      if constexpr (KC) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m = max(m, __float_as_uint(r[i][j]) & 0x7fffffffu);
+        m = max(m, (uint32_t)__shfl_xor((int)m, 1));
+        m = max(m, (uint32_t)__shfl_xor((int)m, 2));
+        m = max(m, (uint32_t)__shfl_xor((int)m, 4));
+        if ((tid & 7) == 0) amax[idx / 8] = m;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          atomicMax(&amax[4 * (idx % (R / 4)) + j], __float_as_uint(r[i][j]) & 0x7fffffffu);
+      }
+    }
+  }
+  __device__ __forceinline__ void scales(const uint32_t* amax, int tid) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int idx = tid + i * kGT;
+      if constexpr (KC) {
+        sc[i] = h2::scale2(amax[idx / 8]);
+      } else if (R != 128 || i == 0) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) sc[4 * i + j] = h2::scale2(amax[4 * (idx % (R / 4)) + j]);
+      }
+    }
+  }
+  __device__ __forceinline__ void put(_Float16* __restrict__ lds, f32x4 r, float zero, int i) const {
+    f32x4 x2;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x2[j] = r[j] * sc[KC ? i : R == 128 ? j : 4 * i + j];
+    uint2 h, l;
+    h2::split(x2, zero, h, l);
+    *reinterpret_cast<uint2*>(lds + put_at(i)) = h;
+    *reinterpret_cast<uint2*>(lds + PS + put_at(i)) = l;
+  }
+  // piece p's MFMA operand for k 16 sub .. +15 of tile rows rb .. rb+31: lane
+  // l gets row rb + l%32 and k = 16 sub + 8(l/32) + 0..7
+  __device__ __forceinline__ static f16x8 frag(const _Float16* __restrict__ lds, int p, int sub, int rb, int lane) {
+    if constexpr (KC) {
+      const int row = rb + (lane & 31);
+      return *reinterpret_cast<const f16x8*>(lds + p * PS + row * h2::BK +
+                                             8 * ((2 * sub + (lane >> 5)) ^ ((row >> 2) & 3)));
+    } else {
+      // transposing read, as X3Stage::frag
+      const int G = lane >> 4, j = lane & 15;
+      const int k = 16 * sub + 8 * (G >> 1) + (j >> 2);
+      int c = rb + 16 * (G & 1) + 4 * (j & 3);
+      if constexpr (R == 128) c ^= 32 * (k & 3);
+      const _Float16* p0 = lds + p * PS + k * R + c;
+      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p0);
+      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + 4 * R));
+      const uint2 ul = __builtin_bit_cast(uint2, lo), uh = __builtin_bit_cast(uint2, hi);
+      return __builtin_bit_cast(f16x8, make_uint4(ul.x, ul.y, uh.x, uh.y));
+    }
+  }
+};
+
+template <int MI, int NI, int WM, int WN, bool AK, bool BN1, int ACT>
+__global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
+  static_assert(WM * WN == 4, "four waves");
+  constexpr int BM = 32 * MI * WM, BN = 32 * NI * WN;
+  using SA = H2Stage<AK, BM>;
+  using SB = H2Stage<!BN1, BN>;  // B^T: rows = n, contiguous along k iff !BN1
+  using XA = X3Stage<AK, BM>;
+  using XB = X3Stage<!BN1, BN>;
+  constexpr int kBuf = 2 * (SA::PS + SB::PS);  // one stage's planes (fp16)
+  constexpr int EW = 32 * NI + 8;              // row stride of the epilogue's 16-row strips (floats)
+  constexpr int kEp = 4 * 16 * EW * 4;
+  constexpr int kX3 = 3 * (XA::PS + XB::PS) * 2;
+  constexpr int kTiles = 2 * kBuf * 2;
+  static_assert(kTiles >= kEp && kTiles >= kX3 && kTiles >= 8 * BN * 4, "LDS");
+  __shared__ __attribute__((aligned(16))) char smem[kTiles];
+  __shared__ uint32_t amax[BM + BN];  // rows' and columns' largest sample
+  __shared__ int again;
+  _Float16* buf0 = reinterpret_cast<_Float16*>(smem);
+  _Float16* buf1 = buf0 + kBuf;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = (wid / WN) * 32 * MI, wn = (wid % WN) * 32 * NI;
+  // Workgroups are dealt round-robin over the 8 XCDs in dispatch order; give
+  // each XCD a contiguous run of row-major tiles, so the column tiles that
+  // share an A row panel read it through the same L2
+  int tx, ty, zb;
+  {
+    const int nt = gridDim.x * gridDim.y * gridDim.z;
+    const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const int xcd = lin & 7, per = nt >> 3, more = nt & 7;
+    const int t = xcd * per + min(xcd, more) + (lin >> 3);
+    tx = t % gridDim.x;
+    ty = (t / gridDim.x) % gridDim.y;
+    zb = t / (gridDim.x * gridDim.y);
+  }
+  const int m0 = ty * BM, n0 = tx * BN;
   const int bidx = zb % g.batch, split = zb / g.batch;
   const int kbeg = split * g.kchunk;
   const int kend = min(g.K, kbeg + g.kchunk);
+  const float* A = g.a + (int64_t)bidx * g.sab;
+  const float* B = g.b + (int64_t)bidx * g.sbb;
 
-  SA sa;
-  SB sb;
-  sa.init(g.a + (int64_t)bidx * g.sab, g.sam, g.sak, g.M, m0, tid);
-  sb.init(g.b + (int64_t)bidx * g.sbb, g.sbn, g.sbk, g.N, n0, tid);
-  const bool interior = g.vec_ok && m0 + x3::T <= g.M && n0 + x3::T <= g.N;
+  f32x16 acc[MI][NI], accx[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = accx[i][j][e] = 0.f;
+  // ACT 3: column sums of B from the values each thread stages
+  float cs[SB::NV][4];
+#pragma unroll
+  for (int i = 0; i < SB::NV; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) cs[i][j] = 0.f;
+  const bool two = g.fast && kend - kbeg >= h2::MINK;  // the two-piece form is tried
+  bool scaled = false;                                 // acc, accx hold its sums
 
-  f32x16 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-  // ACT 3: the first row of tiles sums the B columns it stages
-  const bool cs_block = ACT == 3 && m0 == 0;
-  float cs[4] = {0.f, 0.f, 0.f, 0.f};
+  if (two) {
+    SA sa;
+    SB sb;
+    sa.init(A, g.sam, g.sak, g.M, g.K, m0, tid);
+    sb.init(B, g.sbn, g.sbk, g.N, g.K, n0, tid);
+    for (int i = tid; i < BM + BN; i += kGT) amax[i] = 0;
+    if (tid == 0) again = 0;
+    const int steps = (kend - kbeg + h2::BK - 1) / h2::BK;
+    // The k steps that the unchecked loads take: whole ones, and (where the
+    // rows of an operand contiguous along them do not end on a vector) not
+    // the operand's last, whose last vectors reach past its end.
+    int whole = (kend - kbeg) / h2::BK;
+    if (((!AK && (g.M & 3)) || (BN1 && (g.N & 3))) && kend == g.K && whole == steps) --whole;
 
-  // one k-tile: stage the fetched values, request the next tile (pref),
-  // multiply out of LDS
-  auto tile = [&](auto&& pref) {
-    __syncthreads();
-    sa.put(As, tid);
-    sb.put(Bs, tid);
-    if constexpr (ACT == 3) {
-      if (cs_block) sb.colsum_add(cs);
-    }
-    __syncthreads();
-    pref();
-    bf16x8 a[3][2], b[3][2];
+    f32x4 ra[SA::NV], rb[SB::NV];
+    auto fetch_any = [&](int t) {
+      const int k0 = kbeg + t * h2::BK;
+      if (t < whole) {
+        const auto ta = sa.tile(k0), tb = sb.tile(k0);
 #pragma unroll
-    for (int p = 0; p < 3; ++p)
+        for (int i = 0; i < SA::NV; ++i) ra[i] = sa.fetch(ta, i);
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        a[p][i] = sa.frag(As, p, wm + 32 * i, lane);
-        b[p][i] = sb.frag(Bs, p, wn + 32 * i, lane);
-      }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        f32x16 c = acc[i][j];
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2][i], b[0][j], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[1][j], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[2][j], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[0][j], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[1][j], c, 0, 0, 0);
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[0][j], c, 0, 0, 0);
-        acc[i][j] = c;
-      }
-  };
-  auto checked_next = [&](int kn) {
-    if (kn < kend) {
-      sa.fetch_checked(kn, kend, tid);
-      sb.fetch_checked(kn, kend, tid);
-    }
-  };
-  int k0 = kbeg;
-  if (interior) {
-    // whole k-tiles through the unchecked loads in a branch-free loop; the
-    // last whole tile and a ragged tail after it
-    const int kfull = kbeg + (kend - kbeg) / x3::BK * x3::BK;
-    if (k0 < kfull) {
-      sa.fetch_fast(k0);
-      sb.fetch_fast(k0);
-    } else {
-      checked_next(k0);
-    }
-    for (; k0 + x3::BK < kfull; k0 += x3::BK)
-      tile([&] {
-        sa.fetch_fast(k0 + x3::BK);
-        sb.fetch_fast(k0 + x3::BK);
-      });
-  } else {
-    checked_next(k0);
-  }
-  for (; k0 < kend; k0 += x3::BK) tile([&] { checked_next(k0 + x3::BK); });
-
-  if constexpr (ACT == 3) {
-    // reduce the per-thread column sums through LDS (As is free after the
-    // barrier): KC: 4 threads per column, else 8 threads per 4 columns;
-    // contributors are added in a fixed order
-    if (cs_block) {
-      float* red = reinterpret_cast<float*>(As);  // [8][128]
-      __syncthreads();
-      if constexpr (!BN1) {
-#pragma unroll
-        for (int i = 0; i < x3::NV; ++i) {
-          const int idx = tid + i * kGT;
-          red[(idx % 4) * x3::T + idx / 4] = cs[i];
-        }
+        for (int i = 0; i < SB::NV; ++i) rb[i] = sb.fetch(tb, i);
       } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) red[(tid / 32) * x3::T + 4 * (tid % 32) + j] = cs[j];
+        for (int i = 0; i < SA::NV; ++i) ra[i] = sa.fetch_checked(k0, kend, g.M - m0, g.sam, i, tid);
+#pragma unroll
+        for (int i = 0; i < SB::NV; ++i) rb[i] = sb.fetch_checked(k0, kend, g.N - n0, g.sbn, i, tid);
+      }
+    };
+    auto colsum = [&] {
+      if constexpr (ACT == 3) {
+#pragma unroll
+        for (int i = 0; i < SB::NV; ++i) {
+          if constexpr (!BN1) cs[i][0] += (rb[i][0] + rb[i][1]) + (rb[i][2] + rb[i][3]);
+          else
+#pragma unroll
+            for (int j = 0; j < 4; ++j) cs[BN == 128 ? 0 : i][j] += rb[i][j];
+        }
+      }
+    };
+    float zero = 0.f;
+    asm("" : "+s"(zero));
+    // The products of one step, MFMA by MFMA: half a step (sub) at a time the
+    // four fragments' three products.  fa, fb: [sub][piece][tile].
+    constexpr int kT = MI * NI, kM = 6 * kT;
+    f16x8 fa[2][2][MI], fb[2][2][NI];
+    auto read_frags = [&](const _Float16* cur, int sub) {
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) fa[sub][p][i] = SA::frag(cur, p, sub, wm + 32 * i, lane);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) fb[sub][p][j] = SB::frag(cur + 2 * SA::PS, p, sub, wn + 32 * j, lane);
+      }
+    };
+    auto product = [&](int q) {
+      const int sub = q / (3 * kT), kind = q / kT % 3, i = q % kT / NI, j = q % NI;
+      if (kind == 0) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][0][i], fb[sub][0][j], acc[i][j], 0, 0, 0);
+      else if (kind == 1)
+        accx[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][1][i], fb[sub][0][j], accx[i][j], 0, 0, 0);
+      else accx[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][0][i], fb[sub][1][j], accx[i][j], 0, 0, 0);
+    };
+    // One step: its products in as many groups as there are vectors to stage
+    // (kS); beside each group's products one vector of the next step is split
+    // and stored, and its register refilled with the step after's.
+    constexpr int kS = SA::NV + SB::NV;
+    auto step = [&](const _Float16* cur, _Float16* nxt, int t2) {
+      const int k0 = kbeg + t2 * h2::BK;
+      const auto ta = sa.tile(k0), tb = sb.tile(k0);
+      read_frags(cur, 0);
+      colsum();
+#pragma unroll
+      for (int c = 0; c < kS; ++c) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (c == 1) read_frags(cur, 1);
+#pragma unroll
+        for (int q = c * kM / kS; q < (c + 1) * kM / kS; ++q) product(q);
+        if (c < SA::NV) {
+          sa.put(nxt, ra[c], zero, c);
+          ra[c] = sa.fetch(ta, c);
+        } else {
+          sb.put(nxt + 2 * SA::PS, rb[c - SA::NV], zero, c - SA::NV);
+          rb[c - SA::NV] = sb.fetch(tb, c - SA::NV);
+        }
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          if (c == 1) __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        }
       }
       __syncthreads();
-      if (tid < x3::T) {
-        constexpr int NC = BN1 ? 8 : 4;
-        float v = 0.f;
+    };
+    auto put_all = [&](_Float16* nxt) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) v += red[c * x3::T + tid];
+      for (int i = 0; i < SA::NV; ++i) sa.put(nxt, ra[i], zero, i);
+#pragma unroll
+      for (int i = 0; i < SB::NV; ++i) sb.put(nxt + 2 * SA::PS, rb[i], zero, i);
+    };
+
+    {
+      f32x4 qa[SA::NV], qb[SB::NV];
+      sa.sample(qa, kbeg, kend - kbeg, (uint32_t)(AK ? g.sam : g.sak) * 4u, tid);
+      sb.sample(qb, kbeg, kend - kbeg, (uint32_t)(BN1 ? g.sbk : g.sbn) * 4u, tid);
+      fetch_any(0);
+      __syncthreads();
+      sa.row_max(qa, amax, tid);
+      sb.row_max(qb, amax + BM, tid);
+    }
+    __syncthreads();
+    sa.scales(amax, tid);
+    sb.scales(amax + BM, tid);
+    colsum();
+    put_all(buf0);
+    if (steps > 1) fetch_any(1);
+    __syncthreads();
+    int t = 0;
+    for (; t + 3 < whole; t += 2) {
+      step(buf0, buf1, t + 2);
+      step(buf1, buf0, t + 3);
+    }
+    for (; t < steps; ++t) {  // t is even at first; the last step has nothing to stage
+      read_frags((t & 1) ? buf1 : buf0, 0);
+      read_frags((t & 1) ? buf1 : buf0, 1);
+#pragma unroll
+      for (int q = 0; q < kM; ++q) product(q);
+      if (t + 1 < steps) {
+        colsum();
+        put_all((t & 1) ? buf0 : buf1);
+        if (t + 2 < steps) fetch_any(t + 2);
+      }
+      __syncthreads();
+    }
+    // Inf or NaN in a row or column of the tile: every row of the wave's
+    // tile in its first column, every column in its first row
+    float z = 0.f;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) z += 0.f * acc[i][0][e] + 0.f * accx[i][0][e];
+#pragma unroll
+    for (int j = 1; j < NI; ++j) z += 0.f * acc[0][j][0] + 0.f * accx[0][j][0];
+    if (!(z == 0.f)) again = 1;  // any lane
+    __syncthreads();
+    scaled = again == 0;
+  }
+
+  if (!scaled) {
+    XA xa;
+    XB xb;
+    xa.init(A, g.sam, g.sak, g.M, m0, tid);
+    xb.init(B, g.sbn, g.sbk, g.N, n0, tid);
+    __bf16* As = reinterpret_cast<__bf16*>(smem);
+    __bf16* Bs = As + 3 * XA::PS;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+    const bool sums = ACT == 3 && !two;  // else they are there already
+    f32x4 ra[XA::NV], rb[XB::NV];
+    xa.fetch_checked(ra, kbeg, kend, tid);
+    xb.fetch_checked(rb, kbeg, kend, tid);
+    for (int k0 = kbeg; k0 < kend; k0 += x3::BK) {
+      __syncthreads();
+      xa.put(As, ra);
+      xb.put(Bs, rb);
+      if (sums) XB::colsum_add(cs[0], rb);
+      __syncthreads();
+      if (k0 + x3::BK < kend) {
+        xa.fetch_checked(ra, k0 + x3::BK, kend, tid);
+        xb.fetch_checked(rb, k0 + x3::BK, kend, tid);
+      }
+      bf16x8 a[3][MI], b[3][NI];
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i) a[p][i] = XA::frag(As, p, wm + 32 * i, lane);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) b[p][j] = XB::frag(Bs, p, wn + 32 * j, lane);
+      }
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          f32x16 c = acc[i][j];
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2][i], b[0][j], c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[1][j], c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[2][j], c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[0][j], c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[1][j], c, 0, 0, 0);
+          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[0][j], c, 0, 0, 0);
+          acc[i][j] = c;
+        }
+    }
+    __syncthreads();
+  }
+
+  if constexpr (ACT == 3) {
+    // the first row of tiles reduces the per-thread column sums through LDS:
+    // KC: 8 (three pieces: 4) threads per column, else 8 threads per 4 columns; contributors
+    // are added in a fixed order
+    static_assert(BN == 128, "column sums");
+    if (m0 == 0) {
+      float* red = reinterpret_cast<float*>(smem);  // [8][BN]
+#pragma unroll
+      for (int i = 0; i < SB::NV; ++i) {
+        if constexpr (!BN1) {
+          const int idx = tid + i * kGT;
+          if (two) red[(idx % 8) * BN + idx / 8] = cs[i][0];
+          else if (i < XB::NV) red[(idx % 4) * BN + idx / 4] = cs[0][i];
+        } else if (i == 0) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) red[(tid / 32) * BN + 4 * (tid % 32) + j] = cs[0][j];
+        }
+      }
+      __syncthreads();
+      if (tid < BN) {
+        const int NC = BN1 || two ? 8 : 4;
+        float v = 0.f;
+        for (int c = 0; c < NC; ++c) v += red[c * BN + tid];
         const int n = n0 + tid;
         if (n < g.N) {
           if (g.ksplit > 1) g.ws[(int64_t)g.ksplit * g.M * g.N + (int64_t)split * g.N + n] = v;
           else g.colsum[n] = g.colsum_acc ? g.colsum[n] + v : v;
         }
       }
+      __syncthreads();
     }
   }
 
-  // Epilogue, in two halves of 64 rows: the waves put acc[half] into LDS
-  // (row r of the half holds tile row 64(r/32) + 32 half + r%32; columns
-  // XOR-permuted by 32 on rows 4..7 mod 8, so the two rows a store
-  // instruction writes use disjoint banks), then each thread finishes float4
-  // runs of C rows: coalesced loads and stores, no per-element addresses.
-  // acc[i][j][e] = tile element (wm + 32i + 8(e/4) + 4(lane/32) + e%4, wn + 32j + lane%32).
-  float* ep = reinterpret_cast<float*>(smem);
+  // Epilogue, each wave on its own (no barriers): strips of 16 rows of the
+  // wave's tile go through the wave's own LDS (elements 8 half .. +7 of one
+  // row of MFMA tiles; rows of EW floats, so the two rows a store instruction
+  // writes use disjoint banks), then each lane finishes float4 runs of C
+  // rows: coalesced loads and stores, no per-element addresses.
+  // acc[i][j][e] = wave tile element (32i + 8(e/4) + 4(lane/32) + e%4, 32j + lane%32).
+  float* ep = reinterpret_cast<float*>(smem) + wid * 16 * EW;
   const int lr = lane & 31, lh = lane >> 5;
   const bool to_ws = g.ksplit > 1;
   float* W = g.ws + ((int64_t)split * g.batch + bidx) * (int64_t)g.M * g.N;
@@ -744,76 +1139,84 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
                           : (g.scn == 1 && g.scm % 4 == 0 && g.scb % 4 == 0 && (((uintptr_t)g.c) & 15u) == 0 &&
                              (!use_x || (g.sxn == 1 && g.sxm % 4 == 0 && g.sxb % 4 == 0 &&
                                          (((uintptr_t)g.aux) & 15u) == 0)));
+  float unB[NI];  // of this lane's columns
 #pragma unroll
-  for (int half = 0; half < 2; ++half) {
-    __syncthreads();
+  for (int j = 0; j < NI; ++j) unB[j] = scaled ? h2::unscale(amax[BM + wn + 32 * j + lr]) : 1.f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+  for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int r = (wm >> 1) + 8 * (e >> 2) + 4 * lh + (e & 3);
-        ep[r * x3::T + ((wn + 32 * j + lr) ^ ((r & 4) << 3))] = acc[half][j][e];
-      }
-    __syncthreads();
+    for (int half = 0; half < 2; ++half) {
+      __builtin_amdgcn_wave_barrier();
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int r = 8 * (e >> 2) + 4 * lh + (e & 3);
+          float v = acc[i][j][8 * half + e];
+          if (scaled)
+            v = __builtin_fmaf(accx[i][j][8 * half + e], 0x1p-14f, v) * h2::unscale(amax[wm + 32 * i + 16 * half + r]) * unB[j];
+          ep[r * EW + 32 * j + lr] = v;
+        }
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll 2
-    for (int q = 0; q < 8; ++q) {
-      const int idx = tid + q * kGT;
-      const int r = idx >> 5, c = 4 * (idx & 31);
-      const int m = m0 + 64 * (r >> 5) + 32 * half + (r & 31);
-      const int n = n0 + c;
-      if (m >= g.M || n >= g.N) continue;
-      const f32x4 a4 = *reinterpret_cast<const f32x4*>(ep + r * x3::T + (c ^ ((r & 4) << 3)));
-      const int nv = min(4, g.N - n);
-      if (to_ws) {
-        float* w = W + (int64_t)m * g.N + n;
-        if (cvec && nv == 4) {
-          *reinterpret_cast<f32x4*>(w) = a4;
+      for (int q = 0; q < 2 * NI; ++q) {
+        const int idx = lane + q * 64;
+        const int r = idx / (8 * NI), c = 4 * (idx % (8 * NI));
+        const int m = m0 + wm + 32 * i + 16 * half + r;
+        const int n = n0 + wn + c;
+        const f32x4 a4 = *reinterpret_cast<const f32x4*>(ep + r * EW + c);
+        if (m >= g.M || n >= g.N) continue;
+        const int nv = min(4, g.N - n);
+        if (to_ws) {
+          float* w = W + (int64_t)m * g.N + n;
+          if (cvec && nv == 4) {
+            *reinterpret_cast<f32x4*>(w) = a4;
+          } else {
+            for (int u = 0; u < nv; ++u) w[u] = a4[u];
+          }
+          continue;
+        }
+        float* cp = Cp + (int64_t)m * g.scm + (int64_t)n * g.scn;
+        float* xp = X + (int64_t)m * g.sxm + (int64_t)n * g.sxn;
+        f32x4 v, old = {0.f, 0.f, 0.f, 0.f}, xa = {0.f, 0.f, 0.f, 0.f}, bv = {0.f, 0.f, 0.f, 0.f};
+        const bool vecs = cvec && nv == 4;
+        if (vecs) {
+          if (rd_c) old = *reinterpret_cast<const f32x4*>(cp);
+          if constexpr (ACT == 2 || ACT == 4) xa = *reinterpret_cast<const f32x4*>(xp);
         } else {
-          for (int t = 0; t < nv; ++t) w[t] = a4[t];
+          for (int u = 0; u < nv; ++u) {
+            if (rd_c) old[u] = cp[(int64_t)u * g.scn];
+            if constexpr (ACT == 2 || ACT == 4) xa[u] = xp[(int64_t)u * g.sxn];
+          }
         }
-        continue;
-      }
-      float* cp = Cp + (int64_t)m * g.scm + (int64_t)n * g.scn;
-      float* xp = X + (int64_t)m * g.sxm + (int64_t)n * g.sxn;
-      f32x4 v, old = {0.f, 0.f, 0.f, 0.f}, xa = {0.f, 0.f, 0.f, 0.f}, bv = {0.f, 0.f, 0.f, 0.f};
-      const bool vec = cvec && nv == 4;
-      if (vec) {
-        if (rd_c) old = *reinterpret_cast<const f32x4*>(cp);
-        if constexpr (ACT == 2 || ACT == 4) xa = *reinterpret_cast<const f32x4*>(xp);
-      } else {
-        for (int t = 0; t < nv; ++t) {
-          if (rd_c) old[t] = cp[(int64_t)t * g.scn];
-          if constexpr (ACT == 2 || ACT == 4) xa[t] = xp[(int64_t)t * g.sxn];
-        }
-      }
-      if (g.bias) {
-        for (int t = 0; t < nv; ++t) bv[t] = g.bias[n + t];
-      }
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        float u = g.alpha * a4[t] + bv[t];
-        if (rd_c) u += g.beta * old[t];
-        v[t] = u;
-      }
-      if constexpr (ACT == 1) {
-        if (g.aux) {
-          if (vec) *reinterpret_cast<f32x4*>(xp) = v;
-          else
-            for (int t = 0; t < nv; ++t) xp[(int64_t)t * g.sxn] = v[t];
+        if (g.bias) {
+          for (int u = 0; u < nv; ++u) bv[u] = g.bias[n + u];
         }
 #pragma unroll
-        for (int t = 0; t < 4; ++t) v[t] = gelu_tanh_fast(v[t]);
-      } else if constexpr (ACT == 2) {
+        for (int u = 0; u < 4; ++u) {
+          float w = g.alpha * a4[u] + bv[u];
+          if (rd_c) w += g.beta * old[u];
+          v[u] = w;
+        }
+        if constexpr (ACT == 1) {
+          if (g.aux) {
+            if (vecs) *reinterpret_cast<f32x4*>(xp) = v;
+            else
+              for (int u = 0; u < nv; ++u) xp[(int64_t)u * g.sxn] = v[u];
+          }
 #pragma unroll
-        for (int t = 0; t < 4; ++t) v[t] *= gelu_grad_fast(xa[t]);
-      } else if constexpr (ACT == 4) {
-        v += xa;
+          for (int u = 0; u < 4; ++u) v[u] = gelu_tanh_fast(v[u]);
+        } else if constexpr (ACT == 2) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] *= gelu_grad_fast(xa[u]);
+        } else if constexpr (ACT == 4) {
+          v += xa;
+        }
+        if (vecs) *reinterpret_cast<f32x4*>(cp) = v;
+        else
+          for (int u = 0; u < nv; ++u) cp[(int64_t)u * g.scn] = v[u];
       }
-      if (vec) *reinterpret_cast<f32x4*>(cp) = v;
-      else
-        for (int t = 0; t < nv; ++t) cp[(int64_t)t * g.scn] = v[t];
     }
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1182,20 +1585,30 @@ Plan plan_x3(int M, int N, int K, int batch, size_t ws_bytes) {
     want = std::min(want, std::max(1, K / MTX_SPLIT_MINK));
     const size_t need = (size_t)want * batch * (size_t)(M + 1) * N * sizeof(float);
     if (want > 1 && need <= ws_bytes) {
-      p.kchunk = cdiv(cdiv(K, want), x3::BK) * x3::BK;
+      p.kchunk = cdiv(cdiv(K, want), h2::BK) * h2::BK;
       p.ksplit = cdiv(K, p.kchunk);
     }
   }
   return p;
 }
 
+// Whether the two-piece form may be tried (the kernel leaves it to K ranges of
+// h2::MINK or more): 32-bit offsets reach a tile's rows and its samples' k rows.
+bool two_pieces(const GemmArgs& g) {
+  const int64_t lim = (int64_t)1 << 29;
+  auto ok = [&](int64_t s_row, int64_t s_k) {
+    return s_row >= 0 && s_k >= 0 && (s_k == 1 ? 128 * s_row + g.kchunk : g.kchunk * s_k + 128) < lim;
+  };
+  return ok(g.sam, g.sak) && ok(g.sbn, g.sbk);
+}
+
 template <int ACT>
 void launch_x3_act(const GemmArgs& g, bool ak, bool bn1, hipStream_t st) {
   const dim3 grid(cdiv(g.N, x3::T), cdiv(g.M, x3::T), g.batch * g.ksplit);
-  if (ak && bn1) hipLaunchKernelGGL((gemm_x3_kernel<true, true, ACT>), grid, dim3(kGT), 0, st, g);
-  else if (ak) hipLaunchKernelGGL((gemm_x3_kernel<true, false, ACT>), grid, dim3(kGT), 0, st, g);
-  else if (bn1) hipLaunchKernelGGL((gemm_x3_kernel<false, true, ACT>), grid, dim3(kGT), 0, st, g);
-  else hipLaunchKernelGGL((gemm_x3_kernel<false, false, ACT>), grid, dim3(kGT), 0, st, g);
+  if (ak && bn1) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, true, true, ACT>), grid, dim3(kGT), 0, st, g);
+  else if (ak) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, true, false, ACT>), grid, dim3(kGT), 0, st, g);
+  else if (bn1) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, false, true, ACT>), grid, dim3(kGT), 0, st, g);
+  else hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, false, false, ACT>), grid, dim3(kGT), 0, st, g);
 }
 
 // as launch_tile: with split K the reduce kernel applies the activation
@@ -1311,6 +1724,7 @@ int gemm_impl(int M, int N, int K, int batch, float alpha, const float* a, int64
                   : plan_gemm(M, N, K, batch, workspace ? workspace_bytes : 0);
   g.ksplit = p.ksplit;
   g.kchunk = p.kchunk;
+  g.fast = split3 && two_pieces(g);
   int rc = split3 ? launch_x3(g, ak, bn1, st)
                   : (p.bm == 128) ? launch_tile<128, 128>(g, ak, bn1, st) : launch_tile<64, 64>(g, ak, bn1, st);
   if (rc) return rc;

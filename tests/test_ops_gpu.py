@@ -658,6 +658,52 @@ def test_gemm_nonfinite_and_near_overflow(dev, gemm_mode):
         assert np.all(np.isnan(c[0])) and np.all(np.isnan(c[1]))
 
 
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("values", ["plain", "late", "far", "tiny", "zero_start", "range"])
+@pytest.mark.parametrize("M,N,K", [(512, 4096, 256), (4101, 1003, 290), (391, 515, 2085)])
+def test_gemm_two_piece_scaling(dev, M, N, K, values, ta, tb):
+    """Split products of K >= 256 scale every row of A and column of B by its
+    values in the first 32 k; here those say little about the rest: rows and
+    columns whose later values are 2^14 times larger ("late", inside the
+    scaled form's range) or 2^30 times ("far", outside: the tile is computed
+    again from three pieces), rows of 1e-25 ("tiny", outside), rows and columns
+    that begin with 40 zeros ("zero_start") and rows spread over 2^40
+    ("range").  Odd sizes: no aligned vectors, ragged tiles on every side.
+    Bound: a value is held to 2^-23 of itself or 2^-35 of its row's largest
+    beginning value; 2^-20 of sum |a||b| covers that of both operands and the
+    fp32 accumulation (the three pieces: 2^-23 of |ab|, six sums a k step)."""
+    from minitorch_amd import kernels as Kn
+
+    _say(f"[gemm scaling] M={M} N={N} K={K} {values} ta={ta} tb={tb}")
+    rng = np.random.default_rng(M + N + K)
+    a = rng.standard_normal((M, K), dtype=np.float32)
+    b = rng.standard_normal((K, N), dtype=np.float32)
+    if values in ("late", "far"):
+        f = np.float32(2.0 ** (14 if values == "late" else 30))
+        a[3::50, 200] *= f
+        b[201, 5::60] *= f
+    elif values == "tiny":
+        a[7::40] *= np.float32(1e-25)
+    elif values == "zero_start":
+        a[1::30, :40] = 0
+        b[:40, 2::70] = 0
+        a[5] = 0
+        b[:, 9] = 0
+    elif values == "range":
+        a *= (2.0 ** rng.integers(-20, 21, (M, 1))).astype(np.float32)
+        b *= (2.0 ** rng.integers(-20, 21, (1, N))).astype(np.float32)
+    ta_ = T(np.ascontiguousarray(a.T)).transpose(0, 1) if ta else T(a)
+    tb_ = T(np.ascontiguousarray(b.T)).transpose(0, 1) if tb else T(b)
+    c = empty((M, N))
+    Kn.gemm(ta_, tb_, c)
+    ad, bd = a.astype(np.float64), b.astype(np.float64)
+    err = np.abs(H(c) - ad @ bd)
+    aa, ab = np.abs(ad), np.abs(bd)
+    lim = 2.0 ** -20 * (aa @ ab) + 2.0 ** -35 * (aa[:, :32].max(1, keepdims=True) * ab.sum(0)
+                                                 + aa.sum(1, keepdims=True) * ab[:32].max(0)) + 1e-37
+    assert np.all(err <= lim), (err.max(), (err / lim).max())
+
+
 def test_failed_capture_releases_its_pool(dev):
     """A capture that fails at mtx_graph_end (invalidated by synchronising
     the capturing stream) releases its memory pool: a block freed into that
