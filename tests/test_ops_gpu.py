@@ -136,6 +136,34 @@ def test_reduce_sum(dev, shape, axes):
     close(H(out).reshape(np.shape(ref)), ref, atol=dot_tol(R), name="reduce")
 
 
+@pytest.mark.parametrize("rows,n,pad", [(1, 256, 0), (1, 16384, 0), (1, 1000003, 1), (3, 70001, 3), (200, 257, 0),
+                                        (5, 4099, 2), (1, 6291456, 0)])
+def test_reduce_contiguous_runs(dev, rows, n, pad):
+    """Sum and max over the last axis (runs of 256 and more take the kernel of
+    their own), rows starting at any 4-byte address, accumulated into an
+    output; the sum twice gives the same bits."""
+    from minitorch_amd import _lib as L
+    from minitorch_amd import kernels as Kn
+
+    _say(f"[reduce runs] {rows} x {n} + {pad}")
+    rng = np.random.default_rng(n)
+    a = rng.standard_normal((rows, n + pad), dtype=np.float32)
+    ta = T(a)[:, pad:]
+    base = rng.standard_normal(rows, dtype=np.float32)
+    got = []
+    for _ in range(2):
+        out = T(base)
+        Kn.reduce(ta, [1], out, alpha=0.5, accumulate=True)
+        got.append(H(out))
+    x = a[:, pad:].astype(np.float64)
+    # every value passes through at most log2(n) + 48 rounded sums of a chunk
+    assert np.all(np.abs(got[0] - (base + 0.5 * x.sum(1))) <= 2.0 ** -24 * 70 * np.abs(x).sum(1))
+    assert np.array_equal(got[0], got[1])
+    mx = empty((rows,))
+    Kn.reduce(ta, [1], mx, op=L.RED_MAX)
+    assert np.array_equal(H(mx), a[:, pad:].max(1))
+
+
 def test_reduce_merged_dims_bit_identical(dev):
     """Reducing (B, T, C) over (B, T) merges the two reduced dims into one of
     B*T rows; the result must be bit-identical to reducing the (B*T, C) view,
