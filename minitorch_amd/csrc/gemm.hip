@@ -81,8 +81,9 @@ struct GemmArgs {
   // skinny kernel: write the partial product to ws even when K is not split
   // (the split-K entry points of one range, K <= 16)
   int to_ws;
-  // tiled split kernel: the two-piece form may be tried (set by the host)
-  int fast;
+  // tiled split kernel (set by the host): the two-piece form may be tried; C's
+  // (or the partials') and aux's rows have unit stride and do not overlap
+  int fast, rows_vec;
 };
 
 // the value stored at C[m][n] of batch b from the product's value v
@@ -623,10 +624,15 @@ struct X3Stage {
 // buffer and requests those of step t + 2 into the registers as they come
 // free: each MFMA occupies the matrix pipe for 32 cycles and the issue port
 // for 4, and the split's vector instructions are placed into the gaps
-// (sched_group_barrier).  4096^3: 793 -> 465 us (173 -> 295 TFLOP/s, the
-// three-piece kernel before); 16384 x 384 x 1536: 130 -> 94; its weight
-// gradient 137 -> 104; 16384 x 1152 x 384, where a tile's beginning and end
-// weigh as much as its 12 steps, 106 -> 104.
+// (sched_group_barrier).
+//
+// Two workgroups fit a CU, and a launch has no more than fill the chip: each
+// takes its tiles one after another, and the pipeline runs on across them
+// (the last two steps of a tile request and stage the next one's first two,
+// scaled by samples that were read during the epilogue before).  With a
+// workgroup per tile every tile began with three exposed round trips to
+// memory (samples, first and second step), all 512 resident ones at the same
+// time: 16384 x 1536 products took 57-64 us plus 4.1-4.6 us per 32 of K.
 // ---------------------------------------------------------------------------
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -671,11 +677,11 @@ __device__ __forceinline__ void split(f32x4 x2, float zero, uint2& h, uint2& l) 
 }
 }  // namespace h2
 
-// One operand's R x 32 tile (rows = m for A, n for B), R = 96 or 128.  KC:
-// contiguous along k in global memory (rows strided by srow); else contiguous
-// along the rows (k strided by sk).  Slot i of a thread is the float4 vector
-// idx = tid + 256 i: KC: row idx/8, k 4(idx%8)..+3; else: k idx/(R/4), rows
-// 4(idx%(R/4))..+3.
+// One operand's R x 32 tile (rows = m for A, n for B), R = 64 (KC), 96 or
+// 128.  KC: contiguous along k in global memory (rows strided by srow); else
+// contiguous along the rows (k strided by sk).  Slot i of a thread is the
+// float4 vector idx = tid + 256 i: KC: row idx/8, k 4(idx%8)..+3; else: k
+// idx/(R/4), rows 4(idx%(R/4))..+3.
 // LDS planes.  KC: [row][32 k], rows of 64 bytes, the four 16-byte chunks
 // permuted by (row/4)%4, so the 16 rows of a fragment read's quarter cover
 // all 64 banks.  Else [k][R rows]: the transposing read takes 32 bytes of
@@ -683,106 +689,112 @@ __device__ __forceinline__ void split(f32x4 x2, float zero, uint2& h, uint2& l) 
 // by itself, R = 128 permutes the four 64-byte blocks of a row by k%4.
 template <bool KC, int R>
 struct H2Stage {
-  static_assert(R == 96 || R == 128, "tile rows");
-  static constexpr int NV = R * h2::BK / 4 / kGT;    // float4 per thread
-  static constexpr int PS = R * h2::BK;              // plane size (fp16)
+  static_assert(R == 96 || R == 128 || (KC && R == 64), "tile rows");
+  static constexpr int NV = R * h2::BK / 4 / kGT;              // float4 per thread
+  static constexpr int NQ = 2;                                 // sample vectors per thread
+  static constexpr int PS = R * h2::BK;                        // plane size (fp16)
   static constexpr int NSC = KC ? NV : R == 128 ? 4 : 4 * NV;  // scales a thread needs
-  const char* base;   // the operand at (row r0, k 0)
+  static constexpr bool kEach = !KC && R == 96;                // slots do not lie a constant apart
   int64_t kstep;      // bytes per k
-  int64_t last;       // bytes from base to the operand's end
+  uint32_t sstep;     // bytes per row (KC) or k (else)
   uint32_t voff[NV];  // this thread's byte offsets in a k-tile
-  int lput;           // LDS offset (fp16) of slot 0; slot i adds a constant
-  int lputs[R == 96 && !KC ? NV : 1];
+  int lput[kEach ? NV : 1];
   float sc[NSC];
+  // a tile's place: the operand at (its first row, its first k), and the
+  // bytes from there to the operand's end; uniform
+  struct Src {
+    const char* base;
+    int64_t left;
+  };
 
-  __device__ __forceinline__ void init(const float* b, int64_t srow, int64_t sk, int rows, int K, int r0, int tid) {
-    base = reinterpret_cast<const char*>(b + (int64_t)r0 * srow);
+  __device__ __forceinline__ void init(int64_t srow, int64_t sk, int tid) {
     kstep = sk * 4;
-    last = ((int64_t)(rows - 1 - r0) * srow + (int64_t)(K - 1) * sk + 1) * 4;
+    sstep = (uint32_t)((KC ? srow : sk) * 4);
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int idx = tid + i * kGT;
-      if constexpr (KC) voff[i] = (uint32_t)(idx / 8) * (uint32_t)(srow * 4) + 16 * (idx % 8);
-      else voff[i] = (uint32_t)(idx / (R / 4)) * (uint32_t)(sk * 4) + 16 * (idx % (R / 4));
+      voff[i] = KC ? (uint32_t)(idx / 8) * sstep + 16 * (idx % 8)
+                   : (uint32_t)(idx / (R / 4)) * sstep + 16 * (idx % (R / 4));
+      if constexpr (kEach) lput[i] = idx * 4;
     }
     if constexpr (KC) {
       const int row = tid / 8, c = (tid % 8) / 2;
-      lput = row * h2::BK + 8 * (c ^ ((row >> 2) & 3)) + 4 * (tid & 1);
+      lput[0] = row * h2::BK + 8 * (c ^ ((row >> 2) & 3)) + 4 * (tid & 1);
     } else if constexpr (R == 128) {
       const int k = tid / 32, c = 4 * (tid % 32);
-      lput = k * R + (c ^ (32 * (k & 3)));
-    } else {
-#pragma unroll
-      for (int i = 0; i < NV; ++i) lputs[i] = (tid + i * kGT) * 4;
+      lput[0] = k * R + (c ^ (32 * (k & 3)));
     }
   }
-  __device__ __forceinline__ int put_at(int i) const {
-    if constexpr (KC) return lput + i * 32 * h2::BK;      // 32 rows on: the same permutation
-    else if constexpr (R == 128) return lput + i * 8 * R;  // 8 k on
-    else return lputs[i];
+  __device__ __forceinline__ Src at(const float* b, int64_t srow, int64_t sk, int rows, int K, int r0, int k0) const {
+    return {reinterpret_cast<const char*>(b + (int64_t)r0 * srow + (int64_t)k0 * sk),
+            ((int64_t)(rows - 1 - r0) * srow + (int64_t)(K - 1 - k0) * sk + 1) * 4};
   }
-  // The k-tile at k0 through a buffer resource based at its first value and
-  // ending at the operand's last: no per-lane address arithmetic, and rows
-  // past the operand's end read as zeros.  (A vector reaching past a row's
-  // last value takes what follows it in memory, which the caller allows for
-  // rows only: their products land in rows or columns of C that are not
-  // stored.)
-  __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile(int k0) const {
-    const int64_t off = (int64_t)k0 * kstep, left = last - off;
-    const unsigned bytes = left > 0x7ffffff0ll ? 0x7ffffff0u : left > 0 ? (unsigned)left : 0u;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(base + off), (short)0, (int)bytes, 0x00020000);
+  __device__ __forceinline__ int put_at(int i) const {
+    if constexpr (KC) return lput[0] + i * 32 * h2::BK;       // 32 rows on: the same permutation
+    else if constexpr (R == 128) return lput[0] + i * 8 * R;  // 8 k on
+    else return lput[i];
+  }
+  // The k-tile k values from s on, through a buffer resource based at its
+  // first value and ending at the operand's last: no per-lane address
+  // arithmetic, and rows past the operand's end read as zeros.  (A vector
+  // reaching past a row's last value takes what follows it in memory, which
+  // the caller allows for rows only: their products land in rows or columns
+  // of C that are not stored.)
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile(const Src& s, int k) const {
+    const int64_t off = (int64_t)k * kstep, left = s.left - off;
+    const int hi = (int)(left >> 32);
+    const uint32_t bytes = hi < 0 ? 0u : hi > 0 ? 0xfffffff0u : (uint32_t)left;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(s.base + off), (short)0, (int)bytes, 0x00020000);
   }
   __device__ __forceinline__ f32x4 fetch(__amdgpu_buffer_rsrc_t rs, int i) const {
     return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)voff[i], 0, 0));
   }
-  // the same by element where a vector may reach past the last row or kend
-  __device__ __forceinline__ f32x4 fetch_checked(int k0, int kend, int nrows, int64_t srow, int i, int tid) const {
+  // the same by element where a vector may reach past the last row or k
+  __device__ __forceinline__ f32x4 fetch_checked(const Src& s, int k0, int n, int nrows, int i, int tid) const {
     const int idx = tid + i * kGT;
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    const float* p = reinterpret_cast<const float*>(base);
-    if constexpr (KC) {
-      const int row = idx / 8, k = k0 + 4 * (idx % 8);
+    const int row = KC ? idx / 8 : 4 * (idx % (R / 4)), k = k0 + (KC ? 4 * (idx % 8) : idx / (R / 4));
+    const float* p = reinterpret_cast<const float*>(s.base + (int64_t)(KC ? row : k) * sstep) + (KC ? k : row);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (row < nrows && k + j < kend) v[j] = p[(int64_t)row * srow + k + j];
-    } else {
-      const int k = k0 + idx / (R / 4), row = 4 * (idx % (R / 4));
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if (k < kend && row + j < nrows) v[j] = p[(int64_t)k * (kstep / 4) + row + j];
-    }
+    for (int j = 0; j < 4; ++j)
+      if (row + (KC ? 0 : j) < nrows && k + (KC ? j : 0) < n) v[j] = p[j];
     return v;
   }
-  // 32 values of each row, spread evenly over the n k (n >= 256) from kbeg on:
-  // KC: 8 vectors n/8 apart; else k rows n/32 apart
-  __device__ __forceinline__ void sample(f32x4 (&r)[NV], int kbeg, int n, uint32_t sstep, int tid) const {
-    const __amdgpu_buffer_rsrc_t rs = tile(kbeg);
-    const uint32_t far = KC ? (uint32_t)(n / 32) * 16u : (uint32_t)(n / 32) * sstep;
+  // 16 values of each row, spread evenly over the tile's n k (n >= 256): KC:
+  // four vectors, at 0, 1/3, 2/3 and the end; else 16 k rows.  Thread vector
+  // i is idx = tid + 256 i (repeating those 128 before where that is past the
+  // tile's R*4): KC: row idx/4, place idx%4; else place idx/(R/4).
+  __device__ __forceinline__ static int qvec(int i, int tid) {
+    const int idx = tid + i * kGT;
+    return idx < R * 4 ? idx : idx - (R == 64 ? 256 : 128);
+  }
+  __device__ __forceinline__ void sample(f32x4 (&q)[NQ], const Src& s, int n, int tid) const {
+    const __amdgpu_buffer_rsrc_t rs = tile(s, 0);
+    const uint32_t far = KC ? (uint32_t)((n - 4) / 3) * 4u : (uint32_t)((n - 1) / 15) * sstep;
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = tid + i * kGT;
-      const uint32_t off = KC ? (uint32_t)(idx / 8) * sstep + (uint32_t)(idx % 8) * far
+    for (int i = 0; i < NQ; ++i) {
+      const int idx = qvec(i, tid);
+      const uint32_t off = KC ? (uint32_t)(idx / 4) * sstep + (uint32_t)(idx % 4) * far
                               : (uint32_t)(idx / (R / 4)) * far + 16 * (idx % (R / 4));
-      r[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
+      q[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
     }
   }
   // amax[row] = the largest of each row's samples (as bits); it is zero before
-  __device__ __forceinline__ void row_max(const f32x4 (&r)[NV], uint32_t* amax, int tid) const {
+  __device__ __forceinline__ static void row_max(const f32x4 (&q)[NQ], uint32_t* amax, int tid) {
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = tid + i * kGT;
+    for (int i = 0; i < NQ; ++i) {
+      const int idx = qvec(i, tid);
       if constexpr (KC) {
         uint32_t m = 0;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) m = max(m, __float_as_uint(r[i][j]) & 0x7fffffffu);
+        for (int j = 0; j < 4; ++j) m = max(m, __float_as_uint(q[i][j]) & 0x7fffffffu);
         m = max(m, (uint32_t)__shfl_xor((int)m, 1));
         m = max(m, (uint32_t)__shfl_xor((int)m, 2));
-        m = max(m, (uint32_t)__shfl_xor((int)m, 4));
-        if ((tid & 7) == 0) amax[idx / 8] = m;
+        if ((tid & 3) == 0) amax[idx / 4] = m;
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          atomicMax(&amax[4 * (idx % (R / 4)) + j], __float_as_uint(r[i][j]) & 0x7fffffffu);
+          atomicMax(&amax[4 * (idx % (R / 4)) + j], __float_as_uint(q[i][j]) & 0x7fffffffu);
       }
     }
   }
@@ -829,6 +841,14 @@ struct H2Stage {
   }
 };
 
+// a thread or lane number whose uses are computed where they stand: code that
+// runs once a tile or less otherwise keeps its addresses in registers across
+// the k loop, which needs them all
+__device__ __forceinline__ int here(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
 template <int MI, int NI, int WM, int WN, bool AK, bool BN1, int ACT>
 __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
   static_assert(WM * WN == 4, "four waves");
@@ -838,385 +858,504 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
   using XA = X3Stage<AK, BM>;
   using XB = X3Stage<!BN1, BN>;
   constexpr int kBuf = 2 * (SA::PS + SB::PS);  // one stage's planes (fp16)
-  constexpr int EW = 32 * NI + 8;              // row stride of the epilogue's 16-row strips (floats)
-  constexpr int kEp = 4 * 16 * EW * 4;
   constexpr int kX3 = 3 * (XA::PS + XB::PS) * 2;
-  constexpr int kTiles = 2 * kBuf * 2;
-  static_assert(kTiles >= kEp && kTiles >= kX3 && kTiles >= 8 * BN * 4, "LDS");
+  constexpr int kTiles = 2 * kBuf * 2 > kX3 ? 2 * kBuf * 2 : kX3;
   __shared__ __attribute__((aligned(16))) char smem[kTiles];
-  __shared__ uint32_t amax[BM + BN];  // rows' and columns' largest sample
+  __shared__ float red[ACT == 3 ? 8 * BN : 1];  // column sums
+  // rows' and columns' largest sample of the tiles: one in its epilogue, one
+  // being staged, one being sampled, one being cleared
+  __shared__ __attribute__((aligned(16))) uint32_t amax[4][BM + BN];
   __shared__ int again;
-  _Float16* buf0 = reinterpret_cast<_Float16*>(smem);
-  _Float16* buf1 = buf0 + kBuf;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wid / WN) * 32 * MI, wn = (wid % WN) * 32 * NI;
-  // Workgroups are dealt round-robin over the 8 XCDs in dispatch order; give
-  // each XCD a contiguous run of row-major tiles, so the column tiles that
-  // share an A row panel read it through the same L2
-  int tx, ty, zb;
+
+  // Workgroups are dealt round-robin over the 8 XCDs in dispatch order; each
+  // XCD's take a contiguous run of row-major tiles, one after another, so the
+  // column tiles that share an A row panel read it through the same L2
+  const int gx = (g.N + BN - 1) / BN, gy = (g.M + BM - 1) / BM;
+  int tile, tend;
+  const int wgs = ((int)gridDim.x - (int)(blockIdx.x & 7) + 7) >> 3;  // this XCD's workgroups
   {
-    const int nt = gridDim.x * gridDim.y * gridDim.z;
-    const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-    const int xcd = lin & 7, per = nt >> 3, more = nt & 7;
-    const int t = xcd * per + min(xcd, more) + (lin >> 3);
-    tx = t % gridDim.x;
-    ty = (t / gridDim.x) % gridDim.y;
-    zb = t / (gridDim.x * gridDim.y);
+    const int nt = gx * gy * g.batch * g.ksplit;
+    const int xcd = blockIdx.x & 7, per = nt >> 3, more = nt & 7;
+    tile = xcd * per + min(xcd, more);
+    tend = tile + per + (xcd < more ? 1 : 0);
+    tile += blockIdx.x >> 3;
   }
-  const int m0 = ty * BM, n0 = tx * BN;
-  const int bidx = zb % g.batch, split = zb / g.batch;
-  const int kbeg = split * g.kchunk;
-  const int kend = min(g.K, kbeg + g.kchunk);
-  const float* A = g.a + (int64_t)bidx * g.sab;
-  const float* B = g.b + (int64_t)bidx * g.sbb;
+  struct Place {
+    int m0, n0, bidx, split, kbeg, n;
+  };
+  auto place = [&](int t) {
+    Place p;
+    p.n0 = t % gx * BN;
+    p.m0 = t / gx % gy * BM;
+    const int z = t / (gx * gy);
+    p.bidx = z % g.batch;
+    p.split = z / g.batch;
+    p.kbeg = p.split * g.kchunk;
+    p.n = min(g.K, p.kbeg + g.kchunk) - p.kbeg;
+    return p;
+  };
+  if (tile >= tend) return;
+
+  SA sa;
+  SB sb;
+  sa.init(g.sam, g.sak, tid);
+  sb.init(g.sbn, g.sbk, tid);
+  auto src_a = [&](const Place& p) {
+    return sa.at(g.a + (int64_t)p.bidx * g.sab, g.sam, g.sak, g.M, g.K, p.m0, p.kbeg);
+  };
+  auto src_b = [&](const Place& p) {
+    return sb.at(g.b + (int64_t)p.bidx * g.sbb, g.sbn, g.sbk, g.N, g.K, p.n0, p.kbeg);
+  };
 
   f32x16 acc[MI][NI], accx[MI][NI];
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int j = 0; j < NI; ++j)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = accx[i][j][e] = 0.f;
+  f32x4 ra[SA::NV], rb[SB::NV];
   // ACT 3: column sums of B from the values each thread stages
   float cs[SB::NV][4];
-#pragma unroll
-  for (int i = 0; i < SB::NV; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) cs[i][j] = 0.f;
-  const bool two = g.fast && kend - kbeg >= h2::MINK;  // the two-piece form is tried
-  bool scaled = false;                                 // acc, accx hold its sums
+  float zero = 0.f;
+  asm("" : "+s"(zero));
+  int par = 0;  // the buffer that holds the step to multiply
+  auto buf = [&](int b) { return reinterpret_cast<_Float16*>(smem) + b * kBuf; };
 
-  if (two) {
-    SA sa;
-    SB sb;
-    sa.init(A, g.sam, g.sak, g.M, g.K, m0, tid);
-    sb.init(B, g.sbn, g.sbk, g.N, g.K, n0, tid);
-    for (int i = tid; i < BM + BN; i += kGT) amax[i] = 0;
-    if (tid == 0) again = 0;
-    const int steps = (kend - kbeg + h2::BK - 1) / h2::BK;
-    // The k steps that the unchecked loads take: whole ones, and (where the
-    // rows of an operand contiguous along them do not end on a vector) not
-    // the operand's last, whose last vectors reach past its end.
-    int whole = (kend - kbeg) / h2::BK;
-    if (((!AK && (g.M & 3)) || (BN1 && (g.N & 3))) && kend == g.K && whole == steps) --whole;
+  auto colsum = [&] {
+    if constexpr (ACT == 3) {
+#pragma unroll
+      for (int i = 0; i < SB::NV; ++i) {
+        if constexpr (!BN1) cs[i][0] += (rb[i][0] + rb[i][1]) + (rb[i][2] + rb[i][3]);
+        else
+#pragma unroll
+          for (int j = 0; j < 4; ++j) cs[0][j] += rb[i][j];
+      }
+    }
+  };
+  // the products of one step, MFMA by MFMA: half a step (sub) at a time the
+  // four fragments' three products.  fa, fb: [sub][piece][tile].
+  constexpr int kT = MI * NI, kM = 6 * kT;
+  f16x8 fa[2][2][MI], fb[2][2][NI];
+  auto read_frags = [&](const _Float16* cur, int sub, int p) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) fa[sub][p][i] = SA::frag(cur, p, sub, wm + 32 * i, lane);
+#pragma unroll
+    for (int j = 0; j < NI; ++j) fb[sub][p][j] = SB::frag(cur + 2 * SA::PS, p, sub, wn + 32 * j, lane);
+  };
+  auto product = [&](int q) {
+    const int sub = q / (3 * kT), kind = q / kT % 3, i = q % kT / NI, j = q % NI;
+    if (kind == 0) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][0][i], fb[sub][0][j], acc[i][j], 0, 0, 0);
+    else if (kind == 1)
+      accx[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][1][i], fb[sub][0][j], accx[i][j], 0, 0, 0);
+    else accx[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][0][i], fb[sub][1][j], accx[i][j], 0, 0, 0);
+  };
+  // One step: its products in as many groups as there are vectors to stage
+  // (kS); beside each group's products one vector of the next step is split
+  // and stored, and its register refilled with the step after's (refill).
+  constexpr int kS = SA::NV + SB::NV;
+  auto step = [&](auto refill, __amdgpu_buffer_rsrc_t ta, __amdgpu_buffer_rsrc_t tb) {
+    const _Float16* cur = buf(par);
+    _Float16* nxt = buf(par ^ 1);
+    read_frags(cur, 0, 0);
+    read_frags(cur, 0, 1);
+    colsum();
+#pragma unroll
+    for (int c = 0; c < kS; ++c) {
+      __builtin_amdgcn_sched_barrier(0);
+      // the second half's fragments, as the first half's come free
+      if (c == kS / 2 - 2) read_frags(cur, 1, 0);
+      if (c == kS / 2 - 1) read_frags(cur, 1, 1);
+#pragma unroll
+      for (int q = c * kM / kS; q < (c + 1) * kM / kS; ++q) product(q);
+      if (c < SA::NV) {
+        sa.put(nxt, ra[c], zero, c);
+        if constexpr (decltype(refill)::value) ra[c] = sa.fetch(ta, c);
+      } else {
+        sb.put(nxt + 2 * SA::PS, rb[c - SA::NV], zero, c - SA::NV);
+        if constexpr (decltype(refill)::value) rb[c - SA::NV] = sb.fetch(tb, c - SA::NV);
+      }
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        if (c == kS / 2 - 2 || c == kS / 2 - 1) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+      }
+    }
+    par ^= 1;
+    __syncthreads();
+  };
 
-    f32x4 ra[SA::NV], rb[SB::NV];
-    auto fetch_any = [&](int t) {
-      const int k0 = kbeg + t * h2::BK;
-      if (t < whole) {
-        const auto ta = sa.tile(k0), tb = sb.tile(k0);
+  Place cur = place(tile);
+  bool primed = false;  // this tile's first step is staged, its second one in registers
+  if (tid == 0) again = 0;
+  for (int i = tid; i < 4 * (BM + BN); i += kGT) amax[0][i] = 0;
+  if (g.fast) {
+    f32x4 qa[2][SA::NQ], qb[2][SB::NQ];
+    const bool more = tile + wgs < tend;
+    const Place p1 = place(more ? tile + wgs : tile);
+    sa.sample(qa[0], src_a(cur), cur.n, tid);
+    sb.sample(qb[0], src_b(cur), cur.n, tid);
+    sa.sample(qa[1], src_a(p1), p1.n, tid);
+    sb.sample(qb[1], src_b(p1), p1.n, tid);
+    __syncthreads();
+    SA::row_max(qa[0], amax[0], tid);
+    SB::row_max(qb[0], amax[0] + BM, tid);
+    SA::row_max(qa[1], amax[1], tid);
+    SB::row_max(qb[1], amax[1] + BM, tid);
+    __syncthreads();
+  }
+
+  for (int seq = 0;; ++seq) {
+    const bool more = tile + wgs < tend;
+    const Place next = place(more ? tile + wgs : tile);
+    bool scaled = false;  // acc, accx hold the two-piece sums
+    float cso[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = accx[i][j][e] = 0.f;
+
+    if (g.fast) {
+      const typename SA::Src a0 = src_a(cur);
+      const typename SB::Src b0 = src_b(cur);
+      const int steps = (cur.n + h2::BK - 1) / h2::BK;
+      // The k steps that the unchecked loads take: whole ones, and (where the
+      // rows of an operand contiguous along them do not end on a vector) not
+      // the operand's last, whose last vectors reach past its end.
+      int whole = cur.n / h2::BK;
+      if (((!AK && (g.M & 3)) || (BN1 && (g.N & 3))) && cur.kbeg + cur.n == g.K && whole == steps) --whole;
+      for (int i = tid; i < BM + BN; i += kGT) amax[(seq + 2) & 3][i] = 0;
+      if (!primed) {
+        sa.scales(amax[seq & 3], tid);
+        sb.scales(amax[seq & 3] + BM, tid);
+        // (n >= 256: the first two steps are whole)
+        auto ta = sa.tile(a0, 0);
+        auto tb = sb.tile(b0, 0);
 #pragma unroll
         for (int i = 0; i < SA::NV; ++i) ra[i] = sa.fetch(ta, i);
 #pragma unroll
         for (int i = 0; i < SB::NV; ++i) rb[i] = sb.fetch(tb, i);
-      } else {
+        if constexpr (ACT == 3) {
 #pragma unroll
-        for (int i = 0; i < SA::NV; ++i) ra[i] = sa.fetch_checked(k0, kend, g.M - m0, g.sam, i, tid);
+          for (int i = 0; i < SB::NV; ++i)
 #pragma unroll
-        for (int i = 0; i < SB::NV; ++i) rb[i] = sb.fetch_checked(k0, kend, g.N - n0, g.sbn, i, tid);
-      }
-    };
-    auto colsum = [&] {
-      if constexpr (ACT == 3) {
+            for (int j = 0; j < 4; ++j) cs[i][j] = 0.f;
+        }
+        colsum();
+        ta = sa.tile(a0, h2::BK);
+        tb = sb.tile(b0, h2::BK);
+#pragma unroll
+        for (int i = 0; i < SA::NV; ++i) {
+          sa.put(buf(par), ra[i], zero, i);
+          ra[i] = sa.fetch(ta, i);
+        }
 #pragma unroll
         for (int i = 0; i < SB::NV; ++i) {
-          if constexpr (!BN1) cs[i][0] += (rb[i][0] + rb[i][1]) + (rb[i][2] + rb[i][3]);
-          else
+          sb.put(buf(par) + 2 * SA::PS, rb[i], zero, i);
+          rb[i] = sb.fetch(tb, i);
+        }
+        __syncthreads();
+      }
+      int t = 0;
+      for (; t + 2 < whole; ++t)
+        step(std::true_type{}, sa.tile(a0, (t + 2) * h2::BK), sb.tile(b0, (t + 2) * h2::BK));
+      if (t + 2 < steps) {  // at most one step that is not whole
+        step(std::false_type{}, sa.tile(a0, 0), sb.tile(b0, 0));
+        ++t;
+        const int tv = here(tid);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) cs[BN == 128 ? 0 : i][j] += rb[i][j];
+        for (int i = 0; i < SA::NV; ++i) ra[i] = sa.fetch_checked(a0, (t + 1) * h2::BK, cur.n, g.M - cur.m0, i, tv);
+#pragma unroll
+        for (int i = 0; i < SB::NV; ++i) rb[i] = sb.fetch_checked(b0, (t + 1) * h2::BK, cur.n, g.N - cur.n0, i, tv);
+      }
+      // the last two steps: request, then stage, the next tile's first two
+      typename SA::Src a1 = src_a(next);
+      typename SB::Src b1 = src_b(next);
+      if (!more) a1.left = b1.left = 0;  // reads as zeros
+      step(std::true_type{}, sa.tile(a1, 0), sb.tile(b1, 0));
+      if constexpr (ACT == 3) {  // from here on the sums are the next tile's
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          cso[j] = BN1 ? cs[0][j] : cs[j % SB::NV][0];
+          (BN1 ? cs[0][j] : cs[j % SB::NV][0]) = 0.f;
         }
       }
-    };
-    float zero = 0.f;
-    asm("" : "+s"(zero));
-    // The products of one step, MFMA by MFMA: half a step (sub) at a time the
-    // four fragments' three products.  fa, fb: [sub][piece][tile].
-    constexpr int kT = MI * NI, kM = 6 * kT;
-    f16x8 fa[2][2][MI], fb[2][2][NI];
-    auto read_frags = [&](const _Float16* cur, int sub) {
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-#pragma unroll
-        for (int i = 0; i < MI; ++i) fa[sub][p][i] = SA::frag(cur, p, sub, wm + 32 * i, lane);
-#pragma unroll
-        for (int j = 0; j < NI; ++j) fb[sub][p][j] = SB::frag(cur + 2 * SA::PS, p, sub, wn + 32 * j, lane);
-      }
-    };
-    auto product = [&](int q) {
-      const int sub = q / (3 * kT), kind = q / kT % 3, i = q % kT / NI, j = q % NI;
-      if (kind == 0) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][0][i], fb[sub][0][j], acc[i][j], 0, 0, 0);
-      else if (kind == 1)
-        accx[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][1][i], fb[sub][0][j], accx[i][j], 0, 0, 0);
-      else accx[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][0][i], fb[sub][1][j], accx[i][j], 0, 0, 0);
-    };
-    // One step: its products in as many groups as there are vectors to stage
-    // (kS); beside each group's products one vector of the next step is split
-    // and stored, and its register refilled with the step after's.
-    constexpr int kS = SA::NV + SB::NV;
-    auto step = [&](const _Float16* cur, _Float16* nxt, int t2) {
-      const int k0 = kbeg + t2 * h2::BK;
-      const auto ta = sa.tile(k0), tb = sb.tile(k0);
-      read_frags(cur, 0);
-      colsum();
-#pragma unroll
-      for (int c = 0; c < kS; ++c) {
-        __builtin_amdgcn_sched_barrier(0);
-        if (c == 1) read_frags(cur, 1);
-#pragma unroll
-        for (int q = c * kM / kS; q < (c + 1) * kM / kS; ++q) product(q);
-        if (c < SA::NV) {
-          sa.put(nxt, ra[c], zero, c);
-          ra[c] = sa.fetch(ta, c);
-        } else {
-          sb.put(nxt + 2 * SA::PS, rb[c - SA::NV], zero, c - SA::NV);
-          rb[c - SA::NV] = sb.fetch(tb, c - SA::NV);
-        }
-#pragma unroll
-        for (int q = 0; q < 3; ++q) {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          if (c == 1) __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-        }
-      }
-      __syncthreads();
-    };
-    auto put_all = [&](_Float16* nxt) {
-#pragma unroll
-      for (int i = 0; i < SA::NV; ++i) sa.put(nxt, ra[i], zero, i);
-#pragma unroll
-      for (int i = 0; i < SB::NV; ++i) sb.put(nxt + 2 * SA::PS, rb[i], zero, i);
-    };
-
-    {
-      f32x4 qa[SA::NV], qb[SB::NV];
-      sa.sample(qa, kbeg, kend - kbeg, (uint32_t)(AK ? g.sam : g.sak) * 4u, tid);
-      sb.sample(qb, kbeg, kend - kbeg, (uint32_t)(BN1 ? g.sbk : g.sbn) * 4u, tid);
-      fetch_any(0);
-      __syncthreads();
-      sa.row_max(qa, amax, tid);
-      sb.row_max(qb, amax + BM, tid);
-    }
-    __syncthreads();
-    sa.scales(amax, tid);
-    sb.scales(amax + BM, tid);
-    colsum();
-    put_all(buf0);
-    if (steps > 1) fetch_any(1);
-    __syncthreads();
-    int t = 0;
-    for (; t + 3 < whole; t += 2) {
-      step(buf0, buf1, t + 2);
-      step(buf1, buf0, t + 3);
-    }
-    for (; t < steps; ++t) {  // t is even at first; the last step has nothing to stage
-      read_frags((t & 1) ? buf1 : buf0, 0);
-      read_frags((t & 1) ? buf1 : buf0, 1);
-#pragma unroll
-      for (int q = 0; q < kM; ++q) product(q);
-      if (t + 1 < steps) {
-        colsum();
-        put_all((t & 1) ? buf0 : buf1);
-        if (t + 2 < steps) fetch_any(t + 2);
-      }
-      __syncthreads();
-    }
-    // Inf or NaN in a row or column of the tile: every row of the wave's
-    // tile in its first column, every column in its first row
-    float z = 0.f;
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) z += 0.f * acc[i][0][e] + 0.f * accx[i][0][e];
-#pragma unroll
-    for (int j = 1; j < NI; ++j) z += 0.f * acc[0][j][0] + 0.f * accx[0][j][0];
-    if (!(z == 0.f)) again = 1;  // any lane
-    __syncthreads();
-    scaled = again == 0;
-  }
-
-  if (!scaled) {
-    XA xa;
-    XB xb;
-    xa.init(A, g.sam, g.sak, g.M, m0, tid);
-    xb.init(B, g.sbn, g.sbk, g.N, n0, tid);
-    __bf16* As = reinterpret_cast<__bf16*>(smem);
-    __bf16* Bs = As + 3 * XA::PS;
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-      for (int j = 0; j < NI; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-    const bool sums = ACT == 3 && !two;  // else they are there already
-    f32x4 ra[XA::NV], rb[XB::NV];
-    xa.fetch_checked(ra, kbeg, kend, tid);
-    xb.fetch_checked(rb, kbeg, kend, tid);
-    for (int k0 = kbeg; k0 < kend; k0 += x3::BK) {
-      __syncthreads();
-      xa.put(As, ra);
-      xb.put(Bs, rb);
-      if (sums) XB::colsum_add(cs[0], rb);
-      __syncthreads();
-      if (k0 + x3::BK < kend) {
-        xa.fetch_checked(ra, k0 + x3::BK, kend, tid);
-        xb.fetch_checked(rb, k0 + x3::BK, kend, tid);
-      }
-      bf16x8 a[3][MI], b[3][NI];
-#pragma unroll
-      for (int p = 0; p < 3; ++p) {
-#pragma unroll
-        for (int i = 0; i < MI; ++i) a[p][i] = XA::frag(As, p, wm + 32 * i, lane);
-#pragma unroll
-        for (int j = 0; j < NI; ++j) b[p][j] = XB::frag(Bs, p, wn + 32 * j, lane);
-      }
+      sa.scales(amax[(seq + 1) & 3], tid);
+      sb.scales(amax[(seq + 1) & 3] + BM, tid);
+      step(std::true_type{}, sa.tile(a1, more ? h2::BK : 0), sb.tile(b1, more ? h2::BK : 0));
+      primed = more;
+      // Inf or NaN in a row or column of the tile: every row of the wave's
+      // tile in its first column, every column in its first row
+      float z = 0.f;
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NI; ++j) {
-          f32x16 c = acc[i][j];
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2][i], b[0][j], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[1][j], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[2][j], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[0][j], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[1][j], c, 0, 0, 0);
-          c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[0][j], c, 0, 0, 0);
-          acc[i][j] = c;
-        }
+        for (int e = 0; e < 16; ++e) z += 0.f * acc[i][0][e] + 0.f * accx[i][0][e];
+#pragma unroll
+      for (int j = 1; j < NI; ++j) z += 0.f * acc[0][j][0] + 0.f * accx[0][j][0];
+      if (!(z == 0.f)) again = seq + 1;  // any lane
+      __syncthreads();
+      scaled = again != seq + 1;
     }
-    __syncthreads();
-  }
 
-  if constexpr (ACT == 3) {
-    // the first row of tiles reduces the per-thread column sums through LDS:
-    // KC: 8 (three pieces: 4) threads per column, else 8 threads per 4 columns; contributors
-    // are added in a fixed order
-    static_assert(BN == 128, "column sums");
-    if (m0 == 0) {
-      float* red = reinterpret_cast<float*>(smem);  // [8][BN]
+    if (!scaled) {
+      primed = false;  // the buffers are used otherwise
+      const int tv = here(tid), lv = tv & 63;
+      XA xa;
+      XB xb;
+      xa.init(g.a + (int64_t)cur.bidx * g.sab, g.sam, g.sak, g.M, cur.m0, tv);
+      xb.init(g.b + (int64_t)cur.bidx * g.sbb, g.sbn, g.sbk, g.N, cur.n0, tv);
+      __bf16* As = reinterpret_cast<__bf16*>(smem);
+      __bf16* Bs = As + 3 * XA::PS;
 #pragma unroll
-      for (int i = 0; i < SB::NV; ++i) {
-        if constexpr (!BN1) {
-          const int idx = tid + i * kGT;
-          if (two) red[(idx % 8) * BN + idx / 8] = cs[i][0];
-          else if (i < XB::NV) red[(idx % 4) * BN + idx / 4] = cs[0][i];
-        } else if (i == 0) {
+      for (int i = 0; i < MI; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) red[(tid / 32) * BN + 4 * (tid % 32) + j] = cs[0][j];
+        for (int j = 0; j < NI; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      const bool sums = ACT == 3 && !g.fast;  // else they are there already
+      const int kbeg = cur.kbeg, kend = cur.kbeg + cur.n;
+      f32x4 pa[XA::NV], pb[XB::NV];
+      xa.fetch_checked(pa, kbeg, kend, tv);
+      xb.fetch_checked(pb, kbeg, kend, tv);
+      for (int k0 = kbeg; k0 < kend; k0 += x3::BK) {
+        __syncthreads();
+        xa.put(As, pa);
+        xb.put(Bs, pb);
+        if constexpr (ACT == 3) {
+          if (sums) XB::colsum_add(cso, pb);
         }
+        __syncthreads();
+        if (k0 + x3::BK < kend) {
+          xa.fetch_checked(pa, k0 + x3::BK, kend, tv);
+          xb.fetch_checked(pb, k0 + x3::BK, kend, tv);
+        }
+        bf16x8 a[3][MI], b[3][NI];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+#pragma unroll
+          for (int i = 0; i < MI; ++i) a[p][i] = XA::frag(As, p, wm + 32 * i, lv);
+#pragma unroll
+          for (int j = 0; j < NI; ++j) b[p][j] = XB::frag(Bs, p, wn + 32 * j, lv);
+        }
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j) {
+            f32x16 c = acc[i][j];
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2][i], b[0][j], c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[1][j], c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[2][j], c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[0][j], c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[1][j], c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[0][j], c, 0, 0, 0);
+            acc[i][j] = c;
+          }
       }
       __syncthreads();
-      if (tid < BN) {
-        const int NC = BN1 || two ? 8 : 4;
-        float v = 0.f;
-        for (int c = 0; c < NC; ++c) v += red[c * BN + tid];
-        const int n = n0 + tid;
-        if (n < g.N) {
-          if (g.ksplit > 1) g.ws[(int64_t)g.ksplit * g.M * g.N + (int64_t)split * g.N + n] = v;
-          else g.colsum[n] = g.colsum_acc ? g.colsum[n] + v : v;
-        }
-      }
-      __syncthreads();
     }
-  }
 
-  // Epilogue, each wave on its own (no barriers): strips of 16 rows of the
-  // wave's tile go through the wave's own LDS (elements 8 half .. +7 of one
-  // row of MFMA tiles; rows of EW floats, so the two rows a store instruction
-  // writes use disjoint banks), then each lane finishes float4 runs of C
-  // rows: coalesced loads and stores, no per-element addresses.
-  // acc[i][j][e] = wave tile element (32i + 8(e/4) + 4(lane/32) + e%4, 32j + lane%32).
-  float* ep = reinterpret_cast<float*>(smem) + wid * 16 * EW;
-  const int lr = lane & 31, lh = lane >> 5;
-  const bool to_ws = g.ksplit > 1;
-  float* W = g.ws + ((int64_t)split * g.batch + bidx) * (int64_t)g.M * g.N;
-  float* Cp = g.c + (int64_t)bidx * g.scb;
-  float* X = g.aux + (int64_t)bidx * g.sxb;
-  const bool rd_c = !to_ws && g.beta != 0.f;
-  const bool use_x = !to_ws && (ACT == 2 || ACT == 4 || (ACT == 1 && g.aux != nullptr));
-  // whole float4 runs of C (and aux) are aligned vectors
-  const bool cvec = to_ws ? (g.N % 4 == 0)
-                          : (g.scn == 1 && g.scm % 4 == 0 && g.scb % 4 == 0 && (((uintptr_t)g.c) & 15u) == 0 &&
-                             (!use_x || (g.sxn == 1 && g.sxm % 4 == 0 && g.sxb % 4 == 0 &&
-                                         (((uintptr_t)g.aux) & 15u) == 0)));
-  float unB[NI];  // of this lane's columns
+    // the samples of the tile after the next, on their way during the epilogue
+    const bool more2 = g.fast && tile + 2 * wgs < tend;
+    const int tq = here(tid);
+    f32x4 qa[SA::NQ], qb[SB::NQ];
+    if (more2) {
+      const Place p2 = place(tile + 2 * wgs);
+      sa.sample(qa, src_a(p2), p2.n, tq);
+      sb.sample(qb, src_b(p2), p2.n, tq);
+    }
+
+    if constexpr (ACT == 3) {
+      // the first row of tiles reduces the per-thread column sums through
+      // LDS: KC: 8 (three pieces: 4) threads per column, else 8 threads per 4
+      // columns; contributors are added in a fixed order
+      static_assert(BN == 128, "column sums");
+      if (cur.m0 == 0) {
 #pragma unroll
-  for (int j = 0; j < NI; ++j) unB[j] = scaled ? h2::unscale(amax[BM + wn + 32 * j + lr]) : 1.f;
-#pragma unroll
-  for (int i = 0; i < MI; ++i)
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int j = 0; j < NI; ++j)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const int r = 8 * (e >> 2) + 4 * lh + (e & 3);
-          float v = acc[i][j][8 * half + e];
-          if (scaled)
-            v = __builtin_fmaf(accx[i][j][8 * half + e], 0x1p-14f, v) * h2::unscale(amax[wm + 32 * i + 16 * half + r]) * unB[j];
-          ep[r * EW + 32 * j + lr] = v;
-        }
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll 2
-      for (int q = 0; q < 2 * NI; ++q) {
-        const int idx = lane + q * 64;
-        const int r = idx / (8 * NI), c = 4 * (idx % (8 * NI));
-        const int m = m0 + wm + 32 * i + 16 * half + r;
-        const int n = n0 + wn + c;
-        const f32x4 a4 = *reinterpret_cast<const f32x4*>(ep + r * EW + c);
-        if (m >= g.M || n >= g.N) continue;
-        const int nv = min(4, g.N - n);
-        if (to_ws) {
-          float* w = W + (int64_t)m * g.N + n;
-          if (cvec && nv == 4) {
-            *reinterpret_cast<f32x4*>(w) = a4;
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (BN1) {
+            red[(tid / 32) * BN + 4 * (tid % 32) + i] = cso[i];
           } else {
-            for (int u = 0; u < nv; ++u) w[u] = a4[u];
-          }
-          continue;
-        }
-        float* cp = Cp + (int64_t)m * g.scm + (int64_t)n * g.scn;
-        float* xp = X + (int64_t)m * g.sxm + (int64_t)n * g.sxn;
-        f32x4 v, old = {0.f, 0.f, 0.f, 0.f}, xa = {0.f, 0.f, 0.f, 0.f}, bv = {0.f, 0.f, 0.f, 0.f};
-        const bool vecs = cvec && nv == 4;
-        if (vecs) {
-          if (rd_c) old = *reinterpret_cast<const f32x4*>(cp);
-          if constexpr (ACT == 2 || ACT == 4) xa = *reinterpret_cast<const f32x4*>(xp);
-        } else {
-          for (int u = 0; u < nv; ++u) {
-            if (rd_c) old[u] = cp[(int64_t)u * g.scn];
-            if constexpr (ACT == 2 || ACT == 4) xa[u] = xp[(int64_t)u * g.sxn];
+            const int idx = tid + i * kGT;
+            if (g.fast) red[(idx % 8) * BN + idx / 8] = cso[i];
+            else if (i < XB::NV) red[(idx % 4) * BN + idx / 4] = cso[i];
           }
         }
-        if (g.bias) {
-          for (int u = 0; u < nv; ++u) bv[u] = g.bias[n + u];
+        __syncthreads();
+        if (tid < BN) {
+          const int nc = BN1 || g.fast ? 8 : 4;
+          float v = 0.f;
+          for (int c = 0; c < nc; ++c) v += red[c * BN + tid];
+          const int n = cur.n0 + tid;
+          if (n < g.N) {
+            if (g.ksplit > 1) g.ws[(int64_t)g.ksplit * g.M * g.N + (int64_t)cur.split * g.N + n] = v;
+            else g.colsum[n] = g.colsum_acc ? g.colsum[n] + v : v;
+          }
+        }
+        __syncthreads();
+      }
+    }
+
+    // Epilogue, from the accumulators: acc[i][j][e] = wave tile element
+    // (32i + 8(e/4) + 4(lane/32) + e%4, 32j + lane%32), so an element e of all
+    // lanes is two rows' 32 columns, a whole 128-byte line each.  A row pair
+    // is stored (and its aux and old values read) through a resource that
+    // begins at its first row and ends with the output: rows past it are
+    // dropped, a column past it has an offset that is.
+    const int lv = here(lane), lr = lv & 31, lh = lv >> 5;
+    const bool to_ws = g.ksplit > 1;
+    const bool rd_c = !to_ws && g.beta != 0.f;
+    const bool use_x = !to_ws && (ACT == 2 || ACT == 4 || (ACT == 1 && g.aux != nullptr));
+    const uint32_t* am = amax[seq & 3];
+    const int n1 = cur.n0 + wn;  // the wave's first column
+    float unB[NI], bv[NI];       // of this lane's columns
+#pragma unroll
+    for (int j = 0; j < NI; ++j) {
+      unB[j] = scaled ? h2::unscale(am[BM + wn + 32 * j + lr]) : 1.f;
+      bv[j] = !to_ws && g.bias && n1 + 32 * j + lr < g.N ? g.bias[n1 + 32 * j + lr] : 0.f;
+    }
+    // the product's values of row group (i, q): [u][j]
+    auto values = [&](int i, int q, float (&v)[4][NI]) {
+      const uint4 a4 = *reinterpret_cast<const uint4*>(am + wm + 32 * i + 8 * q + 4 * lh);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float unA = h2::unscale(u == 0 ? a4.x : u == 1 ? a4.y : u == 2 ? a4.z : a4.w);
+#pragma unroll
+        for (int j = 0; j < NI; ++j) {
+          float x = acc[i][j][4 * q + u];
+          if (scaled) x = __builtin_fmaf(accx[i][j][4 * q + u], 0x1p-14f, x) * unA * unB[j];
+          v[u][j] = to_ws ? x : g.alpha * x + bv[j];
+        }
+      }
+    };
+    // the output (or this split's partials), its row stride, and the aux rows
+    float* Out = to_ws ? g.ws + ((int64_t)cur.split * g.batch + cur.bidx) * (int64_t)g.M * g.N
+                       : g.c + (int64_t)cur.bidx * g.scb;
+    const int64_t so = to_ws ? g.N : g.scm;
+    float* X = g.aux + (int64_t)cur.bidx * g.sxb;
+    if (g.rows_vec) {
+      uint32_t oo[NI], xo[NI];
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        const bool ok = n1 + 32 * j + lr < g.N;
+        oo[j] = ok ? (uint32_t)(4 * lh * so + 32 * j + lr) * 4u : 0xfffffff0u;
+        xo[j] = ok ? (uint32_t)(4 * lh * g.sxm + 32 * j + lr) * 4u : 0xfffffff0u;
+      }
+      // the wave's rows of an array: a resource at row r (rows are asked for in
+      // steps, the address and the bytes left move by uniform additions)
+      struct Rows {
+        const char* p;
+        int64_t left, step;
+        __device__ __forceinline__ __amdgpu_buffer_rsrc_t at(int r) const {
+          const int64_t l = left - r * step;
+          const int hi = (int)(l >> 32);
+          const uint32_t bytes = hi < 0 ? 0u : hi > 0 ? 0xffffff00u : (uint32_t)l;
+          return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p + r * step), (short)0, (int)bytes, 0x00020000);
+        }
+      };
+      const int mw = cur.m0 + wm;
+      auto rows = [&](const float* p, int64_t stride) {
+        return Rows{reinterpret_cast<const char*>(p + (int64_t)mw * stride + n1),
+                    n1 < g.N ? ((int64_t)(g.M - 1 - mw) * stride + (g.N - n1)) * 4 : -1, stride * 4};
+      };
+      const Rows ro = rows(Out, so), rx = rows(X, g.sxm);
+      // aux values are requested kAhead row groups before their use
+      constexpr int kAhead = 4;
+      float xv[kAhead][4][NI];
+      auto aux = [&](int iq) {
+        if constexpr (ACT == 2 || ACT == 4) {
+          if (use_x) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const auto r = rx.at(8 * iq + u);
+#pragma unroll
+              for (int j = 0; j < NI; ++j)
+                xv[iq % kAhead][u][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)xo[j], 0, 0));
+            }
+          }
+        }
+      };
+#pragma unroll
+      for (int iq = 0; iq < kAhead; ++iq) aux(iq);
+#pragma unroll
+      for (int iq = 0; iq < 4 * MI; ++iq) {
+        __builtin_amdgcn_sched_barrier(0);
+        float old[4][NI], v[4][NI];
+        if (rd_c) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const auto r = ro.at(8 * iq + u);
+#pragma unroll
+            for (int j = 0; j < NI; ++j)
+              old[u][j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, (int)oo[j], 0, 0));
+          }
+        }
+        values(iq / 4, iq % 4, v);
+        if (rd_c) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < NI; ++j) v[u][j] += g.beta * old[u][j];
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          float w = g.alpha * a4[u] + bv[u];
-          if (rd_c) w += g.beta * old[u];
-          v[u] = w;
-        }
-        if constexpr (ACT == 1) {
-          if (g.aux) {
-            if (vecs) *reinterpret_cast<f32x4*>(xp) = v;
-            else
-              for (int u = 0; u < nv; ++u) xp[(int64_t)u * g.sxn] = v[u];
+          if constexpr (ACT == 1) {
+            if (use_x) {
+              const auto r = rx.at(8 * iq + u);
+#pragma unroll
+              for (int j = 0; j < NI; ++j)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[u][j]), r, (int)xo[j], 0, 0);
+            }
           }
+          const auto r = ro.at(8 * iq + u);
 #pragma unroll
-          for (int u = 0; u < 4; ++u) v[u] = gelu_tanh_fast(v[u]);
-        } else if constexpr (ACT == 2) {
-#pragma unroll
-          for (int u = 0; u < 4; ++u) v[u] *= gelu_grad_fast(xa[u]);
-        } else if constexpr (ACT == 4) {
-          v += xa;
+          for (int j = 0; j < NI; ++j) {
+            float w = v[u][j];
+            if constexpr (ACT == 1) w = to_ws ? w : gelu_tanh_fast(w);
+            if constexpr (ACT == 2) w = use_x ? w * gelu_grad_fast(xv[iq % kAhead][u][j]) : w;
+            if constexpr (ACT == 4) w = use_x ? w + xv[iq % kAhead][u][j] : w;
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(w), r, (int)oo[j], 0, 0);
+          }
         }
-        if (vecs) *reinterpret_cast<f32x4*>(cp) = v;
-        else
-          for (int u = 0; u < nv; ++u) cp[(int64_t)u * g.scn] = v[u];
+        if (iq + kAhead < 4 * MI) aux(iq + kAhead);
       }
+    } else {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float v[4][NI];
+          values(i, q, v);
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < NI; ++j) {
+              const int m = cur.m0 + wm + 32 * i + 8 * q + 4 * lh + u, n = n1 + 32 * j + lr;
+              if (m >= g.M || n >= g.N) continue;
+              float* p = Out + (int64_t)m * so + (int64_t)n * (to_ws ? 1 : g.scn);
+              float* xp = X + (int64_t)m * g.sxm + (int64_t)n * g.sxn;
+              float w = v[u][j];
+              if (rd_c) w += g.beta * *p;
+              if constexpr (ACT == 1) {
+                if (use_x) *xp = w;
+                w = to_ws ? w : gelu_tanh_fast(w);
+              }
+              if constexpr (ACT == 2) w = use_x ? w * gelu_grad_fast(*xp) : w;
+              if constexpr (ACT == 4) w = use_x ? w + *xp : w;
+              *p = w;
+            }
+        }
     }
+
+    if (more2) {
+      SA::row_max(qa, amax[(seq + 2) & 3], tq);
+      SB::row_max(qb, amax[(seq + 2) & 3] + BM, tq);
+    }
+    if (!more) break;
+    tile += wgs;
+    cur = next;
+    if (!g.fast || !primed) __syncthreads();
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1622,40 +1761,44 @@ bool use_x3(int M, int N, int K, int batch) {
   return tiles >= 256 || K >= 1024;
 }
 
+// Two workgroups of the split kernel fit a CU.
+constexpr int kX3Wgs = 512;
+
 // Split K only when the 128 x 128 tiles leave the CUs idle (weight gradients,
-// K = B*T): aim at MTX_X3_SPLIT_TARGET workgroups (two fit a CU), each split
-// keeping >= MTX_SPLIT_MINK of K.
-#ifndef MTX_X3_SPLIT_TARGET
-#define MTX_X3_SPLIT_TARGET 576
-#endif
+// K = B*T): into as many ranges as keep one round of kX3Wgs workgroups, each
+// with >= h2::MINK of K.
 Plan plan_x3(int M, int N, int K, int batch, size_t ws_bytes) {
   Plan p{x3::T, x3::T, 1, K};
   const int64_t t = (int64_t)cdiv(M, x3::T) * cdiv(N, x3::T) * batch;
   if (t < 256 && K >= 1024) {
-    int want = (int)std::min<int64_t>(K >= 4096 ? 64 : 16, (MTX_X3_SPLIT_TARGET + t - 1) / t);
-    want = std::min(want, std::max(1, K / MTX_SPLIT_MINK));
-    const size_t need = (size_t)want * batch * (size_t)(M + 1) * N * sizeof(float);
-    if (want > 1 && need <= ws_bytes) {
-      p.kchunk = cdiv(cdiv(K, want), h2::BK) * h2::BK;
-      p.ksplit = cdiv(K, p.kchunk);
+    for (int want = (int)std::min<int64_t>(K / h2::MINK, kX3Wgs / t); want > 1; --want) {
+      const int chunk = cdiv(cdiv(K, want), h2::BK) * h2::BK, ks = cdiv(K, chunk);
+      const size_t need = (size_t)ks * batch * (size_t)(M + 1) * N * sizeof(float);
+      if (ks > 1 && K - (ks - 1) * chunk >= h2::MINK && need <= ws_bytes) {
+        p.ksplit = ks;
+        p.kchunk = chunk;
+        break;
+      }
     }
   }
   return p;
 }
 
-// Whether the two-piece form may be tried (the kernel leaves it to K ranges of
-// h2::MINK or more): 32-bit offsets reach a tile's rows and its samples' k rows.
+// Whether the two-piece form may be tried: h2::MINK of K and more in every
+// range, and 32-bit offsets reach a tile's rows and its samples' k rows.
 bool two_pieces(const GemmArgs& g) {
   const int64_t lim = (int64_t)1 << 29;
   auto ok = [&](int64_t s_row, int64_t s_k) {
     return s_row >= 0 && s_k >= 0 && (s_k == 1 ? 128 * s_row + g.kchunk : g.kchunk * s_k + 128) < lim;
   };
-  return ok(g.sam, g.sak) && ok(g.sbn, g.sbk);
+  const int last = g.K - (g.ksplit - 1) * g.kchunk;
+  return std::min(g.kchunk, last) >= h2::MINK && ok(g.sam, g.sak) && ok(g.sbn, g.sbk);
 }
 
 template <int ACT>
 void launch_x3_act(const GemmArgs& g, bool ak, bool bn1, hipStream_t st) {
-  const dim3 grid(cdiv(g.N, x3::T), cdiv(g.M, x3::T), g.batch * g.ksplit);
+  const int64_t tiles = (int64_t)cdiv(g.N, x3::T) * cdiv(g.M, x3::T) * g.batch * g.ksplit;
+  const dim3 grid((unsigned)std::min<int64_t>(tiles, kX3Wgs));
   if (ak && bn1) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, true, true, ACT>), grid, dim3(kGT), 0, st, g);
   else if (ak) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, true, false, ACT>), grid, dim3(kGT), 0, st, g);
   else if (bn1) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, false, true, ACT>), grid, dim3(kGT), 0, st, g);
@@ -1770,6 +1913,11 @@ int gemm_impl(int M, int N, int K, int batch, float alpha, const float* a, int64
   g.ksplit = p.ksplit;
   g.kchunk = p.kchunk;
   g.fast = split3 && two_pieces(g);
+  {
+    const int64_t far = (int64_t)1 << 25;
+    const bool x_ok = !act || !aux || (sx_n == 1 && sx_m >= N && sx_m < far);
+    g.rows_vec = p.ksplit > 1 ? N < far : sc_n == 1 && sc_m >= N && sc_m < far && x_ok;
+  }
   int rc = split3 ? launch_x3(g, ak, bn1, st)
                   : (p.bm == 128) ? launch_tile<128, 128>(g, ak, bn1, st) : launch_tile<64, 64>(g, ak, bn1, st);
   if (rc) return rc;

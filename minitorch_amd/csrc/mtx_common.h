@@ -61,9 +61,14 @@ __device__ __forceinline__ float gelu_tanh(float v) {
 // The same two functions with tanh(u) = 1 - 2 / (exp(2u) + 1) (one exp and
 // one reciprocal instead of tanhf's range reduction: absolute error of tanh
 // about 2e-7), for GEMM epilogues where tanhf's cost would stall the tile's
-// stores.  exp overflowing to +inf gives tanh = 1, underflowing to 0 gives -1.
+// stores.  exp underflowing to 0 gives -1; its argument is capped where tanh
+// is 1.  The reciprocal is v_rcp_f32 (1 ulp) with one Newton step (a correctly
+// rounded division takes 11 instructions, a third of the GELU epilogue's).
 __device__ __forceinline__ float tanh_fast(float u) {
-  return 1.0f - 2.0f * __frcp_rn(__expf(2.0f * u) + 1.0f);
+  const float d = __expf(fminf(2.0f * u, 80.0f)) + 1.0f;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
+  return __builtin_fmaf(-2.0f, r, 1.0f);
 }
 __device__ __forceinline__ float gelu_tanh_fast(float v) {
   const float inner = (v + v * v * v * gelu_c1()) * gelu_c0();
