@@ -101,18 +101,19 @@ __global__ __launch_bounds__(256) void reduce_kernel(const RedArgs g) {
 
 // Reduced values that lie one after another in memory (sum of everything, of
 // the last axis): a workgroup per output and chunk, its 256 threads reading
-// float4 vectors side by side, four in flight each (HBM bound).  reduce_kernel
-// gives an output four threads and a read four values: the sum of 64 x 256 x
-// 384 values took 142 + 8 us (512 chunks and their combination) against 7.9 +
-// 1.9 here (25 MB, 3.2 TB/s).
+// float4 vectors side by side, four in flight each, and adding them in
+// float64 (free beside the reads: HBM bound), so a chunk's sum is rounded
+// once.  reduce_kernel gives an output four threads and a read four values:
+// the sum of 64 x 256 x 384 values took 142 + 8 us (512 chunks and their
+// combination) against 8.2 + 2.7 here (25 MB).
 struct __attribute__((packed, aligned(4))) unaligned4 {
   float v[4];
 };
-__device__ __forceinline__ float red_op(bool is_max, float a, float b) { return is_max ? fmaxf(a, b) : a + b; }
+__device__ __forceinline__ double red_op(bool is_max, double a, double b) { return is_max ? fmax(a, b) : a + b; }
 
 // the block's 256 values in a fixed order; the result in thread 0
-__device__ __forceinline__ float block_reduce(bool is_max, float v) {
-  __shared__ float part[4];
+__device__ __forceinline__ double block_reduce(bool is_max, double v) {
+  __shared__ double part[4];
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) v = red_op(is_max, v, __shfl_xor(v, m, 64));
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
@@ -126,8 +127,8 @@ __global__ __launch_bounds__(256) void reduce_run_kernel(const RedArgs g) {
   const bool is_max = g.op == MTX_RED_MAX;
   const float* __restrict__ base = g.a + kept_offset(g, o);
   const int64_t r0 = (int64_t)s * g.chunk, r1 = min(g.nred, r0 + g.chunk);
-  const float init = is_max ? -INFINITY : 0.f;
-  float acc[4] = {init, init, init, init};
+  const double init = is_max ? -INFINITY : 0.0;
+  double acc[4] = {init, init, init, init};
   const int64_t r4 = r0 + max((int64_t)0, (r1 - r0) / 4 * 4);
   int64_t r = r0 + 4 * threadIdx.x;
   for (; r + 3 * 1024 < r4; r += 4 * 1024) {
@@ -147,7 +148,7 @@ __global__ __launch_bounds__(256) void reduce_run_kernel(const RedArgs g) {
   r = r4 + threadIdx.x;
   if (r < r1) acc[0] = red_op(is_max, acc[0], base[r]);
   const float t =
-      block_reduce(is_max, red_op(is_max, red_op(is_max, acc[0], acc[1]), red_op(is_max, acc[2], acc[3])));
+      (float)block_reduce(is_max, red_op(is_max, red_op(is_max, acc[0], acc[1]), red_op(is_max, acc[2], acc[3])));
   if (threadIdx.x != 0) return;
   if (g.nsplit > 1) {
     g.ws[(int64_t)s * g.nout + o] = t;
@@ -162,10 +163,10 @@ __global__ __launch_bounds__(256) void reduce_run_kernel(const RedArgs g) {
 __global__ __launch_bounds__(256) void reduce_run_combine_kernel(const RedArgs g) {
   const int64_t o = blockIdx.x;
   const bool is_max = g.op == MTX_RED_MAX;
-  float acc = is_max ? -INFINITY : 0.f;
+  double acc = is_max ? -INFINITY : 0.0;
 #pragma unroll 2
   for (int s = threadIdx.x; s < g.nsplit; s += 256) acc = red_op(is_max, acc, g.ws[(int64_t)s * g.nout + o]);
-  const float t = block_reduce(is_max, acc);
+  const float t = (float)block_reduce(is_max, acc);
   if (threadIdx.x != 0) return;
   float v = g.alpha * t;
   if (g.accumulate) v += g.out[o];
