@@ -500,7 +500,7 @@ int mtx_decode_step_reset(void* workspace, void* stream);
  *
  * Products with M >= 128, N >= 128 and M*N*K*batch >= 2^27 run, by default
  * (MTX_GEMM_BF16X3), on the bf16 matrix cores -- unless they have fewer than
- * 256 tiles of 128 x 128 and K < 1024; those, like smaller products, take the
+ * 64 tiles of 128 x 128 and K < 1024; those, like smaller products, take the
  * fp32 kernel -- with every fp32 operand value split into pieces and the
  * products of the pieces accumulated in fp32: for K >= 256 two fp16 pieces of
  * the value scaled by a power of two per row of A and column of B (x to 2^-23

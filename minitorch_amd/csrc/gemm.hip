@@ -433,7 +433,6 @@ __global__ __launch_bounds__(kGT) void gemm_f32_kernel(const GemmArgs g) {
 // accumulator element e of lane l is C[8(e/4) + 4(l/32) + e%4][l%32].
 // ---------------------------------------------------------------------------
 namespace x3 {
-constexpr int T = 128;  // tile rows and columns
 constexpr int BK = 16;  // k-tile depth (one MFMA k step)
 // k-contiguous rows hold two 16-byte chunks, swapped on rows 8..15 mod 16:
 // a fragment read's 16 rows then cover 16 distinct 16-byte bank groups and
@@ -1260,7 +1259,7 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
       };
       const Rows ro = rows(Out, so), rx = rows(X, g.sxm);
       // aux values are requested kAhead row groups before their use
-      constexpr int kAhead = 4;
+      constexpr int kAhead = NI > 2 ? 2 : 4;
       float xv[kAhead][4][NI];
       auto aux = [&](int iq) {
         if constexpr (ACT == 2 || ACT == 4) {
@@ -1669,7 +1668,7 @@ void launch_reduce_ln(const GemmArgs& g, const float* gamma, const float* beta_l
 }
 
 struct Plan {
-  int bm, bn, ksplit, kchunk;
+  int bm, bn, ksplit, kchunk;  // tile rows and columns, K split
 };
 
 // Pick the tile and the K split for a problem so that the launch has enough
@@ -1747,29 +1746,42 @@ std::atomic<int> g_gemm_mode{MTX_GEMM_BF16X3};
 // of 128 x 128 tiles, latency bound) stay on the fp32 kernel's 64 x 64
 // tiles: on the split kernel the C0 training step took 0.445 ms against
 // 0.379 ms.
-// Nor do products whose 128 x 128 tiles leave part of the 256 CUs idle
-// while K is too short to split (< 1024): at M = 2048 (a prefill over 64
-// prompts of 32 tokens) the fp32 kernel's 64 x 64 tiles took 28.5, 17.3 and
-// 32.0 us for q/k/v (N = 1152), out_proj (N = 384, + residual) and fc1 + GELU
-// (N = 1536), all K = 384, against 36.9, 35.7 and 41.6 us on 144, 48 and 192
-// split-kernel tiles.
+// Nor do products with fewer than 64 tiles of 128 x 128 and a K too short to
+// split (< 1024): at K = 384 the fp32 kernel's 64 x 64 tiles and the split
+// kernel took 19.8 and 20 us for 1000 x 384 (24 tiles), 24.5 and 21.9 for
+// 2944 x 384 (69), 22.9 and 19.6 for 1000 x 1152 (72), 26.7 and 25.1 for
+// 1000 x 1536 + GELU (96); 8008 x 512 x 512 (252) 48.4 and 36.4.
 bool use_x3(int M, int N, int K, int batch) {
   if (g_gemm_mode.load(std::memory_order_relaxed) != MTX_GEMM_BF16X3 || M < 128 || N < 128 ||
       (int64_t)M * N * K * batch < ((int64_t)1 << 27))
     return false;
-  const int64_t tiles = (int64_t)cdiv(M, x3::T) * cdiv(N, x3::T) * batch;
-  return tiles >= 256 || K >= 1024;
+  const int64_t tiles = (int64_t)cdiv(M, 128) * cdiv(N, 128) * batch;
+  return tiles >= 64 || K >= 1024;
 }
 
 // Two workgroups of the split kernel fit a CU.
 constexpr int kX3Wgs = 512;
+constexpr double kX3W96 = 0.8;  // a 128 x 96 tile's time against a 128 x 128 one's
 
-// Split K only when the 128 x 128 tiles leave the CUs idle (weight gradients,
-// K = B*T): into as many ranges as keep one round of kX3Wgs workgroups, each
-// with >= h2::MINK of K.
-Plan plan_x3(int M, int N, int K, int batch, size_t ws_bytes) {
-  Plan p{x3::T, x3::T, 1, K};
-  const int64_t t = (int64_t)cdiv(M, x3::T) * cdiv(N, x3::T) * batch;
+// Time of `tiles` tiles of weight w on kX3Wgs resident workgroups, in tile
+// times of two workgroups sharing a CU: whole rounds, and a last one in which
+// a workgroup that has its CU for itself is done sooner.
+double x3_rounds(int64_t tiles, double w) {
+  const int64_t rem = tiles % kX3Wgs;
+  return w * ((double)(tiles / kX3Wgs) + (rem == 0 ? 0.0 : rem <= kX3Wgs / 2 ? 0.65 : 1.0));
+}
+
+// Tiles of 128 x 128 or, where A is contiguous along k (forward and dX
+// products), 128 x 96: whichever ends sooner.  N = 384 is three columns of
+// 128 (M = 16384: 384 tiles, a round three quarters full) or four of 96
+// (512, one full round): K = 384 + residual 42.0 -> 38.5 us, K = 1536 91 ->
+// 83, its dX 84 -> 76.
+// K is split only when the 128 x 128 tiles leave the CUs idle (weight
+// gradients, K = B*T): into as many ranges as keep one round of kX3Wgs
+// workgroups, each with >= h2::MINK of K.
+Plan plan_x3(int M, int N, int K, int batch, size_t ws_bytes, bool ak, bool colsum) {
+  Plan p{128, 128, 1, K};
+  const int64_t t = (int64_t)cdiv(M, 128) * cdiv(N, 128) * batch;
   if (t < 256 && K >= 1024) {
     for (int want = (int)std::min<int64_t>(K / h2::MINK, kX3Wgs / t); want > 1; --want) {
       const int chunk = cdiv(cdiv(K, want), h2::BK) * h2::BK, ks = cdiv(K, chunk);
@@ -1780,6 +1792,9 @@ Plan plan_x3(int M, int N, int K, int batch, size_t ws_bytes) {
         break;
       }
     }
+  } else if (ak && !colsum) {
+    const int64_t t96 = (int64_t)cdiv(M, 128) * cdiv(N, 96) * batch;
+    if (x3_rounds(t96, kX3W96) < x3_rounds(t, 1.0)) p.bn = 96;
   }
   return p;
 }
@@ -1796,23 +1811,30 @@ bool two_pieces(const GemmArgs& g) {
 }
 
 template <int ACT>
-void launch_x3_act(const GemmArgs& g, bool ak, bool bn1, hipStream_t st) {
-  const int64_t tiles = (int64_t)cdiv(g.N, x3::T) * cdiv(g.M, x3::T) * g.batch * g.ksplit;
-  const dim3 grid((unsigned)std::min<int64_t>(tiles, kX3Wgs));
-  if (ak && bn1) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, true, true, ACT>), grid, dim3(kGT), 0, st, g);
-  else if (ak) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, true, false, ACT>), grid, dim3(kGT), 0, st, g);
-  else if (bn1) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, false, true, ACT>), grid, dim3(kGT), 0, st, g);
-  else hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, false, false, ACT>), grid, dim3(kGT), 0, st, g);
+void launch_x3_act(const GemmArgs& g, int bn, bool ak, bool bn1, hipStream_t st) {
+  const int64_t tiles = (int64_t)cdiv(g.N, bn) * cdiv(g.M, 128) * g.batch * g.ksplit;
+  const dim3 grid((unsigned)std::min<int64_t>(tiles, kX3Wgs)), block(kGT);
+  if constexpr (ACT != 3) {
+    if (bn == 96) {  // four waves of 32 x 96
+      if (bn1) hipLaunchKernelGGL((gemm_x3_kernel<1, 3, 4, 1, true, true, ACT>), grid, block, 0, st, g);
+      else hipLaunchKernelGGL((gemm_x3_kernel<1, 3, 4, 1, true, false, ACT>), grid, block, 0, st, g);
+      return;
+    }
+  }
+  if (ak && bn1) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, true, true, ACT>), grid, block, 0, st, g);
+  else if (ak) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, true, false, ACT>), grid, block, 0, st, g);
+  else if (bn1) hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, false, true, ACT>), grid, block, 0, st, g);
+  else hipLaunchKernelGGL((gemm_x3_kernel<2, 2, 2, 2, false, false, ACT>), grid, block, 0, st, g);
 }
 
 // as launch_tile: with split K the reduce kernel applies the activation
-int launch_x3(const GemmArgs& g, bool ak, bool bn1, hipStream_t st) {
+int launch_x3(const GemmArgs& g, int bn, bool ak, bool bn1, hipStream_t st) {
   const int act = g.ksplit > 1 ? 0 : g.act;
-  if (g.colsum) launch_x3_act<3>(g, ak, bn1, st);
-  else if (act == 1) launch_x3_act<1>(g, ak, bn1, st);
-  else if (act == 2) launch_x3_act<2>(g, ak, bn1, st);
-  else if (act == 4) launch_x3_act<4>(g, ak, bn1, st);
-  else launch_x3_act<0>(g, ak, bn1, st);
+  if (g.colsum) launch_x3_act<3>(g, bn, ak, bn1, st);
+  else if (act == 1) launch_x3_act<1>(g, bn, ak, bn1, st);
+  else if (act == 2) launch_x3_act<2>(g, bn, ak, bn1, st);
+  else if (act == 4) launch_x3_act<4>(g, bn, ak, bn1, st);
+  else launch_x3_act<0>(g, bn, ak, bn1, st);
   MTX_LAUNCHED();
   return MTX_OK;
 }
@@ -1834,7 +1856,7 @@ extern "C" size_t mtx_gemm_workspace_bytes(int M, int N, int K, int batch) {
   // column sums [split][N]
   const size_t tiled = p.ksplit > 1 ? (size_t)p.ksplit * batch * (size_t)(M + 1) * N * sizeof(float) : 0;
   // the bf16-split kernel's plan (either mode may be set when the product runs)
-  Plan q = plan_x3(M, N, K, batch, (size_t)-1);
+  Plan q = plan_x3(M, N, K, batch, (size_t)-1, false, false);
   const size_t split3 = q.ksplit > 1 ? (size_t)q.ksplit * batch * (size_t)(M + 1) * N * sizeof(float) : 0;
   return std::max({skinny, tiled, split3});
 }
@@ -1908,7 +1930,7 @@ int gemm_impl(int M, int N, int K, int batch, float alpha, const float* a, int64
   }
   const bool ak = sa_k == 1, bn1 = sb_n == 1;
   const bool split3 = use_x3(M, N, K, batch);
-  Plan p = split3 ? plan_x3(M, N, K, batch, workspace ? workspace_bytes : 0)
+  Plan p = split3 ? plan_x3(M, N, K, batch, workspace ? workspace_bytes : 0, ak, colsum != nullptr)
                   : plan_gemm(M, N, K, batch, workspace ? workspace_bytes : 0);
   g.ksplit = p.ksplit;
   g.kchunk = p.kchunk;
@@ -1918,7 +1940,7 @@ int gemm_impl(int M, int N, int K, int batch, float alpha, const float* a, int64
     const bool x_ok = !act || !aux || (sx_n == 1 && sx_m >= N && sx_m < far);
     g.rows_vec = p.ksplit > 1 ? N < far : sc_n == 1 && sc_m >= N && sc_m < far && x_ok;
   }
-  int rc = split3 ? launch_x3(g, ak, bn1, st)
+  int rc = split3 ? launch_x3(g, p.bn, ak, bn1, st)
                   : (p.bm == 128) ? launch_tile<128, 128>(g, ak, bn1, st) : launch_tile<64, 64>(g, ak, bn1, st);
   if (rc) return rc;
   return p.ksplit > 1 ? launch_splitk_reduce(g, st) : MTX_OK;
