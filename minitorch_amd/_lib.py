@@ -189,6 +189,7 @@ class MtxError(RuntimeError):
 
 
 _lib = None
+_fns: dict = {}  # the library's functions by name
 
 
 def lib():
@@ -204,6 +205,7 @@ def lib():
             fn = getattr(handle, name)
             fn.restype = res
             fn.argtypes = args
+            _fns[name] = fn
         _lib = handle
     return _lib
 
@@ -221,7 +223,12 @@ def check(fn_name: str, status: int) -> None:
 
 
 def call(fn_name: str, *args) -> None:
-    check(fn_name, getattr(lib(), fn_name)(*args))
+    fn = _fns.get(fn_name)
+    if fn is None:
+        fn = getattr(lib(), fn_name)
+    status = fn(*args)
+    if status != MTX_OK:
+        check(fn_name, status)
 
 
 # ---------------------------------------------------------------------------
@@ -241,7 +248,7 @@ def strides(t) -> C.Array:
 
 
 def ptr(t):
-    return C.c_void_p(t.data_ptr())
+    return t.data_ptr()  # an address; the void* arguments take integers
 
 
 def stream_handle(device=None):

@@ -21,8 +21,7 @@ it (back to the library's cache) when the last view goes away.
 from __future__ import annotations
 
 import ctypes as C
-from functools import reduce
-from operator import mul
+import math
 
 import numpy as np
 
@@ -38,6 +37,8 @@ def dtype_name(x) -> str:
     of a DevBuf / DeviceArray, a NumPy dtype or type, a name, or any array
     object whose ``dtype`` prints like one (e.g. a framework tensor a test
     passes in)."""
+    if type(x) is DevBuf:
+        return x.dtype
     d = x if isinstance(x, (str, type, np.dtype)) else getattr(x, "dtype", x)
     if isinstance(d, str):
         name = d
@@ -81,40 +82,42 @@ class _Storage:
     __slots__ = ("ptr", "nbytes", "__weakref__")
 
     def __init__(self, nbytes: int):
-        device()
+        if not _READY:
+            device()
         p = C.c_void_p()
-        L.call("mtx_malloc", C.byref(p), max(1, int(nbytes)))
+        L.call("mtx_malloc", C.byref(p), max(1, nbytes))
         self.ptr = p.value
-        self.nbytes = int(nbytes)
+        self.nbytes = nbytes
 
     def __del__(self):
         try:
             if self.ptr:
-                L.lib().mtx_free(C.c_void_p(self.ptr))
+                L.lib().mtx_free(self.ptr)
                 self.ptr = 0
         except Exception:  # interpreter shutdown: the process frees everything
             pass
 
 
-def _prod(shape):
-    return reduce(mul, shape, 1)
+_prod = math.prod
 
 
 def _contig_strides(shape):
     st, acc = [], 1
-    for s in reversed(shape):
+    for s in shape[::-1]:
         st.append(acc)
-        acc *= max(int(s), 1)
-    return tuple(reversed(st))
+        if s > 1:
+            acc *= s
+    st.reverse()
+    return tuple(st)
 
 
 def _norm_shape(shape, numel=None):
     if len(shape) == 1 and isinstance(shape[0], (tuple, list)):
-        shape = tuple(shape[0])
-    shape = tuple(int(s) for s in shape)
-    if shape.count(-1) > 1:
-        raise ValueError("only one dimension can be inferred")
+        shape = shape[0]
+    shape = tuple(map(int, shape))
     if -1 in shape:
+        if shape.count(-1) > 1:
+            raise ValueError("only one dimension can be inferred")
         if numel is None:
             raise ValueError("cannot infer a dimension here")
         rest = _prod([s for s in shape if s != -1])
@@ -194,8 +197,8 @@ class DevBuf:
 
     def is_contiguous(self) -> bool:
         acc = 1
-        for s, st in zip(reversed(self.shape), reversed(self._strides)):
-            if s != 1 and st != acc:
+        for s, st in zip(self.shape[::-1], self._strides[::-1]):
+            if st != acc and s != 1:
                 return False
             acc *= s
         return True
@@ -207,19 +210,34 @@ class DevBuf:
         return f"DevBuf(shape={self.shape}, strides={self._strides}, dtype={self.dtype})"
 
     def _with(self, off, shape, strides):
-        return DevBuf(self._st, off, shape, strides, self.dtype)
+        """A view of the same allocation; shape and strides hold ints (the
+        views' own arithmetic), so nothing is converted."""
+        b = _new_buf(DevBuf)
+        b._st = self._st
+        b._off = off
+        b.shape = shape if type(shape) is tuple else tuple(shape)
+        b._strides = strides if type(strides) is tuple else tuple(strides)
+        b.dtype = self.dtype
+        return b
 
     # -- views (no copies) ------------------------------------------------------
+    def _restride(self, shape):
+        """Strides that present these elements in `shape` without a copy, or
+        None: C order's for a contiguous array, _view_strides' else."""
+        if self.is_contiguous() and _prod(shape) == self.numel():
+            return _contig_strides(shape)
+        return _view_strides(self.shape, self._strides, shape)
+
     def view(self, *shape):
         shape = _norm_shape(shape, self.numel())
-        st = _view_strides(self.shape, self._strides, shape)
+        st = self._restride(shape)
         if st is None:
             raise RuntimeError(f"view of shape {shape} needs a copy (strides {self._strides}); use reshape")
         return self._with(self._off, shape, st)
 
     def reshape(self, *shape):
         shape = _norm_shape(shape, self.numel())
-        st = _view_strides(self.shape, self._strides, shape)
+        st = self._restride(shape)
         if st is None:
             return self.contiguous().view(*shape)
         return self._with(self._off, shape, st)
@@ -258,7 +276,8 @@ class DevBuf:
     def as_strided(self, shape, strides, offset=None):
         """The same memory seen with explicit shape / element strides (and
         element offset from the allocation's start)."""
-        return self._with(self._off if offset is None else offset, shape, strides)
+        return self._with(self._off if offset is None else int(offset), tuple(map(int, shape)),
+                          tuple(map(int, strides)))
 
     def squeeze(self, d: int):
         d = d % self.dim()
@@ -269,7 +288,7 @@ class DevBuf:
     def unflatten(self, d: int, sizes):
         """Split dimension d into `sizes` (a view)."""
         d = d % self.dim()
-        sizes = tuple(int(x) for x in sizes)
+        sizes = tuple(map(int, sizes))
         if _prod(sizes) != self.shape[d]:
             raise ValueError(f"cannot unflatten size {self.shape[d]} into {sizes}")
         st = self._strides[d]
@@ -420,11 +439,20 @@ def host_array(a, dtype: str) -> np.ndarray:
     return np.ascontiguousarray(np.asarray(a, dtype=_HOST[dtype]))
 
 
+_new_buf = DevBuf.__new__
+
+
 def empty_buf(shape, dtype="float32") -> DevBuf:
-    dtype = dtype_name(dtype)
-    shape = tuple(int(s) for s in shape)
-    st = _Storage(_prod(shape) * ITEMSIZE[dtype])
-    return DevBuf(st, 0, shape, _contig_strides(shape), dtype)
+    if type(dtype) is not str or dtype not in ITEMSIZE:
+        dtype = dtype_name(dtype)
+    shape = tuple(map(int, shape))
+    b = _new_buf(DevBuf)
+    b._st = _Storage(_prod(shape) * ITEMSIZE[dtype])
+    b._off = 0
+    b.shape = shape
+    b._strides = _contig_strides(shape)
+    b.dtype = dtype
+    return b
 
 
 def empty_like_layout(t, dtype="float32") -> DevBuf:
@@ -453,11 +481,12 @@ class DeviceArray:
     # -- numpy-like metadata ------------------------------------------------
     @property
     def shape(self):
-        return tuple(self.t.shape)
+        s = self.t.shape
+        return s if type(s) is tuple else tuple(s)
 
     @property
     def ndim(self):
-        return self.t.dim()
+        return len(self.t.shape)
 
     @property
     def size(self):

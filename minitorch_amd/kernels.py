@@ -9,6 +9,7 @@ arguments, found before any HIP call) or ``MtxError`` (HIP failure).
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import numpy as np
 
@@ -471,7 +472,7 @@ def attn_bwd_noalloc(q, k, v, out, dout, lse, scale: float, causal: bool, dq, dk
 # ---------------------------------------------------------------------------
 
 def _i64(seq):
-    seq = tuple(int(x) for x in seq)
+    seq = tuple(map(int, seq))
     return (L.C.c_int64 * max(1, len(seq)))(*seq)
 
 
@@ -482,6 +483,8 @@ def _bstrides(t, shape):
     pad = nd - len(ts)
     if pad < 0:
         raise ValueError(f"cannot broadcast shape {ts} to {tuple(shape)}")
+    if ts == shape:
+        return [st if sz != 1 else 0 for sz, st in zip(ts, tst)]
     out = []
     for d in range(nd):
         if d < pad:
@@ -629,6 +632,12 @@ def attn_bwd_onepass_used(dtype: str, D: int) -> bool:
     return dtype == "bfloat16" and D <= 64 and get_attn_bwd_mode() == ATTN_BWD_ONEPASS
 
 
+@functools.lru_cache(maxsize=512)
+def _gemm_workspace_bytes(M, N, K, batch):
+    """mtx_gemm_workspace_bytes, a function of the sizes alone."""
+    return L.lib().mtx_gemm_workspace_bytes(M, N, K, batch)
+
+
 def gemm(a, b, c, alpha=1.0, beta=0.0, bias=None, M=None, N=None, K=None, batch=1,
          sa=None, sb=None, sc=None, act=GEMM_ACT_NONE, aux=None, colsum=None, colsum_accumulate=False):
     """C = alpha*A@B + beta*C (+bias) with explicit (row, col, batch) strides
@@ -652,7 +661,7 @@ def gemm(a, b, c, alpha=1.0, beta=0.0, bias=None, M=None, N=None, K=None, batch=
         if t is not None and _dt(t) != "float32":
             raise ValueError(f"gemm: {name} must be fp32 (got {t.dtype})")
     # one operand stride must be unit; otherwise the caller passes a copy
-    ws_bytes = L.lib().mtx_gemm_workspace_bytes(M, N, K, batch)
+    ws_bytes = _gemm_workspace_bytes(int(M), int(N), int(K), int(batch))
     ws = dev.empty_buf((ws_bytes,), "uint8") if ws_bytes else None
     if colsum is not None:
         if batch != 1 or alpha != 1.0 or bias is not None or act != GEMM_ACT_NONE:
