@@ -1000,7 +1000,7 @@ constexpr int dkdv_waves() { return sizeof(T) == 2 ? MTX_DKDV_WAVES : kWaves; }
 // (An issue order that keeps all key blocks of a slice consecutively on one
 // XCD, so that fewer slices take atomic adds at a time, measured the same.)
 template <typename T, int D, int NK, bool DROP, bool FQ = false>
-__global__ __launch_bounds__(64 * dkdv_waves<T>(), ((D == 128 && sizeof(T) == 4) || (is_x3<T>() && D == 64 && MTX_X3_DKDV_WAVES1)) ? 1 : 2) void attn_dkdv_kernel(const BwdArgs a) {
+__global__ __launch_bounds__(64 * dkdv_waves<T>(), ((D == 128 && sizeof(T) == 4) || (is_x3<T>() && D == 64 && MTX_X3_DKDV_WAVES1) || (D == 128 && NK == 2)) ? 1 : 2) void attn_dkdv_kernel(const BwdArgs a) {
   using MF = Mfma<T>;
   using frag = typename MF::frag;
   using DM = DMap<T, D>;
@@ -1808,6 +1808,23 @@ int launch_onepass(const BwdArgs& a, int phases, hipStream_t st) {
   }
 }
 
+// bf16 with 128-wide heads: two 16-query (dQ) or 16-key (dK/dV) sub-blocks per
+// wave read each LDS fragment for two products instead of one, which is what
+// bounds these passes (64 KB of fragments per wave and tile for 64 products),
+// at the price of 220 bytes of spilled registers (dQ) or one wave per SIMD
+// instead of two (dK/dV).  One and two sub-blocks measured, us, dQ: 90 and
+// 76-80 at (B, H, T) = (4, 12, 1531), 352 and 262 at (8, 16, 2048), 169 and 151
+// at (2, 8, 4096), 84 and 72 at (8, 12, 1000), 156 and 145 at (32, 12, 600), but
+// 37 and 44 at (4, 8, 1000) and 122 and 127 at (1, 8, 4000), whose 256
+// 128-row blocks leave half of the chip's workgroup slots empty, and 115 and
+// 138 at (64, 12, 300), whose third block is a third full; dK/dV: 458 and 424 at
+// (8, 16, 2048), 208 and 185 at (2, 8, 4096), the same at (4, 12, 1531), 110 and
+// 114 at (64, 12, 200).
+template <typename T, int D>
+bool two_sub_blocks(const BwdArgs& a, int rows, int least) {
+  return sizeof(T) == 2 && D == 128 && !a.keep && rows >= least && (int64_t)cdiv(rows, 128) * a.B * a.H >= 512;
+}
+
 // Phase order: delta, dQ, dK/dV.  DELTA together with DQ runs as one
 // kernel (the dQ pass computes delta for its rows and stores it), which the
 // dK/dV pass then reads.
@@ -1828,7 +1845,13 @@ int launch_bwd(const BwdArgs& a, int phases, hipStream_t st) {
   }
   if (phases & MTX_ATTN_BWD_DQ) {
     const int gq = cdiv(a.Tq, kWaves * NQ * 16) * a.B * a.H;
-    if (a.keep) {
+    if (two_sub_blocks<T, D>(a, a.Tq, 512)) {
+      if constexpr (sizeof(T) == 2 && D == 128) {
+        const int g2 = cdiv(a.Tq, kWaves * 32) * a.B * a.H;
+        if (fuse) hipLaunchKernelGGL((attn_dq_kernel<T, D, 2, true, false>), dim3(g2), dim3(kThreads), 0, st, a);
+        else hipLaunchKernelGGL((attn_dq_kernel<T, D, 2, false, false>), dim3(g2), dim3(kThreads), 0, st, a);
+      }
+    } else if (a.keep) {
       if (fuse)
         hipLaunchKernelGGL((attn_dq_kernel<T, D, NQ, true, true>), dim3(gq), dim3(kThreads), 0, st, a);
       else
@@ -1844,7 +1867,11 @@ int launch_bwd(const BwdArgs& a, int phases, hipStream_t st) {
   if (phases & MTX_ATTN_BWD_DKDV) {
     constexpr int NWV = dkdv_waves<T>();
     const int gk = cdiv(a.Tk, NWV * NK * 16) * a.B * a.H;
-    if (a.keep)
+    if (two_sub_blocks<T, D>(a, a.Tk, 1792)) {
+      if constexpr (sizeof(T) == 2 && D == 128)
+        hipLaunchKernelGGL((attn_dkdv_kernel<T, D, 2, false>), dim3(cdiv(a.Tk, NWV * 32) * a.B * a.H), dim3(64 * NWV),
+                           0, st, a);
+    } else if (a.keep)
       hipLaunchKernelGGL((attn_dkdv_kernel<T, D, NK, true>), dim3(gk), dim3(64 * NWV), 0, st, a);
     else
       hipLaunchKernelGGL((attn_dkdv_kernel<T, D, NK, false>), dim3(gk), dim3(64 * NWV), 0, st, a);

@@ -470,6 +470,30 @@ def test_bf16_elementwise_ragged_t(dev):
                 [(b, h) for b in range(B) for h in range(H)])
 
 
+@pytest.mark.parametrize("B,H,Tq,Tk,causal", [(8, 13, 513, 513, True), (8, 13, 520, 700, True),
+                                              (4, 26, 577, 577, False), (5, 7, 1793, 1793, True),
+                                              (2, 18, 1800, 1913, True)])
+def test_bf16_wide_heads_two_sub_blocks(dev, B, H, Tq, Tk, causal):
+    """128-wide heads in enough and long enough slices that the backward's
+    waves take two sub-blocks each (dQ from 512 queries, dK/dV from 1792 keys,
+    512 blocks of 128 rows): the first and last slice against the emulation,
+    and those two slices in a launch of their own (one sub-block per wave)."""
+    D = 128
+    _say(f"[attn bf16 two sub-blocks] B={B} H={H} Tq={Tq} Tk={Tk} causal={causal}")
+    rng = np.random.default_rng(Tq + Tk)
+    q, do = (bf16_round(s * rng.standard_normal((B, H, Tq, D), dtype=np.float32)) for s in (0.5, 1.0))
+    k, v = (bf16_round(0.5 * rng.standard_normal((B, H, Tk, D), dtype=np.float32)) for _ in range(2))
+    scale = 1.0 / math.sqrt(D)
+    got = _run(dev, q, k, v, do, scale, causal, "bfloat16")
+    for b, h in ((0, 0), (B - 1, H - 1)):
+        one = [np.ascontiguousarray(x[b:b + 1, h:h + 1]) for x in (q, k, v, do)]
+        emu = attention_bf16_emulated(*one, scale, causal)
+        alone = _run(dev, *one, scale, causal, "bfloat16")
+        for name, g, e, a in zip(("o", "dq", "dk", "dv", "lse"), got, (emu[0], *emu[2:], emu[1]), alone):
+            _emu_bar(g[b, h], e[0, 0], f"{name}[{b},{h}]")
+            _emu_bar(g[b, h], a[0, 0].astype(np.float64), f"{name}[{b},{h}] vs alone")
+
+
 def test_c3_full(dev):
     """Config C3: B=8, H=16, T=2048, D=64; q,k,v = 0.5*N(0,1), dO = N(0,1), all
     rounded to bf16, drawn in that order from default_rng(3).  All 128 (b,h)
