@@ -262,16 +262,13 @@ struct Lay<f32x3_t, D> : Lay<bf16_t, D> {
 
 // eight fp32 values -> three bf16x8 pieces
 __device__ __forceinline__ Frag3 split8(const float (&v)[8]) {
+  uint2 h[2], m[2], l[2];
+  split3(f32x4{v[0], v[1], v[2], v[3]}, h[0], m[0], l[0]);
+  split3(f32x4{v[4], v[5], v[6], v[7]}, h[1], m[1], l[1]);
   Frag3 f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const __bf16 h = (__bf16)v[e];
-    const float r1 = v[e] - (float)h;
-    const __bf16 m = (__bf16)r1;
-    f.p[0][e] = h;
-    f.p[1][e] = m;
-    f.p[2][e] = (__bf16)(r1 - (float)m);
-  }
+  f.p[0] = __builtin_bit_cast(bf16x8, make_uint4(h[0].x, h[0].y, h[1].x, h[1].y));
+  f.p[1] = __builtin_bit_cast(bf16x8, make_uint4(m[0].x, m[0].y, m[1].x, m[1].y));
+  f.p[2] = __builtin_bit_cast(bf16x8, make_uint4(l[0].x, l[0].y, l[1].x, l[1].y));
   return f;
 }
 
@@ -306,18 +303,7 @@ struct TileRegsX3 {
       const int rr = c / CPR, cc = c % CPR;
       const int o = LY::at(rr, 4 * cc);
       uint2 h, m, l;
-      h.x = pack_bf2(r[i][0], r[i][1]);
-      h.y = pack_bf2(r[i][2], r[i][3]);
-      float d0 = r[i][0] - __uint_as_float(h.x << 16), d1 = r[i][1] - __uint_as_float(h.x & 0xffff0000u);
-      float d2 = r[i][2] - __uint_as_float(h.y << 16), d3 = r[i][3] - __uint_as_float(h.y & 0xffff0000u);
-      m.x = pack_bf2(d0, d1);
-      m.y = pack_bf2(d2, d3);
-      d0 -= __uint_as_float(m.x << 16);
-      d1 -= __uint_as_float(m.x & 0xffff0000u);
-      d2 -= __uint_as_float(m.y << 16);
-      d3 -= __uint_as_float(m.y & 0xffff0000u);
-      l.x = pack_bf2(d0, d1);
-      l.y = pack_bf2(d2, d3);
+      split3(r[i], h, m, l);
       *reinterpret_cast<uint2*>(buf + o) = h;
       *reinterpret_cast<uint2*>(buf + Lay<f32x3_t, D>::PS + o) = m;
       *reinterpret_cast<uint2*>(buf + 2 * Lay<f32x3_t, D>::PS + o) = l;

@@ -444,31 +444,6 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-// two bf16 values in a register; opaque to the compiler, which otherwise
-// converts the low one a second time to shift it out of the pair
-__device__ __forceinline__ uint32_t pk_bf16(float x, float y) {
-  bf16x2 v = {(__bf16)x, (__bf16)y};
-  uint32_t u = __builtin_bit_cast(uint32_t, v);
-  asm("" : "+v"(u));
-  return u;
-}
-
-// x = h + m + l (+ 2^-24 |x|), for four values, each plane as four bf16
-__device__ __forceinline__ void split3(f32x4 v, uint2& h, uint2& m, uint2& l) {
-  h.x = pk_bf16(v[0], v[1]);
-  h.y = pk_bf16(v[2], v[3]);
-  float r0 = v[0] - __uint_as_float(h.x << 16), r1 = v[1] - __uint_as_float(h.x & 0xffff0000u);
-  float r2 = v[2] - __uint_as_float(h.y << 16), r3 = v[3] - __uint_as_float(h.y & 0xffff0000u);
-  m.x = pk_bf16(r0, r1);
-  m.y = pk_bf16(r2, r3);
-  r0 -= __uint_as_float(m.x << 16);
-  r1 -= __uint_as_float(m.x & 0xffff0000u);
-  r2 -= __uint_as_float(m.y << 16);
-  r3 -= __uint_as_float(m.y & 0xffff0000u);
-  l.x = pk_bf16(r0, r1);
-  l.y = pk_bf16(r2, r3);
-}
-
 // One operand's R x 16 tile (rows = m for A, n for B).  KC: contiguous along
 // k in global memory (rows strided by srow); else contiguous along the rows
 // (k strided by sk).  The tile is R*4 float4 vectors; slot i of a thread is
