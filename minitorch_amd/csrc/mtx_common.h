@@ -58,26 +58,33 @@ __device__ __forceinline__ float gelu_tanh(float v) {
   const float inner = (v + v * v * v * gelu_c1()) * gelu_c0();
   return v * 0.5f * (tanhf(inner) + 1.0f);
 }
-// The same two functions with tanh(u) = 1 - 2 / (exp(2u) + 1) (one exp and
-// one reciprocal instead of tanhf's range reduction: absolute error of tanh
-// about 2e-7), for GEMM epilogues where tanhf's cost would stall the tile's
-// stores.  exp underflowing to 0 gives -1; its argument is capped where tanh
-// is 1.  The reciprocal is v_rcp_f32 (1 ulp) with one Newton step (a correctly
-// rounded division takes 11 instructions, a third of the GELU epilogue's).
-__device__ __forceinline__ float tanh_fast(float u) {
-  const float d = __expf(fminf(2.0f * u, 80.0f)) + 1.0f;
-  float r = __builtin_amdgcn_rcpf(d);
+// GELU and its derivative for GEMM epilogues, from one exp2 and one
+// reciprocal: with e = exp(2u), u = c0 (v + c1 v^3), r = 1 / (1 + e) and s = e r,
+// 0.5 (1 + tanh u) = s and 1 - tanh(u)^2 = 4 s r, so gelu = v s and gelu' =
+// s (1 + 2 c0 (1 + 3 c1 v^2) v r): no cancellation for negative v, and 10 and 14
+// instructions (through tanh 17 and 25, which bounded those epilogues).  From
+// v = 8 on s is 1 and r below 2^-71; the reciprocal is v_rcp_f32 (1 ulp) with one
+// Newton step.
+__device__ __forceinline__ void gelu_sr(float v, float& w, float& s, float& r) {
+  const float vc = fminf(v, 8.0f);
+  w = vc * vc;
+  constexpr float k0 = 2.302208198f, k1 = 0.10294323895f;  // 2 c0 log2(e), and times c1
+  const float e = __builtin_amdgcn_exp2f(vc * __builtin_fmaf(k1, w, k0));
+  const float d = e + 1.0f;
+  r = __builtin_amdgcn_rcpf(d);
   r = __builtin_fmaf(__builtin_fmaf(-d, r, 1.0f), r, r);
-  return __builtin_fmaf(-2.0f, r, 1.0f);
+  s = e * r;
 }
 __device__ __forceinline__ float gelu_tanh_fast(float v) {
-  const float inner = (v + v * v * v * gelu_c1()) * gelu_c0();
-  return v * 0.5f * (tanh_fast(inner) + 1.0f);
+  float w, s, r;
+  gelu_sr(v, w, s, r);
+  return v * s;
 }
 __device__ __forceinline__ float gelu_grad_fast(float v) {
-  const float inner = (v + v * v * v * gelu_c1()) * gelu_c0();
-  const float t = tanh_fast(inner);
-  return 0.5f * (t + 1.0f) + 0.5f * v * (1.0f - t * t) * gelu_c0() * (1.0f + 3.0f * gelu_c1() * v * v);
+  float w, s, r;
+  gelu_sr(v, w, s, r);
+  const float q = __builtin_fmaf(6.0f * 0.7978845834732056f * 0.044714998453855515f, w, 2.0f * 0.7978845834732056f);
+  return __builtin_fmaf(s, q * v * r, s);
 }
 // d gelu_tanh / dv: the product rule through 0.5 v (1 + tanh(u)),
 // u = c0 (v + c1 v^3) (the reference's gelu backward, functional.py:54-59
