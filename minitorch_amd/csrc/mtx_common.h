@@ -62,11 +62,13 @@ __device__ __forceinline__ float gelu_tanh(float v) {
 // reciprocal: with e = exp(2u), u = c0 (v + c1 v^3), r = 1 / (1 + e) and s = e r,
 // 0.5 (1 + tanh u) = s and 1 - tanh(u)^2 = 4 s r, so gelu = v s and gelu' =
 // s (1 + 2 c0 (1 + 3 c1 v^2) v r): no cancellation for negative v, and 10 and 14
-// instructions (through tanh 17 and 25, which bounded those epilogues).  From
-// v = 8 on s is 1 and r below 2^-71; the reciprocal is v_rcp_f32 (1 ulp) with one
-// Newton step.
-__device__ __forceinline__ void gelu_sr(float v, float& w, float& s, float& r) {
-  const float vc = fminf(v, 8.0f);
+// instructions (through tanh 17 and 25, which bounded those epilogues), and
+// one for the lower bound of vc: from v = 8 on s is 1 and r below 2^-71, up to
+// v = -12 s is 0, and a v further out (1e13 and more) would overflow v^3, Inf
+// times that 0 or r.  The bounds keep NaN.  The reciprocal is v_rcp_f32 (1
+// ulp) with one Newton step.
+__device__ __forceinline__ void gelu_sr(float v, float& vc, float& w, float& s, float& r) {
+  vc = __builtin_elementwise_maximum(__builtin_elementwise_minimum(v, 8.0f), -12.0f);
   w = vc * vc;
   constexpr float k0 = 2.302208198f, k1 = 0.10294323895f;  // 2 c0 log2(e), and times c1
   const float e = __builtin_amdgcn_exp2f(vc * __builtin_fmaf(k1, w, k0));
@@ -76,15 +78,15 @@ __device__ __forceinline__ void gelu_sr(float v, float& w, float& s, float& r) {
   s = e * r;
 }
 __device__ __forceinline__ float gelu_tanh_fast(float v) {
-  float w, s, r;
-  gelu_sr(v, w, s, r);
+  float vc, w, s, r;
+  gelu_sr(v, vc, w, s, r);
   return v * s;
 }
 __device__ __forceinline__ float gelu_grad_fast(float v) {
-  float w, s, r;
-  gelu_sr(v, w, s, r);
+  float vc, w, s, r;
+  gelu_sr(v, vc, w, s, r);
   const float q = __builtin_fmaf(6.0f * 0.7978845834732056f * 0.044714998453855515f, w, 2.0f * 0.7978845834732056f);
-  return __builtin_fmaf(s, q * v * r, s);
+  return __builtin_fmaf(s, q * vc * r, s);
 }
 // d gelu_tanh / dv: the product rule through 0.5 v (1 + tanh(u)),
 // u = c0 (v + c1 v^3) (the reference's gelu backward, functional.py:54-59

@@ -553,6 +553,32 @@ def test_gemm_gelu_epilogues(dev, gemm_mode, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(70, 65, 40), (2048, 2048, 256), (128, 512, 8192)])
+def test_gemm_gelu_far_values(dev, M, N, K):
+    """The GELU epilogues far from zero, in the fp32 kernel, the split kernel
+    and the split-K reduce: GELU' is 1 (to a rounded reciprocal and two
+    products, 2^-22) or 0 there and NaN of NaN, GELU the value itself or 0, up
+    to where fp32's v^2 and v^3 overflow."""
+    from minitorch_amd import kernels as K_
+
+    _say(f"[gemm gelu far] M={M} N={N} K={K}")
+    rng = np.random.default_rng(M)
+    a, b = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((K, N), dtype=np.float32)
+    far = np.array([9, 20, 1e6, 1e13, 1e15, 1e18, 3e18, 3e20, 1e38], np.float32)
+    col = np.concatenate([far, -far[1:], [np.nan]])
+    h = np.resize(col, N)
+    p, d, c = (empty((M, N)) for _ in range(3))
+    K_.gemm(_T(a), _T(b), p)
+    K_.gemm(_T(a), _T(b), d, act=K_.GEMM_ACT_GELU_BWD, aux=_T(np.broadcast_to(h, (M, N)).copy()))
+    want = np.where(np.isnan(h), np.nan, (h > 0).astype(np.float32)) * p.numpy()
+    np.testing.assert_allclose(d.numpy(), want, rtol=2.0 ** -22, atol=0)
+    # a zero product plus the values as its bias
+    K_.gemm(_T(np.zeros_like(a)), _T(b), c, bias=_T(h), act=K_.GEMM_ACT_GELU)
+    want = np.broadcast_to(np.where(np.isnan(h) | (h > 0), h, 0), (M, N))
+    np.testing.assert_allclose(c.numpy(), want, rtol=2.0 ** -22, atol=0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,acc", [(384, 1152, 16384, False), (384, 65, 4096, True), (200, 130, 777, False),
                                        (64, 48, 300, True), (7, 5, 3, False), (384, 384, 0, True),
                                        (130, 300, 4001, True), (1536, 384, 16384, False)])
