@@ -273,8 +273,8 @@ extern "C" int mtx_reduce_f32(int op, int ndim, const int64_t* shape, const floa
   // Runs of 256 values and more (shorter ones leave most of a workgroup's
   // threads without a value), in chunks of 16384 and more: the mean of 16384
   // row losses took 4.1 + 4.9 us in 256 chunks of reduce_kernel's, one
-  // workgroup 4.0.
-  if (g.nr == 1 && g.rstr[0] == 1 && nred >= 256 && nout < (1 << 30)) {
+  // workgroup 4.0.  (A launch has fewer than 2^32 threads.)
+  if (g.nr == 1 && g.rstr[0] == 1 && nred >= 256 && nout < (1 << 24)) {
     s = (int)std::max<int64_t>(1, std::min<int64_t>(s, nred / 16384));
     g.nsplit = s;
     g.chunk = (nred + s - 1) / s;

@@ -164,6 +164,19 @@ def test_reduce_contiguous_runs(dev, rows, n, pad):
     assert np.array_equal(H(mx), a[:, pad:].max(1))
 
 
+def test_reduce_runs_of_many_outputs(dev):
+    """2^24 outputs (one row of 256 values, repeated by a stride of 0): a
+    workgroup each would be 2^32 threads, more than a launch takes."""
+    from minitorch_amd import kernels as Kn
+
+    _say("[reduce runs, 2^24 outputs]")
+    row = np.arange(256, dtype=np.float32)
+    ta = T(row).as_strided((1 << 24, 256), (0, 1))
+    out = empty((1 << 24,))
+    Kn.reduce(ta, [1], out)
+    assert np.all(H(out) == row.sum())
+
+
 def test_reduce_merged_dims_bit_identical(dev):
     """Reducing (B, T, C) over (B, T) merges the two reduced dims into one of
     B*T rows; the result must be bit-identical to reducing the (B*T, C) view,
