@@ -224,10 +224,11 @@ __device__ __forceinline__ void ln_row_lds(float* __restrict__ row, int C, int l
   }
   float mean, sd;
   ln_stats<16>(v, lane, C, pl.eps, mean, sd);
+  const Divisor by_sd(sd);
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const int n = lane + 64 * i;
-    if (n < C) row[n] = ln_apply(v[i], sd, pl.gamma[n], pl.beta[n]);
+    if (n < C) row[n] = ln_apply(v[i], by_sd, pl.gamma[n], pl.beta[n]);
   }
 }
 
@@ -615,10 +616,11 @@ __global__ __launch_bounds__(64) void embed2_ln_kernel(const float* __restrict__
   }
   float mean, sd;
   ln_stats<VPL>(v, lane, C, eps, mean, sd);
+  const Divisor by_sd(sd);
 #pragma unroll
   for (int j = 0; j < VPL; ++j) {
     const int c = lane + 64 * j;
-    if (c < C) y[i * ldy + c] = ln_apply(v[j], sd, gamma[c], beta[c]);
+    if (c < C) y[i * ldy + c] = ln_apply(v[j], by_sd, gamma[c], beta[c]);
   }
 }
 

@@ -206,8 +206,9 @@ __device__ __forceinline__ void ps_ln_row(float* __restrict__ row, int lane, con
   }
   float mean, sd;
   ln_stats<kPsMaxC / 64>(v, lane, C, eps, mean, sd);
+  const Divisor by_sd(sd);
 #pragma unroll
-  for (int i = 0; i < C / 64; ++i) row[lane + 64 * i] = ln_apply(v[i], sd, p.g[i], p.b[i]);
+  for (int i = 0; i < C / 64; ++i) row[lane + 64 * i] = ln_apply(v[i], by_sd, p.g[i], p.b[i]);
 }
 
 // Element n of row b entering a block after the first: the residual X0[b]

@@ -418,7 +418,6 @@ __global__ __launch_bounds__(kGT) void gemm_f32_kernel(const GemmArgs g) {
 // v_mfma_f32_16x16x4_f32 (16 x 32 cycles): 2.7x the fp32 matrix rate.
 // Non-finite inputs give NaN (x - x0 is Inf - Inf).
 //
-//
 // Two fp16 pieces do the same in three products where the values' range
 // allows (h2 below), and this form stays as what those tiles fall back to and
 // for short products.
@@ -1616,11 +1615,12 @@ __global__ __launch_bounds__(64) void splitk_reduce_ln_kernel(const GemmArgs g, 
   }
   float mean, sd;
   ln_stats<VPL>(v, lane, g.N, eps, mean, sd);
+  const Divisor by_sd(sd);
   float* yr = y + (int64_t)m * ldy;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int n = lane + 64 * i;
-    if (n < g.N) yr[n] = ln_apply(v[i], sd, gamma[n], beta_ln[n]);
+    if (n < g.N) yr[n] = ln_apply(v[i], by_sd, gamma[n], beta_ln[n]);
   }
 }
 
@@ -1712,8 +1712,8 @@ int launch_tile(const GemmArgs& g, bool ak, bool bn1, hipStream_t st) {
 }
 
 // Which kernel computes fp32 products of at least 128 x 128 (mtx_gemm_set_mode):
-// MTX_GEMM_BF16X3 (default) the three-piece bf16 split on the bf16 matrix
-// cores, MTX_GEMM_FP32 the fp32 MFMA tile kernel.  Smaller products, and
+// MTX_GEMM_BF16X3 (default) the split kernel on the 16-bit matrix cores (two
+// fp16 or three bf16 pieces), MTX_GEMM_FP32 the fp32 MFMA tile kernel.  Smaller products, and
 // the decode step's skinny ones, always take the fp32 kernels.
 std::atomic<int> g_gemm_mode{MTX_GEMM_BF16X3};
 
@@ -1830,7 +1830,7 @@ extern "C" size_t mtx_gemm_workspace_bytes(int M, int N, int K, int batch) {
   // split partials [split][batch][M][N], then the weight-gradient variant's
   // column sums [split][N]
   const size_t tiled = p.ksplit > 1 ? (size_t)p.ksplit * batch * (size_t)(M + 1) * N * sizeof(float) : 0;
-  // the bf16-split kernel's plan (either mode may be set when the product runs)
+  // the split kernel's plan (either mode may be set when the product runs)
   Plan q = plan_x3(M, N, K, batch, (size_t)-1, false, false);
   const size_t split3 = q.ksplit > 1 ? (size_t)q.ksplit * batch * (size_t)(M + 1) * N * sizeof(float) : 0;
   return std::max({skinny, tiled, split3});

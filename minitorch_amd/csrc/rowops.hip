@@ -95,11 +95,12 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(const float* __restr
   }
   float mean, sd;
   ln_stats<VPL>(v, lane, C, eps, mean, sd);
+  const Divisor by_sd(sd);
   float* yr = y + row * ldy;
 #pragma unroll
   for (int i = 0; i < VPL; ++i) {
     const int j = lane + 64 * i;
-    if (j < C) yr[j] = ln_apply(v[i], sd, gamma[j], beta[j]);
+    if (j < C) yr[j] = ln_apply(v[i], by_sd, gamma[j], beta[j]);
   }
   if (lane == 0) {
     mean_out[row] = mean;
@@ -121,7 +122,8 @@ __global__ __launch_bounds__(256) void layernorm_bwd_kernel(const float* __restr
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   if (row >= rows) return;
-  const float mean = mean_in[row], sd = std_in[row];
+  const float mean = mean_in[row];
+  const Divisor by_sd(std_in[row]);
   const float* xr = x + row * ldx;
   const float* gr = dy + row * lddy;
   float xh[VPL], gg[VPL];
@@ -130,7 +132,7 @@ __global__ __launch_bounds__(256) void layernorm_bwd_kernel(const float* __restr
   for (int i = 0; i < VPL; ++i) {
     const int j = lane + 64 * i;
     if (j < C) {
-      xh[i] = (xr[j] - mean) / sd;
+      xh[i] = by_sd.under(xr[j] - mean);
       gg[i] = gr[j] * gamma[j];
     } else {
       xh[i] = 0.f;
@@ -147,7 +149,7 @@ __global__ __launch_bounds__(256) void layernorm_bwd_kernel(const float* __restr
   for (int i = 0; i < VPL; ++i) {
     const int j = lane + 64 * i;
     if (j < C) {
-      float v = (gg[i] - s1 - xh[i] * s2) / sd;
+      float v = by_sd.under(gg[i] - s1 - xh[i] * s2);
       if (ar) v += ar[j];
       dr[j] = v;
     }
@@ -197,7 +199,8 @@ __global__ __launch_bounds__(64 * LNP_WAVES) void layernorm_bwd_param_kernel(
   int64_t r = r0 + w;
   if constexpr (PF) load_row(r, cx, cg, cd);
   for (; r < r1; r += LNP_WAVES) {
-    const float mean = mean_in[r], sd = std_in[r];
+    const float mean = mean_in[r];
+    const Divisor by_sd(std_in[r]);
     const int64_t rn = r + LNP_WAVES;
     float nx[PF ? VPL : 1], ng[PF ? VPL : 1], nd[PF ? VPL : 1];
     if constexpr (PF) load_row(rn, nx, ng, nd);
@@ -207,7 +210,7 @@ __global__ __launch_bounds__(64 * LNP_WAVES) void layernorm_bwd_param_kernel(
 #pragma unroll
     for (int i = 0; i < VPL; ++i) {
       const int j = lane + 64 * i;
-      const float xh = j < C ? (cx[i] - mean) / sd : 0.f;
+      const float xh = j < C ? by_sd.under(cx[i] - mean) : 0.f;
       const float g = cg[i] * (PF ? gm[i] : (j < C ? gamma[j] : 0.f));
       s1 += g;
       s2 += g * xh;
@@ -224,7 +227,7 @@ __global__ __launch_bounds__(64 * LNP_WAVES) void layernorm_bwd_param_kernel(
       for (int i = 0; i < VPL; ++i) {
         const int j = lane + 64 * i;
         if (j < C) {
-          float v = (cg[i] - s1 - cx[i] * s2) / sd;
+          float v = by_sd.under(cg[i] - s1 - cx[i] * s2);
           if (rd_dx) v += PF ? cd[i] : add[r * ldadd + j];
           dr[j] = v;
         }

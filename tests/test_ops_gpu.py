@@ -566,6 +566,27 @@ def test_gemm_gelu_epilogues(dev, gemm_mode, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,C", [(1, 1), (5, 63), (300, 384), (67, 769), (33, 2048)])
+def test_layernorm_division_bits(dev, rows, C):
+    """LayerNorm divides many values by one deviation through its reciprocal
+    and a residual step: the same bits as a division, over rows of 2^-20 to
+    2^20, and a row of zeros without eps (0 / 0)."""
+    from minitorch_amd import kernels as K_
+
+    _say(f"[layernorm division] {rows} x {C}")
+    rng = np.random.default_rng(rows * C)
+    x = rng.standard_normal((rows, C), dtype=np.float32)
+    x *= (2.0 ** rng.integers(-20, 21, (rows, 1))).astype(np.float32)
+    x[rows // 2] = 0
+    one, zero = np.ones(C, np.float32), np.zeros(C, np.float32)
+    y, mean, std = empty((rows, C)), empty((rows,)), empty((rows,))
+    K_.layernorm_fwd(_T(x), _T(one), _T(zero), y, mean, std, 0.0)
+    with np.errstate(invalid="ignore", divide="ignore"):
+        want = (x - mean.numpy().reshape(-1, 1)) / std.numpy().reshape(-1, 1)
+    np.testing.assert_array_equal(y.numpy(), want)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K", [(70, 65, 40), (2048, 2048, 256), (128, 512, 8192)])
 def test_gemm_gelu_far_values(dev, M, N, K):
     """The GELU epilogues far from zero, in the fp32 kernel, the split kernel
