@@ -365,6 +365,45 @@ __global__ __launch_bounds__(256) void xent_fwd_kernel(const float* __restrict__
   }
 }
 
+// The same for long rows: a workgroup per row, which it reads once, VPT values
+// a thread.  A wave per row reads every row twice, the second time past L2 (a
+// CU's 32 rows of 5003 values are 640 KB): 8192 x 5003 84 -> 34 us, HBM bound
+// (164 MB, 4.8 TB/s).  (A launch has fewer than 2^32 threads.)
+template <int VPT>
+__global__ __launch_bounds__(256) void xent_fwd_row_kernel(const float* __restrict__ x, int64_t ldx,
+                                                           const int64_t* __restrict__ labels,
+                                                           float* __restrict__ row_loss,
+                                                           float* __restrict__ lse_out, int V) {
+  __shared__ float part[2][4];
+  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x, w = tid >> 6;
+  const float* xr = x + row * ldx;
+  float v[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) v[i] = tid + 256 * i < V ? xr[tid + 256 * i] : -INFINITY;
+  int64_t y = labels[row];
+  y = y < 0 ? 0 : (y >= V ? V - 1 : y);  // labels are validated on the host
+  const float xy = xr[y];
+  float mx = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) mx = fmaxf(mx, v[i]);
+  mx = wave_max(mx);
+  if ((tid & 63) == 0) part[0][w] = mx;
+  __syncthreads();
+  mx = fmaxf(fmaxf(part[0][0], part[0][1]), fmaxf(part[0][2], part[0][3]));
+  float s = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) s += tid + 256 * i < V ? expf(v[i] - mx) : 0.f;
+  s = wave_sum(s);
+  if ((tid & 63) == 0) part[1][w] = s;
+  __syncthreads();
+  if (tid == 0) {
+    const float lse = mx + logf((part[1][0] + part[1][1]) + (part[1][2] + part[1][3]));
+    row_loss[row] = lse - xy;
+    lse_out[row] = lse;
+  }
+}
+
 // dx[i,j] = g * (exp(x[i,j] - lse_i) - [j == y_i]) * scale, g read from device
 __global__ __launch_bounds__(256) void xent_bwd_kernel(const float* __restrict__ x, int64_t ldx,
                                                        const int64_t* __restrict__ labels,
@@ -387,6 +426,10 @@ __global__ __launch_bounds__(256) void xent_bwd_kernel(const float* __restrict__
   }
 }
 
+// Long rows by workgroup from here on (wave and workgroup, us: 512 x 65536 rows
+// 53 and 57, 700 x 47934 52 and 44, 1024 x 32768 50 and 33, 5003 x 6706 59 and
+// 26, 8192 x 4096 77 and 24; 2048 rows: 5.1 and 4.5 at 512, 54 and 10 at 5003).
+constexpr int XENT_MIN = 700;
 int rows_grid(int64_t rows) { return (int)((rows + 3) / 4); }
 
 template <template <int> class K>
@@ -533,7 +576,19 @@ extern "C" int mtx_xent_fwd_f32(const float* logits, int64_t ld, const int64_t* 
   MTX_CHECK_ARG(logits && labels && row_loss && lse, "xent: null pointer");
   MTX_CHECK_SHAPE(rows >= 0 && V >= 1 && ld >= V, "xent: bad shape");
   if (rows == 0) return MTX_OK;
-  hipLaunchKernelGGL(xent_fwd_kernel, dim3(rows_grid(rows)), dim3(256), 0, static_cast<hipStream_t>(stream),
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (V >= XENT_MIN && V <= 256 * 32 && rows < (1 << 24)) {
+#define XENT_R(N) hipLaunchKernelGGL(xent_fwd_row_kernel<N>, dim3((unsigned)rows), dim3(256), 0, st, logits, ld, labels, row_loss, lse, V)
+    if (V <= 256 * 4) XENT_R(4);
+    else if (V <= 256 * 8) XENT_R(8);
+    else if (V <= 256 * 16) XENT_R(16);
+    else if (V <= 256 * 24) XENT_R(24);
+    else XENT_R(32);
+#undef XENT_R
+    MTX_LAUNCHED();
+    return MTX_OK;
+  }
+  hipLaunchKernelGGL(xent_fwd_kernel, dim3(rows_grid(rows)), dim3(256), 0, st,
                      logits, ld, labels, row_loss, lse, rows, V);
   MTX_LAUNCHED();
   return MTX_OK;

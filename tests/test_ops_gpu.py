@@ -306,6 +306,33 @@ def test_gelu(dev):
     close(H(dx), h.g, name="gelu_bwd")
 
 
+@pytest.mark.parametrize("V,pad", [(699, 0), (700, 1), (1024, 3), (1025, 0), (2048, 1), (2049, 0), (5003, 0), (6144, 2),
+                                   (6145, 0), (8192, 0), (8193, 1)])
+def test_cross_entropy_long_rows(dev, V, pad):
+    """Row losses and log-sum-exps at the edges of the workgroup-per-row
+    kernel's range, rows at any 4-byte address, with -inf and large logits,
+    the label first, last or anywhere."""
+    from minitorch_amd import kernels as Kn
+    from minitorch_amd.device import index_array
+
+    _say(f"[xent rows] V={V} ld={V + pad}")
+    rng = np.random.default_rng(V)
+    rows = 37
+    x = (5 * rng.standard_normal((rows, V + pad))).astype(np.float32)
+    x[1, : V - 1] = -np.inf
+    x[2] += 3000
+    labels = rng.integers(0, V, rows)
+    labels[0], labels[1] = 0, V - 1
+    loss, lse = empty((rows,)), empty((rows,))
+    Kn.xent_fwd(T(x)[:, :V], index_array(labels).t, loss, lse)
+    xd = x[:, :V].astype(np.float64)
+    ref = np.logaddexp.reduce(xd, axis=1)
+    # exp and log to 2 ulp, 32 sums in a thread and 8 across them; lse and the loss rounded at their size
+    tol = 2.0 ** -24 * (48 + 2 * np.abs(ref))
+    assert np.all(np.abs(H(lse) - ref) <= tol)
+    assert np.all(np.abs(H(loss) - (ref - xd[np.arange(rows), labels])) <= 2 * tol)
+
+
 def test_cross_entropy_and_embedding(dev):
     import minitorch_amd as mt
     from oracle.gpt import cross_entropy, cross_entropy_bwd
