@@ -731,7 +731,7 @@ def main():
     ms_c2, losses_c2 = bench_gpt(C2_CFG, 2, 20, 3, graph=True)
     ms_c2_eager, _ = bench_gpt(C2_CFG, 2, 5, 2)
     # the same replayed step with the products of >= 128 x 128 on the fp32
-    # MFMA kernel instead of the default split kernel
+    # MFMA kernel instead of the default three-piece bf16 split
     from minitorch_amd import kernels as _K
 
     prev_mode = _K.set_gemm_mode(_K.GEMM_FP32)
@@ -829,7 +829,7 @@ def main():
                        "config": "vocab 65, n_embd 384, 6 heads, 6 layers, T=256, B=64, fp32, Adam 3e-4",
                        "losses": [round(x, 5) for x in losses_c2],
                        "mode": "step replayed from a HIP graph (CapturedStep)",
-                       "gemm": "fp32 products of >= 128 x 128 as two-piece fp16 splits on the 16-bit "
+                       "gemm": "fp32 products of >= 128 x 128 as three-piece bf16 splits on the bf16 "
                                "matrix cores (fp32-accurate; mtx_gemm_set_mode MTX_GEMM_BF16X3, the default)",
                        "ms_per_step_eager": round(ms_c2_eager, 3),
                        "fp32_mfma_gemm": {"ms_per_step": round(ms_c2_f32, 3),

@@ -82,7 +82,7 @@ int mtx_attn_fwd(int dtype, int B, int H, int Tq, int Tk, int D,
  * process-wide, read at launch or graph recording: MTX_GEMM_BF16X3 (the
  * default) on the bf16 matrix cores with every fp32 operand value, P and dS
  * split into three bf16 pieces and the six piece products of weight >= 2^-16
- * accumulated in fp32; MTX_GEMM_FP32 on
+ * accumulated in fp32 (as the GEMMs' mode of the same name); MTX_GEMM_FP32 on
  * fp32 MFMA.  Other head sizes and bf16 attention are not affected.  No reference
  * counterpart (the reference computes in NumPy float64 after the scale).
  */
@@ -501,13 +501,9 @@ int mtx_decode_step_reset(void* workspace, void* stream);
  * Products with M >= 128, N >= 128 and M*N*K*batch >= 2^27 run, by default
  * (MTX_GEMM_BF16X3), on the bf16 matrix cores -- unless they have fewer than
  * 64 tiles of 128 x 128 and K < 1024; those, like smaller products, take the
- * fp32 kernel -- with every fp32 operand value split into pieces and the
- * products of the pieces accumulated in fp32: for K >= 256 two fp16 pieces of
- * the value scaled by a power of two per row of A and column of B (x to 2^-23
- * |x|, or 2^-35 of its row's largest sampled value where that is more; three
- * products), and, for shorter products and every tile with a value more than
- * 2^17 times its row's largest sample, three bf16 pieces (x to 2^-24 |x|; six
- * products of weight >= 2^-16).  A dot product's error is the fp32
+ * fp32 kernel -- with every fp32 operand value split into three bf16
+ * pieces (x = x0 + x1 + x2 to 2^-24 |x|) and the six piece products of
+ * weight >= 2^-16 accumulated in fp32: a dot product's error is the fp32
  * accumulation error plus at most ~2^-22 sum|a_k b_k|.  Non-finite inputs,
  * and finite ones of magnitude above bf16's largest value (~3.39e38, whose
  * high piece rounds to Inf), give NaN where fp32 arithmetic could give a

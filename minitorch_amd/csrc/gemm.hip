@@ -81,8 +81,8 @@ struct GemmArgs {
   // skinny kernel: write the partial product to ws even when K is not split
   // (the split-K entry points of one range, K <= 16)
   int to_ws;
-  // tiled split kernel (set by the host): the two-piece form may be tried; C's
-  // (or the partials') and aux's rows have unit stride and do not overlap
+  // tiled split kernel (set by the host): its pipeline with unchecked loads;
+  // C's (or the partials') and aux's rows have unit stride and do not overlap
   int fast, rows_vec;
 };
 
@@ -402,35 +402,50 @@ __global__ __launch_bounds__(kGT) void gemm_f32_kernel(const GemmArgs g) {
 }
 
 // ---------------------------------------------------------------------------
-// fp32 products on the bf16 matrix cores (the default for tiles of 128 x 128).
+// fp32 products on the bf16 matrix cores (the default from 128 x 128 on).
 //
 // Every fp32 operand value x is split into three bf16 pieces while its tile
 // is staged into LDS: x0 = bf16(x), x1 = bf16(x - x0), x2 = bf16(x - x0 - x1)
 // (each conversion rounds to nearest even; each difference is exact in fp32),
 // so x = x0 + x1 + x2 + r with |r| <= 2^-24 |x|: the pieces carry x's 24-bit
-// significand.  A product x*y is accumulated as the six piece products of
-// weight >= 2^-16 (x2y0, x1y1, x0y2, x1y0, x0y1, x0y0, smallest first); the
-// three dropped ones (x1y2, x2y1, x2y2) weigh at most ~2^-23 |xy| together.
-// Each piece product is exact in fp32 and the matrix core adds it into the
-// fp32 accumulator, so a dot product's error is the fp32 accumulation error
-// (as with fp32 multiply-adds) plus at most ~2^-22 sum|x_k y_k|.  Six
+// significand, over fp32's whole range and whatever the other values of its
+// row are.  A product x*y is accumulated as the six piece products of weight
+// >= 2^-16; the three dropped ones (x1y2, x2y1, x2y2) weigh at most ~2^-23
+// |xy| together.  Each piece product is exact in fp32.  x0y0 has an
+// accumulator of its own and the five small ones share another, added at the
+// end: the large sum is rounded once per k step instead of six times.  A dot
+// product's error is then the fp32 accumulation error (as with fp32
+// multiply-adds) plus at most ~2^-22 sum|x_k y_k|.  Six
 // v_mfma_f32_32x32x16_bf16 (6 x 32 cycles) do the work of sixteen
 // v_mfma_f32_16x16x4_f32 (16 x 32 cycles): 2.7x the fp32 matrix rate.
 // Non-finite inputs give NaN (x - x0 is Inf - Inf).
 //
-// Two fp16 pieces do the same in three products where the values' range
-// allows (h2 below), and this form stays as what those tiles fall back to and
-// for short products.
+// (Two fp16 pieces of scaled values need three products and took 0.65-0.85 of
+// the time, but hold a value only relative to its row's largest: one large
+// feature that meets a small or zero weight costs the others their bits.)
 //
-// An operand contiguous along k is staged as [piece][row][k] (rows of 16
-// bf16, the two 16-byte chunks swapped on rows 8..15 mod 16) and read with
-// ds_read_b128; an operand contiguous along its rows (m or n) as
-// [piece][k][row] (rows of R + pad bf16, a stride of 16 or 48 banks mod 64)
-// and read with gfx950's transposing ds_read_b64_tr_b16, so staging never
-// transposes in registers.  Both layouts are free of LDS bank conflicts.
-// MFMA 32x32x16 operands: lane l holds row l%32 and k = 8(l/32) + 0..7;
-// accumulator element e of lane l is C[8(e/4) + 4(l/32) + e%4][l%32].
+// Tiling: 256 threads = 4 waves; a wave owns MI x NI MFMA tiles of 32 x 32
+// and the waves form a WM x WN grid, so the block tile is 32 MI WM x 32 NI
+// WN, and 16 deep.  Pipeline: two LDS buffers and one barrier per k step.
+// While the products of step t run out of one buffer, the wave splits the
+// values of step t + 1 (in registers since the step before) into the other
+// buffer and requests those of step t + 2 into the registers as they come
+// free: each MFMA occupies the matrix pipe for 32 cycles and the issue port
+// for 4, and the split's vector instructions are placed into the gaps
+// (sched_group_barrier).
+//
+// Two workgroups fit a CU, and a launch has no more than fill the chip: each
+// takes its tiles one after another, and the pipeline runs on across them
+// (the last two steps of a tile request and stage the next one's first two).
+// Against a workgroup a tile, staged in one LDS buffer behind two barriers (us
+// before and after): 4096^3 831 -> 743; 16384 x 1536 x 384 + GELU 158 -> 138, its
+// dX 141 -> 126, its weight gradient 143 -> 125; 8192 x 5003 x 384 308 -> 214; 16384 x
+// 384 x 128 26.5 -> 18.8.  Now the products' power bounds it: at 4096^3 the matrix
+// pipe is busy 0.62 of the time at 1.7 of the card's 2.4 GHz (1100 TF of bf16).
 // ---------------------------------------------------------------------------
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
 namespace x3 {
 constexpr int BK = 16;  // k-tile depth (one MFMA k step)
 // k-contiguous rows hold two 16-byte chunks, swapped on rows 8..15 mod 16:
@@ -439,93 +454,90 @@ constexpr int BK = 16;  // k-tile depth (one MFMA k step)
 __device__ __forceinline__ int kswz(int row) { return ((row >> 3) & 1) * 8; }
 }  // namespace x3
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-
-// One operand's R x 16 tile (rows = m for A, n for B).  KC: contiguous along
-// k in global memory (rows strided by srow); else contiguous along the rows
-// (k strided by sk).  The tile is R*4 float4 vectors; slot i of a thread is
-// vector idx = tid + 256 i: KC: row idx/4, k 4(idx%4)..+3; else: k idx/(R/4),
-// rows 4(idx%(R/4))..+3.  Where 256 does not divide R*4 the threads past the
-// end repeat the vector 128 before (the same values to the same place).
+// One operand's R x 16 tile (rows = m for A, n for B), R = 96 or 128.  KC:
+// contiguous along k in global memory (rows strided by srow); else contiguous
+// along the rows (k strided by sk).  The tile is R*4 float4 vectors; slot i
+// of a thread is vector idx = tid + 256 i: KC: row idx/4, k 4(idx%4)..+3;
+// else: k idx/(R/4), rows 4(idx%(R/4))..+3.  Where 256 does not divide R*4
+// the threads past the end repeat the vector 128 before (the same values to
+// the same place).
+// LDS planes, free of bank conflicts.  KC: [piece][row][16 k], read with
+// ds_read_b128; else [piece][k][row], k rows of R + pad bf16 (a stride of 16 or
+// 48 banks mod 64), read with gfx950's transposing ds_read_b64_tr_b16, so
+// staging never transposes in registers.
 template <bool KC, int R>
 struct X3Stage {
-  static constexpr int NV = (R * 4 + kGT - 1) / kGT;  // float4 per thread
+  static_assert(R == 96 || R == 128, "tile rows");
   static constexpr int NVEC = R * 4;
-  static_assert(NVEC % kGT == 0 || NVEC % kGT == 128, "tile rows");
-  // k-plane row stride (bf16): 16 or 48 banks mod 64
-  static constexpr int LDR = (R / 2) % 64 == 16 || (R / 2) % 64 == 48 ? R : R + 32;
+  static constexpr int NV = (NVEC + kGT - 1) / kGT;  // float4 per thread
+  static constexpr int LDR = R == 96 ? R : R + 32;   // k-plane row stride (bf16)
   static_assert((LDR / 2) % 64 == 16 || (LDR / 2) % 64 == 48, "bank stride");
   static constexpr int PS = KC ? R * x3::BK : x3::BK * LDR;  // plane size (bf16)
-  const float* __restrict__ base;  // the operand at (row r0, k 0)
-  int64_t srow, sk;
-  int rows, r0;
-  int lput[NV];  // LDS offsets (bf16) of this thread's vectors
+  int64_t srow, sk;   // element strides; one of them is 1
+  uint32_t voff[NV];  // this thread's byte offsets in a k-tile
+  int lput[NV];       // and where its vectors go in LDS (bf16)
+  // a tile's place: the operand at (its first row, its range's first k), and
+  // the bytes from there to the operand's end; uniform
+  struct Src {
+    const char* base;
+    int64_t left;
+  };
 
-  __device__ __forceinline__ int vec(int i, int tid) const {
+  __device__ __forceinline__ static int vec(int i, int tid) {
     const int idx = tid + i * kGT;
     return idx < NVEC ? idx : idx - 128;
   }
-  __device__ __forceinline__ void init(const float* b, int64_t s_row, int64_t s_k, int nrows, int row0, int tid) {
+  __device__ __forceinline__ void init(int64_t s_row, int64_t s_k, int tid) {
     srow = s_row;
     sk = s_k;
-    rows = nrows;
-    r0 = row0;
-    base = b + (int64_t)r0 * srow;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int idx = vec(i, tid);
       if constexpr (KC) {
+        voff[i] = (uint32_t)(idx / 4) * (uint32_t)(srow * 4) + 16 * (idx % 4);
         lput[i] = (idx / 4) * x3::BK + ((4 * (idx % 4)) ^ x3::kswz(idx / 4));
       } else {
+        voff[i] = (uint32_t)(idx / (R / 4)) * (uint32_t)(sk * 4) + 16 * (idx % (R / 4));
         lput[i] = (idx / (R / 4)) * LDR + 4 * (idx % (R / 4));
       }
     }
   }
-  // rows past `rows` and k past kend read as zero; unaligned vectors by element
-  __device__ __forceinline__ void fetch_checked(f32x4 (&r)[NV], int k0, int kend, int tid) const {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = vec(i, tid);
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
-      if constexpr (KC) {
-        const int row = idx / 4, k = k0 + 4 * (idx % 4);
-        if (r0 + row < rows) {
-          const float* p = base + (int64_t)row * srow + k;
-          if (k + 3 < kend && (((uintptr_t)p) & 15u) == 0) {
-            v = *reinterpret_cast<const f32x4*>(p);
-          } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              if (k + j < kend) v[j] = p[j];
-          }
-        }
-      } else {
-        const int k = k0 + idx / (R / 4), row = 4 * (idx % (R / 4));
-        if (k < kend) {
-          const float* p = base + (int64_t)k * sk + row;
-          if (r0 + row + 3 < rows && (((uintptr_t)p) & 15u) == 0) {
-            v = *reinterpret_cast<const f32x4*>(p);
-          } else {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              if (r0 + row + j < rows) v[j] = p[j];
-          }
-        }
-      }
-      r[i] = v;
-    }
+  __device__ __forceinline__ Src at(const float* b, int rows, int K, int r0, int k0) const {
+    return {reinterpret_cast<const char*>(b + (int64_t)r0 * srow + (int64_t)k0 * sk),
+            ((int64_t)(rows - 1 - r0) * srow + (int64_t)(K - 1 - k0) * sk + 1) * 4};
   }
-  __device__ __forceinline__ void put(__bf16* __restrict__ lds, const f32x4 (&r)[NV]) const {
+  // The k-tile k values from s on, through a buffer resource based at its
+  // first value and ending at the operand's last: no per-lane address
+  // arithmetic, and what lies past the operand's end reads as zeros.  (A vector reaching past a row's last value takes what
+  // follows it in memory, which the caller allows for rows only: their
+  // products land in rows or columns of C that are not stored.)
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile(const Src& s, int k) const {
+    const int64_t off = (int64_t)k * sk * 4, left = s.left - off;
+    const int hi = (int)(left >> 32);
+    const uint32_t bytes = hi < 0 ? 0u : hi > 0 ? 0xfffffff0u : (uint32_t)left;
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(s.base + off), (short)0, (int)bytes, 0x00020000);
+  }
+  __device__ __forceinline__ f32x4 fetch(__amdgpu_buffer_rsrc_t rs, int i) const {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)voff[i], 0, 0));
+  }
+  // the same by element, where a vector may reach past the last row or k, or
+  // offsets past 32 bits: rows from nrows and k from n on read as zeros
+  __device__ __forceinline__ f32x4 fetch_checked(const Src& s, int k0, int n, int nrows, int i, int tid) const {
+    const int idx = vec(i, tid);
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    const int row = KC ? idx / 4 : 4 * (idx % (R / 4)), k = k0 + (KC ? 4 * (idx % 4) : idx / (R / 4));
+    const float* p = reinterpret_cast<const float*>(s.base) + (KC ? row * srow + k : k * sk + row);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      uint2 h, m, l;
-      split3(r[i], h, m, l);
-      *reinterpret_cast<uint2*>(lds + lput[i]) = h;
-      *reinterpret_cast<uint2*>(lds + PS + lput[i]) = m;
-      *reinterpret_cast<uint2*>(lds + 2 * PS + lput[i]) = l;
-    }
+    for (int j = 0; j < 4; ++j)
+      if (row + (KC ? 0 : j) < nrows && k + (KC ? j : 0) < n) v[j] = p[j];
+    return v;
+  }
+  __device__ __forceinline__ void put(__bf16* __restrict__ lds, f32x4 r, int i) const {
+    uint2 h, m, l;
+    split3(r, h, m, l);
+    *reinterpret_cast<uint2*>(lds + lput[i]) = h;
+    *reinterpret_cast<uint2*>(lds + PS + lput[i]) = m;
+    *reinterpret_cast<uint2*>(lds + 2 * PS + lput[i]) = l;
   }
   // piece p's MFMA operand for tile rows rb .. rb+31: lane l gets row
   // rb + l%32 and k = 8(l/32) + 0..7
@@ -545,273 +557,6 @@ struct X3Stage {
       return __builtin_bit_cast(bf16x8, make_uint4(ul.x, ul.y, uh.x, uh.y));
     }
   }
-  // ACT 3 column sums: this thread's share of the staged B values, by
-  // column (KC: the 4 k of slot i belong to column idx/4; else slot i holds
-  // columns 4(idx%(R/4))..+3, the same for every slot; R = 128)
-  __device__ __forceinline__ static void colsum_add(float (&cs)[4], const f32x4 (&r)[NV]) {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      if constexpr (KC) {
-        cs[i] += (r[i][0] + r[i][1]) + (r[i][2] + r[i][3]);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) cs[j] += r[i][j];
-      }
-    }
-  }
-};
-
-// ---------------------------------------------------------------------------
-// fp32 products from two fp16 pieces of every value, three products each.
-//
-// A row of A (a column of B) is scaled by a power of two s, then every value
-// x is split while its tile is staged into LDS: h = fp16(s x) and
-// l = fp16(2^14 (s x - h)), both rounded to nearest, so that s x = h +
-// 2^-14 l with an error of at most 2^-23 |s x|, or 2^-39 where that is more.
-// C is (sum ah bh + 2^-14 sum (al bh + ah bl)) / (sa sb): the cross terms
-// have accumulators of their own, and the dropped al bl weighs at most
-// 2^-24 |ab|.  Three v_mfma_f32_32x32x16_f16 do the work of the three-piece
-// split's six bf16 ones, and the main accumulator is rounded once per k step
-// instead of six times, which is most of a long product's error: against
-// float64 the products of the 384-wide model's training step are off by
-// 0.5-0.6 of what the three-piece form gave (K = 384: 6.2e-8 against 1.1e-7
-// relative; K = 1536: 2.6e-7 against 6.0e-7).
-//
-// The scale comes from 32 of the row's values, spread evenly over its k range
-// (the beginning alone says too little: in the gradient of a packed q/k/v
-// projection a first token's row starts with the query's, which is 0 up to
-// rounding).  Their largest goes to [2^-4, 2^-3), so the error above is 2^-35
-// of it for small values, and other values may be 2^17 times larger before l
-// overflows (65504).  A row without a nonzero sample gets the largest scale,
-// which any value above 2^-99 overflows; a largest sample outside 2^-60 ..
-// 2^60 or not finite gives a scale of Inf.  An overflow leaves Inf or NaN in
-// the accumulators of its whole row or column, so one look at them after the
-// k loop finds it, and the workgroup then computes its tile again from three
-// bf16 pieces (X3Stage), whose range is fp32's.
-//
-// Tiling: 256 threads = 4 waves; a wave owns MI x NI MFMA tiles of 32 x 32
-// and the waves form a WM x WN grid, so the block tile is 32 MI WM x 32 NI
-// WN, and 32 deep.  Pipeline: two LDS buffers and one barrier per k step.
-// While the products of step t run out of one buffer, the wave splits the
-// values of step t + 1 (in registers since the step before) into the other
-// buffer and requests those of step t + 2 into the registers as they come
-// free: each MFMA occupies the matrix pipe for 32 cycles and the issue port
-// for 4, and the split's vector instructions are placed into the gaps
-// (sched_group_barrier).
-//
-// Two workgroups fit a CU, and a launch has no more than fill the chip: each
-// takes its tiles one after another, and the pipeline runs on across them
-// (the last two steps of a tile request and stage the next one's first two,
-// scaled by samples that were read during the epilogue before).  With a
-// workgroup per tile every tile began with three exposed round trips to
-// memory (samples, first and second step), all 512 resident ones at the same
-// time: 16384 x 1536 products took 57-64 us plus 4.1-4.6 us per 32 of K.
-// ---------------------------------------------------------------------------
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-namespace h2 {
-constexpr int BK = 32;  // k-tile depth: a row's 32 floats are one 128-byte line
-// From K = 256 on the error is no larger than the three-piece form's (of a
-// shorter product the split's own 6e-8 is most)
-constexpr int MINK = 256;
-
-// the scale times 2^14 of a row whose largest |sample| has these bits, and the reciprocal of the scale itself
-__device__ __forceinline__ float scale2(uint32_t amax) {
-  const int e = (int)(amax >> 23);
-  if (amax == 0) return __uint_as_float(254u << 23);
-  if (e < 127 - 60 || e > 127 + 60) return __uint_as_float(0x7f800000u);
-  return __uint_as_float((uint32_t)(127 + 127 + 14 - 4 - e) << 23);
-}
-__device__ __forceinline__ float unscale(uint32_t amax) {
-  const int e = (int)(amax >> 23);
-  if (amax == 0) return __uint_as_float(14u << 23);
-  return __uint_as_float((uint32_t)(e + 4) << 23);
-}
-// x2 = 2^14 s x of four values -> h and l, four fp16 each: two mixed-precision
-// multiply-adds a value (zero is a 0 that the compiler cannot see, and the
-// pairs are opaque to it: it would otherwise convert every h twice)
-__device__ __forceinline__ uint32_t pair_h(float x, float y, float zero) {
-  f16x2 h = {(_Float16)__builtin_fmaf(x, 0x1p-14f, zero), (_Float16)__builtin_fmaf(y, 0x1p-14f, zero)};
-  uint32_t u = __builtin_bit_cast(uint32_t, h);
-  asm("" : "+v"(u));
-  return u;
-}
-__device__ __forceinline__ uint32_t pair_l(uint32_t hu, float x, float y) {
-  const f16x2 h = __builtin_bit_cast(f16x2, hu);
-  f16x2 l = {(_Float16)__builtin_fmaf((float)h[0], -16384.f, x), (_Float16)__builtin_fmaf((float)h[1], -16384.f, y)};
-  return __builtin_bit_cast(uint32_t, l);
-}
-__device__ __forceinline__ void split(f32x4 x2, float zero, uint2& h, uint2& l) {
-  h.x = pair_h(x2[0], x2[1], zero);
-  h.y = pair_h(x2[2], x2[3], zero);
-  l.x = pair_l(h.x, x2[0], x2[1]);
-  l.y = pair_l(h.y, x2[2], x2[3]);
-}
-}  // namespace h2
-
-// One operand's R x 32 tile (rows = m for A, n for B), R = 64 (KC), 96 or
-// 128.  KC: contiguous along k in global memory (rows strided by srow); else
-// contiguous along the rows (k strided by sk).  Slot i of a thread is the
-// float4 vector idx = tid + 256 i: KC: row idx/8, k 4(idx%8)..+3; else: k
-// idx/(R/4), rows 4(idx%(R/4))..+3.
-// LDS planes.  KC: [row][32 k], rows of 64 bytes, the four 16-byte chunks
-// permuted by (row/4)%4, so the 16 rows of a fragment read's quarter cover
-// all 64 banks.  Else [k][R rows]: the transposing read takes 32 bytes of
-// four consecutive k rows per 16 lanes; R = 96 (48 banks a row) spreads them
-// by itself, R = 128 permutes the four 64-byte blocks of a row by k%4.
-template <bool KC, int R>
-struct H2Stage {
-  static_assert(R == 96 || R == 128 || (KC && R == 64), "tile rows");
-  static constexpr int NV = R * h2::BK / 4 / kGT;              // float4 per thread
-  static constexpr int NQ = 2;                                 // sample vectors per thread
-  static constexpr int PS = R * h2::BK;                        // plane size (fp16)
-  static constexpr int NSC = KC ? NV : R == 128 ? 4 : 4 * NV;  // scales a thread needs
-  static constexpr bool kEach = !KC && R == 96;                // slots do not lie a constant apart
-  int64_t kstep;      // bytes per k
-  uint32_t sstep;     // bytes per row (KC) or k (else)
-  uint32_t voff[NV];  // this thread's byte offsets in a k-tile
-  int lput[kEach ? NV : 1];
-  float sc[NSC];
-  // a tile's place: the operand at (its first row, its first k), and the
-  // bytes from there to the operand's end; uniform
-  struct Src {
-    const char* base;
-    int64_t left;
-  };
-
-  __device__ __forceinline__ void init(int64_t srow, int64_t sk, int tid) {
-    kstep = sk * 4;
-    sstep = (uint32_t)((KC ? srow : sk) * 4);
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = tid + i * kGT;
-      voff[i] = KC ? (uint32_t)(idx / 8) * sstep + 16 * (idx % 8)
-                   : (uint32_t)(idx / (R / 4)) * sstep + 16 * (idx % (R / 4));
-      if constexpr (kEach) lput[i] = idx * 4;
-    }
-    if constexpr (KC) {
-      const int row = tid / 8, c = (tid % 8) / 2;
-      lput[0] = row * h2::BK + 8 * (c ^ ((row >> 2) & 3)) + 4 * (tid & 1);
-    } else if constexpr (R == 128) {
-      const int k = tid / 32, c = 4 * (tid % 32);
-      lput[0] = k * R + (c ^ (32 * (k & 3)));
-    }
-  }
-  __device__ __forceinline__ Src at(const float* b, int64_t srow, int64_t sk, int rows, int K, int r0, int k0) const {
-    return {reinterpret_cast<const char*>(b + (int64_t)r0 * srow + (int64_t)k0 * sk),
-            ((int64_t)(rows - 1 - r0) * srow + (int64_t)(K - 1 - k0) * sk + 1) * 4};
-  }
-  __device__ __forceinline__ int put_at(int i) const {
-    if constexpr (KC) return lput[0] + i * 32 * h2::BK;       // 32 rows on: the same permutation
-    else if constexpr (R == 128) return lput[0] + i * 8 * R;  // 8 k on
-    else return lput[i];
-  }
-  // The k-tile k values from s on, through a buffer resource based at its
-  // first value and ending at the operand's last: no per-lane address
-  // arithmetic, and rows past the operand's end read as zeros.  (A vector
-  // reaching past a row's last value takes what follows it in memory, which
-  // the caller allows for rows only: their products land in rows or columns
-  // of C that are not stored.)
-  __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile(const Src& s, int k) const {
-    const int64_t off = (int64_t)k * kstep, left = s.left - off;
-    const int hi = (int)(left >> 32);
-    const uint32_t bytes = hi < 0 ? 0u : hi > 0 ? 0xfffffff0u : (uint32_t)left;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(s.base + off), (short)0, (int)bytes, 0x00020000);
-  }
-  __device__ __forceinline__ f32x4 fetch(__amdgpu_buffer_rsrc_t rs, int i) const {
-    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)voff[i], 0, 0));
-  }
-  // the same by element where a vector may reach past the last row or k
-  __device__ __forceinline__ f32x4 fetch_checked(const Src& s, int k0, int n, int nrows, int i, int tid) const {
-    const int idx = tid + i * kGT;
-    f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    const int row = KC ? idx / 8 : 4 * (idx % (R / 4)), k = k0 + (KC ? 4 * (idx % 8) : idx / (R / 4));
-    const float* p = reinterpret_cast<const float*>(s.base + (int64_t)(KC ? row : k) * sstep) + (KC ? k : row);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if (row + (KC ? 0 : j) < nrows && k + (KC ? j : 0) < n) v[j] = p[j];
-    return v;
-  }
-  // 16 values of each row, spread evenly over the tile's n k (n >= 256): KC:
-  // four vectors, at 0, 1/3, 2/3 and the end; else 16 k rows.  Thread vector
-  // i is idx = tid + 256 i (repeating those 128 before where that is past the
-  // tile's R*4): KC: row idx/4, place idx%4; else place idx/(R/4).
-  __device__ __forceinline__ static int qvec(int i, int tid) {
-    const int idx = tid + i * kGT;
-    return idx < R * 4 ? idx : idx - (R == 64 ? 256 : 128);
-  }
-  __device__ __forceinline__ void sample(f32x4 (&q)[NQ], const Src& s, int n, int tid) const {
-    const __amdgpu_buffer_rsrc_t rs = tile(s, 0);
-    const uint32_t far = KC ? (uint32_t)((n - 4) / 3) * 4u : (uint32_t)((n - 1) / 15) * sstep;
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      const int idx = qvec(i, tid);
-      const uint32_t off = KC ? (uint32_t)(idx / 4) * sstep + (uint32_t)(idx % 4) * far
-                              : (uint32_t)(idx / (R / 4)) * far + 16 * (idx % (R / 4));
-      q[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)off, 0, 0));
-    }
-  }
-  // amax[row] = the largest of each row's samples (as bits); it is zero before
-  __device__ __forceinline__ static void row_max(const f32x4 (&q)[NQ], uint32_t* amax, int tid) {
-#pragma unroll
-    for (int i = 0; i < NQ; ++i) {
-      const int idx = qvec(i, tid);
-      if constexpr (KC) {
-        uint32_t m = 0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) m = max(m, __float_as_uint(q[i][j]) & 0x7fffffffu);
-        m = max(m, (uint32_t)__shfl_xor((int)m, 1));
-        m = max(m, (uint32_t)__shfl_xor((int)m, 2));
-        if ((tid & 3) == 0) amax[idx / 4] = m;
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          atomicMax(&amax[4 * (idx % (R / 4)) + j], __float_as_uint(q[i][j]) & 0x7fffffffu);
-      }
-    }
-  }
-  __device__ __forceinline__ void scales(const uint32_t* amax, int tid) {
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-      const int idx = tid + i * kGT;
-      if constexpr (KC) {
-        sc[i] = h2::scale2(amax[idx / 8]);
-      } else if (R != 128 || i == 0) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sc[4 * i + j] = h2::scale2(amax[4 * (idx % (R / 4)) + j]);
-      }
-    }
-  }
-  __device__ __forceinline__ void put(_Float16* __restrict__ lds, f32x4 r, float zero, int i) const {
-    f32x4 x2;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) x2[j] = r[j] * sc[KC ? i : R == 128 ? j : 4 * i + j];
-    uint2 h, l;
-    h2::split(x2, zero, h, l);
-    *reinterpret_cast<uint2*>(lds + put_at(i)) = h;
-    *reinterpret_cast<uint2*>(lds + PS + put_at(i)) = l;
-  }
-  // piece p's MFMA operand for k 16 sub .. +15 of tile rows rb .. rb+31: lane
-  // l gets row rb + l%32 and k = 16 sub + 8(l/32) + 0..7
-  __device__ __forceinline__ static f16x8 frag(const _Float16* __restrict__ lds, int p, int sub, int rb, int lane) {
-    if constexpr (KC) {
-      const int row = rb + (lane & 31);
-      return *reinterpret_cast<const f16x8*>(lds + p * PS + row * h2::BK +
-                                             8 * ((2 * sub + (lane >> 5)) ^ ((row >> 2) & 3)));
-    } else {
-      // transposing read, as X3Stage::frag
-      const int G = lane >> 4, j = lane & 15;
-      const int k = 16 * sub + 8 * (G >> 1) + (j >> 2);
-      int c = rb + 16 * (G & 1) + 4 * (j & 3);
-      if constexpr (R == 128) c ^= 32 * (k & 3);
-      const _Float16* p0 = lds + p * PS + k * R + c;
-      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p0);
-      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p0 + 4 * R));
-      const uint2 ul = __builtin_bit_cast(uint2, lo), uh = __builtin_bit_cast(uint2, hi);
-      return __builtin_bit_cast(f16x8, make_uint4(ul.x, ul.y, uh.x, uh.y));
-    }
-  }
 };
 
 // a thread or lane number whose uses are computed where they stand: code that
@@ -826,19 +571,11 @@ template <int MI, int NI, int WM, int WN, bool AK, bool BN1, int ACT>
 __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
   static_assert(WM * WN == 4, "four waves");
   constexpr int BM = 32 * MI * WM, BN = 32 * NI * WN;
-  using SA = H2Stage<AK, BM>;
-  using SB = H2Stage<!BN1, BN>;  // B^T: rows = n, contiguous along k iff !BN1
-  using XA = X3Stage<AK, BM>;
-  using XB = X3Stage<!BN1, BN>;
-  constexpr int kBuf = 2 * (SA::PS + SB::PS);  // one stage's planes (fp16)
-  constexpr int kX3 = 3 * (XA::PS + XB::PS) * 2;
-  constexpr int kTiles = 2 * kBuf * 2 > kX3 ? 2 * kBuf * 2 : kX3;
-  __shared__ __attribute__((aligned(16))) char smem[kTiles];
+  using SA = X3Stage<AK, BM>;
+  using SB = X3Stage<!BN1, BN>;  // B^T: rows = n, contiguous along k iff !BN1
+  constexpr int kBuf = 3 * (SA::PS + SB::PS);  // one stage's planes (bf16)
+  __shared__ __attribute__((aligned(16))) __bf16 smem[2 * kBuf];
   __shared__ float red[ACT == 3 ? 8 * BN : 1];  // column sums
-  // rows' and columns' largest sample of the tiles: one in its epilogue, one
-  // being staged, one being sampled, one being cleared
-  __shared__ __attribute__((aligned(16))) uint32_t amax[4][BM + BN];
-  __shared__ int again;
   const int tid = threadIdx.x;
   const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = (wid / WN) * 32 * MI, wn = (wid % WN) * 32 * NI;
@@ -876,80 +613,92 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
   SB sb;
   sa.init(g.sam, g.sak, tid);
   sb.init(g.sbn, g.sbk, tid);
-  auto src_a = [&](const Place& p) {
-    return sa.at(g.a + (int64_t)p.bidx * g.sab, g.sam, g.sak, g.M, g.K, p.m0, p.kbeg);
-  };
-  auto src_b = [&](const Place& p) {
-    return sb.at(g.b + (int64_t)p.bidx * g.sbb, g.sbn, g.sbk, g.N, g.K, p.n0, p.kbeg);
-  };
 
-  f32x16 acc[MI][NI], accx[MI][NI];
+  f32x16 acc[MI][NI], accx[MI][NI];  // x0y0, and the small piece products
   f32x4 ra[SA::NV], rb[SB::NV];
   // ACT 3: column sums of B from the values each thread stages
-  float cs[SB::NV][4];
-  float zero = 0.f;
-  asm("" : "+s"(zero));
+  float cs[BN1 ? 4 : SB::NV];
+#pragma unroll
+  for (int j = 0; j < (BN1 ? 4 : SB::NV); ++j) cs[j] = 0.f;
   int par = 0;  // the buffer that holds the step to multiply
-  auto buf = [&](int b) { return reinterpret_cast<_Float16*>(smem) + b * kBuf; };
+  auto buf = [&](int b) { return smem + b * kBuf; };
 
   auto colsum = [&] {
     if constexpr (ACT == 3) {
 #pragma unroll
       for (int i = 0; i < SB::NV; ++i) {
-        if constexpr (!BN1) cs[i][0] += (rb[i][0] + rb[i][1]) + (rb[i][2] + rb[i][3]);
+        if constexpr (!BN1) cs[i] += (rb[i][0] + rb[i][1]) + (rb[i][2] + rb[i][3]);
         else
 #pragma unroll
-          for (int j = 0; j < 4; ++j) cs[0][j] += rb[i][j];
+          for (int j = 0; j < 4; ++j) cs[j] += rb[i][j];
       }
     }
   };
-  // the products of one step, MFMA by MFMA: half a step (sub) at a time the
-  // four fragments' three products.  fa, fb: [sub][piece][tile].
+
+  auto src_a = [&](const Place& p) {
+    return sa.at(g.a + (int64_t)p.bidx * g.sab, g.M, g.K, p.m0, p.kbeg);
+  };
+  auto src_b = [&](const Place& p) {
+    return sb.at(g.b + (int64_t)p.bidx * g.sbb, g.N, g.K, p.n0, p.kbeg);
+  };
+  auto fetch_checked = [&](const Place& p, int k) {
+    const auto a = src_a(p);
+    const auto b = src_b(p);
+    const int tv = here(tid);
+#pragma unroll
+    for (int i = 0; i < SA::NV; ++i) ra[i] = sa.fetch_checked(a, k, p.n, g.M - p.m0, i, tv);
+#pragma unroll
+    for (int i = 0; i < SB::NV; ++i) rb[i] = sb.fetch_checked(b, k, p.n, g.N - p.n0, i, tv);
+  };
+  auto put_all = [&](__bf16* to) {
+#pragma unroll
+    for (int i = 0; i < SA::NV; ++i) sa.put(to, ra[i], i);
+#pragma unroll
+    for (int i = 0; i < SB::NV; ++i) sb.put(to + 3 * SA::PS, rb[i], i);
+  };
+
+  // the products of one step, MFMA by MFMA; pa, pb: [piece][tile]
   constexpr int kT = MI * NI, kM = 6 * kT;
-  f16x8 fa[2][2][MI], fb[2][2][NI];
-  auto read_frags = [&](const _Float16* cur, int sub, int p) {
+  bf16x8 pa[3][MI], pb[3][NI];
+  auto read_frags = [&](const __bf16* from) {
 #pragma unroll
-    for (int i = 0; i < MI; ++i) fa[sub][p][i] = SA::frag(cur, p, sub, wm + 32 * i, lane);
+    for (int p = 0; p < 3; ++p) {
 #pragma unroll
-    for (int j = 0; j < NI; ++j) fb[sub][p][j] = SB::frag(cur + 2 * SA::PS, p, sub, wn + 32 * j, lane);
+      for (int i = 0; i < MI; ++i) pa[p][i] = SA::frag(from, p, wm + 32 * i, lane);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) pb[p][j] = SB::frag(from + 3 * SA::PS, p, wn + 32 * j, lane);
+    }
   };
   auto product = [&](int q) {
-    const int sub = q / (3 * kT), kind = q / kT % 3, i = q % kT / NI, j = q % NI;
-    if (kind == 0) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][0][i], fb[sub][0][j], acc[i][j], 0, 0, 0);
-    else if (kind == 1)
-      accx[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][1][i], fb[sub][0][j], accx[i][j], 0, 0, 0);
-    else accx[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa[sub][0][i], fb[sub][1][j], accx[i][j], 0, 0, 0);
+    constexpr int kA[6] = {0, 1, 0, 1, 2, 0}, kB[6] = {0, 0, 1, 1, 0, 2};
+    const int kind = q / kT, i = q % kT / NI, j = q % NI;
+    f32x16& c = kind == 0 ? acc[i][j] : accx[i][j];
+    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pa[kA[kind]][i], pb[kB[kind]][j], c, 0, 0, 0);
   };
   // One step: its products in as many groups as there are vectors to stage
   // (kS); beside each group's products one vector of the next step is split
   // and stored, and its register refilled with the step after's (refill).
   constexpr int kS = SA::NV + SB::NV;
   auto step = [&](auto refill, __amdgpu_buffer_rsrc_t ta, __amdgpu_buffer_rsrc_t tb) {
-    const _Float16* cur = buf(par);
-    _Float16* nxt = buf(par ^ 1);
-    read_frags(cur, 0, 0);
-    read_frags(cur, 0, 1);
+    __bf16* nxt = buf(par ^ 1);
+    read_frags(buf(par));
     colsum();
 #pragma unroll
     for (int c = 0; c < kS; ++c) {
       __builtin_amdgcn_sched_barrier(0);
-      // the second half's fragments, as the first half's come free
-      if (c == kS / 2 - 2) read_frags(cur, 1, 0);
-      if (c == kS / 2 - 1) read_frags(cur, 1, 1);
 #pragma unroll
       for (int q = c * kM / kS; q < (c + 1) * kM / kS; ++q) product(q);
       if (c < SA::NV) {
-        sa.put(nxt, ra[c], zero, c);
+        sa.put(nxt, ra[c], c);
         if constexpr (decltype(refill)::value) ra[c] = sa.fetch(ta, c);
       } else {
-        sb.put(nxt + 2 * SA::PS, rb[c - SA::NV], zero, c - SA::NV);
+        sb.put(nxt + 3 * SA::PS, rb[c - SA::NV], c - SA::NV);
         if constexpr (decltype(refill)::value) rb[c - SA::NV] = sb.fetch(tb, c - SA::NV);
       }
 #pragma unroll
-      for (int q = 0; q < 3; ++q) {
+      for (int q = c * kM / kS; q < (c + 1) * kM / kS; ++q) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        if (c == kS / 2 - 2 || c == kS / 2 - 1) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
       }
     }
     par ^= 1;
@@ -957,30 +706,30 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
   };
 
   Place cur = place(tile);
-  bool primed = false;  // this tile's first step is staged, its second one in registers
-  if (tid == 0) again = 0;
-  for (int i = tid; i < 4 * (BM + BN); i += kGT) amax[0][i] = 0;
-  if (g.fast) {
-    f32x4 qa[2][SA::NQ], qb[2][SB::NQ];
-    const bool more = tile + wgs < tend;
-    const Place p1 = place(more ? tile + wgs : tile);
-    sa.sample(qa[0], src_a(cur), cur.n, tid);
-    sb.sample(qb[0], src_b(cur), cur.n, tid);
-    sa.sample(qa[1], src_a(p1), p1.n, tid);
-    sb.sample(qb[1], src_b(p1), p1.n, tid);
-    __syncthreads();
-    SA::row_max(qa[0], amax[0], tid);
-    SB::row_max(qb[0], amax[0] + BM, tid);
-    SA::row_max(qa[1], amax[1], tid);
-    SB::row_max(qb[1], amax[1] + BM, tid);
+  if (g.fast) {  // the first tile's first step into LDS, its second one on its way
+    const auto a0 = src_a(cur);
+    const auto b0 = src_b(cur);
+    auto ta = sa.tile(a0, 0);
+    auto tb = sb.tile(b0, 0);
+#pragma unroll
+    for (int i = 0; i < SA::NV; ++i) ra[i] = sa.fetch(ta, i);
+#pragma unroll
+    for (int i = 0; i < SB::NV; ++i) rb[i] = sb.fetch(tb, i);
+    colsum();
+    put_all(buf(0));
+    ta = sa.tile(a0, x3::BK);
+    tb = sb.tile(b0, x3::BK);
+#pragma unroll
+    for (int i = 0; i < SA::NV; ++i) ra[i] = sa.fetch(ta, i);
+#pragma unroll
+    for (int i = 0; i < SB::NV; ++i) rb[i] = sb.fetch(tb, i);
     __syncthreads();
   }
 
-  for (int seq = 0;; ++seq) {
+  for (;;) {
     const bool more = tile + wgs < tend;
     const Place next = place(more ? tile + wgs : tile);
-    bool scaled = false;  // acc, accx hold the two-piece sums
-    float cso[4] = {0.f, 0.f, 0.f, 0.f};
+    float cso[BN1 ? 4 : SB::NV];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -988,177 +737,74 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[i][j][e] = accx[i][j][e] = 0.f;
 
+    auto take_sums = [&] {
+#pragma unroll
+      for (int j = 0; j < (BN1 ? 4 : SB::NV); ++j) {
+        cso[j] = cs[j];
+        cs[j] = 0.f;
+      }
+    };
     if (g.fast) {
-      const typename SA::Src a0 = src_a(cur);
-      const typename SB::Src b0 = src_b(cur);
-      const int steps = (cur.n + h2::BK - 1) / h2::BK;
+      const auto a0 = src_a(cur);
+      const auto b0 = src_b(cur);
+      const int steps = (cur.n + x3::BK - 1) / x3::BK;
       // The k steps that the unchecked loads take: whole ones, and (where the
       // rows of an operand contiguous along them do not end on a vector) not
       // the operand's last, whose last vectors reach past its end.
-      int whole = cur.n / h2::BK;
+      int whole = cur.n / x3::BK;
       if (((!AK && (g.M & 3)) || (BN1 && (g.N & 3))) && cur.kbeg + cur.n == g.K && whole == steps) --whole;
-      for (int i = tid; i < BM + BN; i += kGT) amax[(seq + 2) & 3][i] = 0;
-      if (!primed) {
-        sa.scales(amax[seq & 3], tid);
-        sb.scales(amax[seq & 3] + BM, tid);
-        // (n >= 256: the first two steps are whole)
-        auto ta = sa.tile(a0, 0);
-        auto tb = sb.tile(b0, 0);
-#pragma unroll
-        for (int i = 0; i < SA::NV; ++i) ra[i] = sa.fetch(ta, i);
-#pragma unroll
-        for (int i = 0; i < SB::NV; ++i) rb[i] = sb.fetch(tb, i);
-        if constexpr (ACT == 3) {
-#pragma unroll
-          for (int i = 0; i < SB::NV; ++i)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) cs[i][j] = 0.f;
-        }
-        colsum();
-        ta = sa.tile(a0, h2::BK);
-        tb = sb.tile(b0, h2::BK);
-#pragma unroll
-        for (int i = 0; i < SA::NV; ++i) {
-          sa.put(buf(par), ra[i], zero, i);
-          ra[i] = sa.fetch(ta, i);
-        }
-#pragma unroll
-        for (int i = 0; i < SB::NV; ++i) {
-          sb.put(buf(par) + 2 * SA::PS, rb[i], zero, i);
-          rb[i] = sb.fetch(tb, i);
-        }
-        __syncthreads();
-      }
       int t = 0;
       for (; t + 2 < whole; ++t)
-        step(std::true_type{}, sa.tile(a0, (t + 2) * h2::BK), sb.tile(b0, (t + 2) * h2::BK));
+        step(std::true_type{}, sa.tile(a0, (t + 2) * x3::BK), sb.tile(b0, (t + 2) * x3::BK));
       if (t + 2 < steps) {  // at most one step that is not whole
         step(std::false_type{}, sa.tile(a0, 0), sb.tile(b0, 0));
         ++t;
-        const int tv = here(tid);
-#pragma unroll
-        for (int i = 0; i < SA::NV; ++i) ra[i] = sa.fetch_checked(a0, (t + 1) * h2::BK, cur.n, g.M - cur.m0, i, tv);
-#pragma unroll
-        for (int i = 0; i < SB::NV; ++i) rb[i] = sb.fetch_checked(b0, (t + 1) * h2::BK, cur.n, g.N - cur.n0, i, tv);
+        fetch_checked(cur, (t + 1) * x3::BK);
       }
       // the last two steps: request, then stage, the next tile's first two
-      typename SA::Src a1 = src_a(next);
-      typename SB::Src b1 = src_b(next);
+      auto a1 = src_a(next);
+      auto b1 = src_b(next);
       if (!more) a1.left = b1.left = 0;  // reads as zeros
       step(std::true_type{}, sa.tile(a1, 0), sb.tile(b1, 0));
-      if constexpr (ACT == 3) {  // from here on the sums are the next tile's
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          cso[j] = BN1 ? cs[0][j] : cs[j % SB::NV][0];
-          (BN1 ? cs[0][j] : cs[j % SB::NV][0]) = 0.f;
-        }
-      }
-      sa.scales(amax[(seq + 1) & 3], tid);
-      sb.scales(amax[(seq + 1) & 3] + BM, tid);
-      step(std::true_type{}, sa.tile(a1, more ? h2::BK : 0), sb.tile(b1, more ? h2::BK : 0));
-      primed = more;
-      // Inf or NaN in a row or column of the tile: every row of the wave's
-      // tile in its first column, every column in its first row
-      float z = 0.f;
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) z += 0.f * acc[i][0][e] + 0.f * accx[i][0][e];
-#pragma unroll
-      for (int j = 1; j < NI; ++j) z += 0.f * acc[0][j][0] + 0.f * accx[0][j][0];
-      if (!(z == 0.f)) again = seq + 1;  // any lane
-      __syncthreads();
-      scaled = again != seq + 1;
-    }
-
-    if (!scaled) {
-      primed = false;  // the buffers are used otherwise
-      const int tv = here(tid), lv = tv & 63;
-      XA xa;
-      XB xb;
-      xa.init(g.a + (int64_t)cur.bidx * g.sab, g.sam, g.sak, g.M, cur.m0, tv);
-      xb.init(g.b + (int64_t)cur.bidx * g.sbb, g.sbn, g.sbk, g.N, cur.n0, tv);
-      __bf16* As = reinterpret_cast<__bf16*>(smem);
-      __bf16* Bs = As + 3 * XA::PS;
-#pragma unroll
-      for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NI; ++j)
-#pragma unroll
-          for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-      const bool sums = ACT == 3 && !g.fast;  // else they are there already
-      const int kbeg = cur.kbeg, kend = cur.kbeg + cur.n;
-      f32x4 pa[XA::NV], pb[XB::NV];
-      xa.fetch_checked(pa, kbeg, kend, tv);
-      xb.fetch_checked(pb, kbeg, kend, tv);
-      for (int k0 = kbeg; k0 < kend; k0 += x3::BK) {
+      take_sums();  // from here on they are the next tile's
+      step(std::true_type{}, sa.tile(a1, more ? x3::BK : 0), sb.tile(b1, more ? x3::BK : 0));
+    } else {
+      fetch_checked(cur, 0);
+      for (int k = 0; k < cur.n; k += x3::BK) {
+        colsum();
         __syncthreads();
-        xa.put(As, pa);
-        xb.put(Bs, pb);
-        if constexpr (ACT == 3) {
-          if (sums) XB::colsum_add(cso, pb);
-        }
+        put_all(buf(0));
         __syncthreads();
-        if (k0 + x3::BK < kend) {
-          xa.fetch_checked(pa, k0 + x3::BK, kend, tv);
-          xb.fetch_checked(pb, k0 + x3::BK, kend, tv);
-        }
-        bf16x8 a[3][MI], b[3][NI];
+        if (k + x3::BK < cur.n) fetch_checked(cur, k + x3::BK);
+        read_frags(buf(0));
 #pragma unroll
-        for (int p = 0; p < 3; ++p) {
-#pragma unroll
-          for (int i = 0; i < MI; ++i) a[p][i] = XA::frag(As, p, wm + 32 * i, lv);
-#pragma unroll
-          for (int j = 0; j < NI; ++j) b[p][j] = XB::frag(Bs, p, wn + 32 * j, lv);
-        }
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NI; ++j) {
-            f32x16 c = acc[i][j];
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[2][i], b[0][j], c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[1][j], c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[2][j], c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[1][i], b[0][j], c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[1][j], c, 0, 0, 0);
-            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[0][i], b[0][j], c, 0, 0, 0);
-            acc[i][j] = c;
-          }
+        for (int q = 0; q < kM; ++q) product(q);
       }
-      __syncthreads();
-    }
-
-    // the samples of the tile after the next, on their way during the epilogue
-    const bool more2 = g.fast && tile + 2 * wgs < tend;
-    const int tq = here(tid);
-    f32x4 qa[SA::NQ], qb[SB::NQ];
-    if (more2) {
-      const Place p2 = place(tile + 2 * wgs);
-      sa.sample(qa, src_a(p2), p2.n, tq);
-      sb.sample(qb, src_b(p2), p2.n, tq);
+      take_sums();
     }
 
     if constexpr (ACT == 3) {
       // the first row of tiles reduces the per-thread column sums through
-      // LDS: KC: 8 (three pieces: 4) threads per column, else 8 threads per 4
-      // columns; contributors are added in a fixed order
+      // LDS: KC: 4 threads per column, else 8 threads per 4 columns;
+      // contributors are added in a fixed order
       static_assert(BN == 128, "column sums");
       if (cur.m0 == 0) {
+        if constexpr (BN1) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if constexpr (BN1) {
-            red[(tid / 32) * BN + 4 * (tid % 32) + i] = cso[i];
-          } else {
+          for (int j = 0; j < 4; ++j) red[(tid / 32) * BN + 4 * (tid % 32) + j] = cso[j];
+        } else {
+#pragma unroll
+          for (int i = 0; i < SB::NV; ++i) {
             const int idx = tid + i * kGT;
-            if (g.fast) red[(idx % 8) * BN + idx / 8] = cso[i];
-            else if (i < XB::NV) red[(idx % 4) * BN + idx / 4] = cso[i];
+            red[(idx % 4) * BN + idx / 4] = cso[i];
           }
         }
         __syncthreads();
         if (tid < BN) {
-          const int nc = BN1 || g.fast ? 8 : 4;
+          constexpr int NC = BN1 ? 8 : 4;
           float v = 0.f;
-          for (int c = 0; c < nc; ++c) v += red[c * BN + tid];
+#pragma unroll
+          for (int c = 0; c < NC; ++c) v += red[c * BN + tid];
           const int n = cur.n0 + tid;
           if (n < g.N) {
             if (g.ksplit > 1) g.ws[(int64_t)g.ksplit * g.M * g.N + (int64_t)cur.split * g.N + n] = v;
@@ -1179,27 +825,19 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
     const bool to_ws = g.ksplit > 1;
     const bool rd_c = !to_ws && g.beta != 0.f;
     const bool use_x = !to_ws && (ACT == 2 || ACT == 4 || (ACT == 1 && g.aux != nullptr));
-    const uint32_t* am = amax[seq & 3];
     const int n1 = cur.n0 + wn;  // the wave's first column
-    float unB[NI], bv[NI];       // of this lane's columns
+    float bv[NI];                // of this lane's columns
 #pragma unroll
-    for (int j = 0; j < NI; ++j) {
-      unB[j] = scaled ? h2::unscale(am[BM + wn + 32 * j + lr]) : 1.f;
-      bv[j] = !to_ws && g.bias && n1 + 32 * j + lr < g.N ? g.bias[n1 + 32 * j + lr] : 0.f;
-    }
+    for (int j = 0; j < NI; ++j) bv[j] = !to_ws && g.bias && n1 + 32 * j + lr < g.N ? g.bias[n1 + 32 * j + lr] : 0.f;
     // the product's values of row group (i, q): [u][j]
     auto values = [&](int i, int q, float (&v)[4][NI]) {
-      const uint4 a4 = *reinterpret_cast<const uint4*>(am + wm + 32 * i + 8 * q + 4 * lh);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float unA = h2::unscale(u == 0 ? a4.x : u == 1 ? a4.y : u == 2 ? a4.z : a4.w);
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
         for (int j = 0; j < NI; ++j) {
-          float x = acc[i][j][4 * q + u];
-          if (scaled) x = __builtin_fmaf(accx[i][j][4 * q + u], 0x1p-14f, x) * unA * unB[j];
+          const float x = acc[i][j][4 * q + u] + accx[i][j][4 * q + u];
           v[u][j] = to_ws ? x : g.alpha * x + bv[j];
         }
-      }
     };
     // the output (or this split's partials), its row stride, and the aux rows
     float* Out = to_ws ? g.ws + ((int64_t)cur.split * g.batch + cur.bidx) * (int64_t)g.M * g.N
@@ -1320,14 +958,9 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
         }
     }
 
-    if (more2) {
-      SA::row_max(qa, amax[(seq + 2) & 3], tq);
-      SB::row_max(qb, amax[(seq + 2) & 3] + BM, tq);
-    }
     if (!more) break;
     tile += wgs;
     cur = next;
-    if (!g.fast || !primed) __syncthreads();
   }
 }
 
@@ -1712,9 +1345,9 @@ int launch_tile(const GemmArgs& g, bool ak, bool bn1, hipStream_t st) {
 }
 
 // Which kernel computes fp32 products of at least 128 x 128 (mtx_gemm_set_mode):
-// MTX_GEMM_BF16X3 (default) the split kernel on the 16-bit matrix cores (two
-// fp16 or three bf16 pieces), MTX_GEMM_FP32 the fp32 MFMA tile kernel.  Smaller products, and
-// the decode step's skinny ones, always take the fp32 kernels.
+// MTX_GEMM_BF16X3 (default) the split kernel on the bf16 matrix cores,
+// MTX_GEMM_FP32 the fp32 MFMA tile kernel.  Smaller products, and the decode
+// step's skinny ones, always take the fp32 kernels.
 std::atomic<int> g_gemm_mode{MTX_GEMM_BF16X3};
 
 // Products below 2^27 multiply-adds (the C0 model's 512-row ones: a handful
@@ -1736,7 +1369,9 @@ bool use_x3(int M, int N, int K, int batch) {
 
 // Two workgroups of the split kernel fit a CU.
 constexpr int kX3Wgs = 512;
-constexpr double kX3W96 = 0.8;  // a 128 x 96 tile's time against a 128 x 128 one's
+// A 128 x 96 tile's time against a 128 x 128 one's is 0.87 (4096^3: 1376 of them
+// 899 us, 1024 of those 767); a little more, so that a draw keeps the squares.
+constexpr double kX3W96 = 0.95;
 
 // Time of `tiles` tiles of weight w on kX3Wgs resident workgroups, in tile
 // times of two workgroups sharing a CU: whole rounds, and a last one in which
@@ -1749,19 +1384,19 @@ double x3_rounds(int64_t tiles, double w) {
 // Tiles of 128 x 128 or, where A is contiguous along k (forward and dX
 // products), 128 x 96: whichever ends sooner.  N = 384 is three columns of
 // 128 (M = 16384: 384 tiles, a round three quarters full) or four of 96
-// (512, one full round): K = 384 + residual 42.0 -> 38.5 us, K = 1536 91 ->
-// 83, its dX 84 -> 76.
+// (512, one full round): K = 384 + residual 41.8 -> 40.1 us, K = 1152 dX 100.8 ->
+// 96.7, K = 1536 dX 133.7 -> 126.6; N = 1152 stays (94.7 against 106.8).
 // K is split only when the 128 x 128 tiles leave the CUs idle (weight
 // gradients, K = B*T): into as many ranges as keep one round of kX3Wgs
-// workgroups, each with >= h2::MINK of K.
+// workgroups, each with >= MTX_SPLIT_MINK of K.
 Plan plan_x3(int M, int N, int K, int batch, size_t ws_bytes, bool ak, bool colsum) {
   Plan p{128, 128, 1, K};
   const int64_t t = (int64_t)cdiv(M, 128) * cdiv(N, 128) * batch;
   if (t < 256 && K >= 1024) {
-    for (int want = (int)std::min<int64_t>(K / h2::MINK, kX3Wgs / t); want > 1; --want) {
-      const int chunk = cdiv(cdiv(K, want), h2::BK) * h2::BK, ks = cdiv(K, chunk);
+    for (int want = (int)std::min<int64_t>(K / MTX_SPLIT_MINK, kX3Wgs / t); want > 1; --want) {
+      const int chunk = cdiv(cdiv(K, want), 32) * 32, ks = cdiv(K, chunk);
       const size_t need = (size_t)ks * batch * (size_t)(M + 1) * N * sizeof(float);
-      if (ks > 1 && K - (ks - 1) * chunk >= h2::MINK && need <= ws_bytes) {
+      if (ks > 1 && K - (ks - 1) * chunk >= MTX_SPLIT_MINK && need <= ws_bytes) {
         p.ksplit = ks;
         p.kchunk = chunk;
         break;
@@ -1774,15 +1409,20 @@ Plan plan_x3(int M, int N, int K, int batch, size_t ws_bytes, bool ak, bool cols
   return p;
 }
 
-// Whether the two-piece form may be tried: h2::MINK of K and more in every
-// range, and 32-bit offsets reach a tile's rows and its samples' k rows.
-bool two_pieces(const GemmArgs& g) {
-  const int64_t lim = (int64_t)1 << 29;
-  auto ok = [&](int64_t s_row, int64_t s_k) {
-    return s_row >= 0 && s_k >= 0 && (s_k == 1 ? 128 * s_row + g.kchunk : g.kchunk * s_k + 128) < lim;
+// Whether the split kernel's pipeline may run, with its unchecked loads: two
+// whole k steps in every range (a third where an operand contiguous along its
+// rows does not end on a vector, whose last step the checked loads take), and
+// 32-bit offsets to a k-tile's rows.  Such an operand's vectors, which pass the
+// last row by up to three values, stay inside it in every other step if its k
+// rows do not lie closer than that.
+bool pipelined(const GemmArgs& g, bool ak, bool bn1) {
+  const bool ra = !ak && g.M % 4, rb = bn1 && g.N % 4;
+  auto ok = [](bool kc, int64_t s_row, int64_t s_k) {
+    return s_row >= 0 && s_k >= 0 && (kc ? 128 * s_row : x3::BK * s_k) < ((int64_t)1 << 29);
   };
-  const int last = g.K - (g.ksplit - 1) * g.kchunk;
-  return std::min(g.kchunk, last) >= h2::MINK && ok(g.sam, g.sak) && ok(g.sbn, g.sbk);
+  const int least = std::min(g.kchunk, g.K - (g.ksplit - 1) * g.kchunk);
+  return least >= (ra || rb ? 3 : 2) * x3::BK && ok(ak, g.sam, g.sak) && ok(!bn1, g.sbn, g.sbk) &&
+         (!ra || g.sak >= 3) && (!rb || g.sbk >= 3);
 }
 
 template <int ACT>
@@ -1909,7 +1549,7 @@ int gemm_impl(int M, int N, int K, int batch, float alpha, const float* a, int64
                   : plan_gemm(M, N, K, batch, workspace ? workspace_bytes : 0);
   g.ksplit = p.ksplit;
   g.kchunk = p.kchunk;
-  g.fast = split3 && two_pieces(g);
+  g.fast = split3 && pipelined(g, ak, bn1);
   {
     const int64_t far = (int64_t)1 << 25;
     const bool x_ok = !act || !aux || (sx_n == 1 && sx_m >= N && sx_m < far);

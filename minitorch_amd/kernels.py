@@ -583,8 +583,8 @@ GEMM_FP32, GEMM_BF16X3 = L.MTX_GEMM_FP32, L.MTX_GEMM_BF16X3
 def set_gemm_mode(mode: int) -> int:
     """Select how products of at least 128 x 128 are computed
     (mtx_gemm_set_mode): GEMM_BF16X3 (the default: fp32 values split into
-    two fp16 or three bf16 pieces on the 16-bit matrix cores,
-    fp32-accurate) or GEMM_FP32 (fp32 MFMA).  Returns the previous mode."""
+    three bf16 pieces on the bf16 matrix cores, fp32-accurate) or GEMM_FP32
+    (fp32 MFMA).  Returns the previous mode."""
     prev = int(L.lib().mtx_gemm_get_mode())
     L.call("mtx_gemm_set_mode", int(mode))
     return prev

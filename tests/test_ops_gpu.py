@@ -773,23 +773,26 @@ def test_gemm_nonfinite_and_near_overflow(dev, gemm_mode):
         assert np.all(np.isnan(c[0])) and np.all(np.isnan(c[1]))
 
 
+def _split_tol(K, absprod):
+    """A split product's bound: 2^-22 sum |a_k b_k| for the pieces, and the
+    rounded sums: one per 16 k and a few after them, of 2^-24 of at most that
+    sum each, adding up like the square root of their number (times 4)."""
+    return (2.0 ** -22 + 4 * 2.0 ** -24 * np.sqrt(K / 16 + 8)) * absprod + 1e-37
+
+
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
-@pytest.mark.parametrize("values", ["plain", "late", "far", "tiny", "zero_start", "range"])
+@pytest.mark.parametrize("values", ["plain", "late", "far", "tiny", "zero_start", "sparse", "range"])
 @pytest.mark.parametrize("M,N,K", [(512, 4096, 256), (4101, 1003, 290), (391, 515, 2085)])
-def test_gemm_two_piece_scaling(dev, M, N, K, values, ta, tb):
-    """Split products of K >= 256 scale every row of A and column of B by its
-    values in the first 32 k; here those say little about the rest: rows and
-    columns whose later values are 2^14 times larger ("late", inside the
-    scaled form's range) or 2^30 times ("far", outside: the tile is computed
-    again from three pieces), rows of 1e-25 ("tiny", outside), rows and columns
-    that begin with 40 zeros ("zero_start") and rows spread over 2^40
-    ("range").  Odd sizes: no aligned vectors, ragged tiles on every side.
-    Bound: a value is held to 2^-23 of itself or 2^-35 of its row's largest
-    beginning value; 2^-20 of sum |a||b| covers that of both operands and the
-    fp32 accumulation (the three pieces: 2^-23 of |ab|, six sums a k step)."""
+def test_gemm_split_ranges(dev, M, N, K, values, ta, tb):
+    """Split products hold every value to its own 24 bits, whatever the rest
+    of its row or column is: single values 2^14 ("late") or 2^30 ("far") times
+    larger than the others, rows of 1e-25 ("tiny"), rows and columns that
+    begin with 40 zeros ("zero_start") or are 95% zeros ("sparse"), rows and
+    columns spread over 2^40 ("range").  Odd sizes: no aligned vectors, ragged
+    tiles on every side."""
     from minitorch_amd import kernels as Kn
 
-    _say(f"[gemm scaling] M={M} N={N} K={K} {values} ta={ta} tb={tb}")
+    _say(f"[gemm ranges] M={M} N={N} K={K} {values} ta={ta} tb={tb}")
     rng = np.random.default_rng(M + N + K)
     a = rng.standard_normal((M, K), dtype=np.float32)
     b = rng.standard_normal((K, N), dtype=np.float32)
@@ -804,6 +807,9 @@ def test_gemm_two_piece_scaling(dev, M, N, K, values, ta, tb):
         b[:40, 2::70] = 0
         a[5] = 0
         b[:, 9] = 0
+    elif values == "sparse":
+        a[rng.random((M, K)) < 0.95] = 0
+        b[rng.random((K, N)) < 0.95] = 0
     elif values == "range":
         a *= (2.0 ** rng.integers(-20, 21, (M, 1))).astype(np.float32)
         b *= (2.0 ** rng.integers(-20, 21, (1, N))).astype(np.float32)
@@ -812,11 +818,43 @@ def test_gemm_two_piece_scaling(dev, M, N, K, values, ta, tb):
     c = empty((M, N))
     Kn.gemm(ta_, tb_, c)
     ad, bd = a.astype(np.float64), b.astype(np.float64)
-    err = np.abs(H(c) - ad @ bd)
-    aa, ab = np.abs(ad), np.abs(bd)
-    lim = 2.0 ** -20 * (aa @ ab) + 2.0 ** -35 * (aa[:, :32].max(1, keepdims=True) * ab.sum(0)
-                                                 + aa.sum(1, keepdims=True) * ab[:32].max(0)) + 1e-37
+    err, lim = np.abs(H(c) - ad @ bd), _split_tol(K, np.abs(ad) @ np.abs(bd))
     assert np.all(err <= lim), (err.max(), (err / lim).max())
+
+
+@pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
+@pytest.mark.parametrize("values", [1e4, 1e6, 1e9, 1e12, "zero", "lognormal"])
+def test_gemm_unbalanced_features(dev, values, ta, tb):
+    """One input feature p times larger than the others, its weights 1 / p or
+    zero, or features of log-normal scales exp(4 N(0, 1)) with the inverse
+    weights: every term of a sum is of one size, so values far below their
+    row's largest count as much as that one.  The large feature is the first,
+    the last or one between."""
+    from minitorch_amd import kernels as Kn
+
+    M, N, K = 1024, 1024, 384
+    for at in (0, K // 2 + 3, K - 1):
+        _say(f"[gemm features] {values} at {at} ta={ta} tb={tb}")
+        rng = np.random.default_rng(at)
+        a = rng.standard_normal((M, K), dtype=np.float32)
+        b = rng.standard_normal((K, N), dtype=np.float32)
+        if values == "zero":
+            a[:, at] *= np.float32(1e6)
+            b[at] = 0
+        elif values == "lognormal":
+            d = np.exp(4 * rng.standard_normal(K)).astype(np.float32)
+            a *= d
+            b /= d[:, None]
+        else:
+            a[:, at] *= np.float32(values)
+            b[at] /= np.float32(values)
+        ta_ = T(np.ascontiguousarray(a.T)).transpose(0, 1) if ta else T(a)
+        tb_ = T(np.ascontiguousarray(b.T)).transpose(0, 1) if tb else T(b)
+        c = empty((M, N))
+        Kn.gemm(ta_, tb_, c)
+        ad, bd = a.astype(np.float64), b.astype(np.float64)
+        err, lim = np.abs(H(c) - ad @ bd), _split_tol(K, np.abs(ad) @ np.abs(bd))
+        assert np.all(err <= lim), (values, at, (err / lim).max())
 
 
 def test_failed_capture_releases_its_pool(dev):
