@@ -559,6 +559,20 @@ struct X3Stage {
   }
 };
 
+// Epilogue accesses past the last column take the offset kPastRow, and no row
+// resource may reach it: its bytes are cut at kRowEnd (a wave's rows lie within
+// 2^30 bytes, so no element of theirs is cut off).  Uncut, the 4 GiB less 12, 8
+// or 4 bytes that can lie between a row and the array's end would take such a
+// store in.
+constexpr uint32_t kRowEnd = 0xffffff00u, kPastRow = 0xfffffff0u;
+constexpr uint32_t row_bytes(int64_t left) {
+  return left < 0 ? 0u : left > (int64_t)kRowEnd ? kRowEnd : (uint32_t)left;
+}
+static_assert(row_bytes(((int64_t)1 << 32) - 12) <= kPastRow && row_bytes(((int64_t)1 << 32) - 4) <= kPastRow &&
+                  row_bytes((int64_t)1 << 32) <= kPastRow && row_bytes((int64_t)1 << 40) <= kPastRow &&
+                  row_bytes(-4) == 0 && row_bytes(kRowEnd - 4) == kRowEnd - 4,
+              "stores past the last column are dropped");
+
 // a thread or lane number whose uses are computed where they stand: code that
 // runs once a tile or less otherwise keeps its addresses in registers across
 // the k loop, which needs them all
@@ -849,8 +863,8 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
 #pragma unroll
       for (int j = 0; j < NI; ++j) {
         const bool ok = n1 + 32 * j + lr < g.N;
-        oo[j] = ok ? (uint32_t)(4 * lh * so + 32 * j + lr) * 4u : 0xfffffff0u;
-        xo[j] = ok ? (uint32_t)(4 * lh * g.sxm + 32 * j + lr) * 4u : 0xfffffff0u;
+        oo[j] = ok ? (uint32_t)(4 * lh * so + 32 * j + lr) * 4u : kPastRow;
+        xo[j] = ok ? (uint32_t)(4 * lh * g.sxm + 32 * j + lr) * 4u : kPastRow;
       }
       // the wave's rows of an array: a resource at row r (rows are asked for in
       // steps, the address and the bytes left move by uniform additions)
@@ -858,10 +872,8 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
         const char* p;
         int64_t left, step;
         __device__ __forceinline__ __amdgpu_buffer_rsrc_t at(int r) const {
-          const int64_t l = left - r * step;
-          const int hi = (int)(l >> 32);
-          const uint32_t bytes = hi < 0 ? 0u : hi > 0 ? 0xffffff00u : (uint32_t)l;
-          return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p + r * step), (short)0, (int)bytes, 0x00020000);
+          return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p + r * step), (short)0,
+                                                   (int)row_bytes(left - r * step), 0x00020000);
         }
       };
       const int mw = cur.m0 + wm;

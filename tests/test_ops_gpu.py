@@ -857,6 +857,27 @@ def test_gemm_unbalanced_features(dev, values, ta, tb):
         assert np.all(err <= lim), (values, at, (err / lim).max())
 
 
+def test_gemm_rows_near_four_gib(dev):
+    """A C of which 2^32 - 12 bytes follow its first row's second column tile
+    (from 2^32 - 16 on, the columns past N are told apart by their offset):
+    its first and last rows, added to zeros so that a stray store into the last
+    element stays in the result."""
+    from minitorch_amd import kernels as Kn
+
+    M, N, K = 7304367, 147, 8
+    assert ((M - 1) * N + N - 128) * 4 == 2 ** 32 - 12
+    _say(f"[gemm near 4 GiB] M={M} N={N} K={K}")
+    rng = np.random.default_rng(0)
+    a = np.resize(rng.standard_normal((K, 4099), dtype=np.float32), (K, M))
+    b = rng.standard_normal((K, N), dtype=np.float32)
+    c = empty((M, N))
+    c.fill_(0.0)
+    Kn.gemm(T(a).transpose(0, 1), T(b), c, beta=1.0)
+    for rows in (slice(0, 300), slice(M - 300, M)):
+        ref = a[:, rows].T.astype(np.float64) @ b.astype(np.float64)
+        close(H(c[rows]), ref, atol=dot_tol(K), name=str(rows))
+
+
 def test_failed_capture_releases_its_pool(dev):
     """A capture that fails at mtx_graph_end (invalidated by synchronising
     the capturing stream) releases its memory pool: a block freed into that
