@@ -1366,17 +1366,20 @@ std::atomic<int> g_gemm_mode{MTX_GEMM_BF16X3};
 // of 128 x 128 tiles, latency bound) stay on the fp32 kernel's 64 x 64
 // tiles: on the split kernel the C0 training step took 0.445 ms against
 // 0.379 ms.
-// Nor do products with fewer than 64 tiles of 128 x 128 and a K too short to
-// split (< 1024): at K = 384 the fp32 kernel's 64 x 64 tiles and the split
-// kernel took 19.8 and 20 us for 1000 x 384 (24 tiles), 24.5 and 21.9 for
-// 2944 x 384 (69), 22.9 and 19.6 for 1000 x 1152 (72), 26.7 and 25.1 for
-// 1000 x 1536 + GELU (96); 8008 x 512 x 512 (252) 48.4 and 36.4.
+// So do products with K too short to split (< 1024) whose 64 x 64 tiles take
+// the fp32 kernel at most two rounds of the 256 CUs (512 tiles), and, below K =
+// 128, four.  fp32 and split kernel, us: 256 tiles 13.7 and 23.1 (1024 x 1024 x
+// 384), 512 tiles 10.2 and 13.2 (16384 x 128 x 128), 21.2 and 24.4 (4096 x 512 x
+// 384), 36.6 and 40.9 (K = 768); 576 tiles 12.8 and 12.9 (2048 x 1152 x 128), 27.2
+// and 24.6 (K = 384); 1008 tiles 11.5 and 12.4 (8008 x 512 x 64), 37.5 and 28.8 (K =
+// 384); 1536 tiles 15.7 and 13.9 (16384 x 384 x 64), 52.8 and 37.8 (K = 384); 2048
+// tiles 19.3 and 13.3 (8192 x 1024 x 32).
 bool use_x3(int M, int N, int K, int batch) {
   if (g_gemm_mode.load(std::memory_order_relaxed) != MTX_GEMM_BF16X3 || M < 128 || N < 128 ||
       (int64_t)M * N * K * batch < ((int64_t)1 << 27))
     return false;
-  const int64_t tiles = (int64_t)cdiv(M, 128) * cdiv(N, 128) * batch;
-  return tiles >= 64 || K >= 1024;
+  const int64_t tiles = (int64_t)cdiv(M, 64) * cdiv(N, 64) * batch;
+  return K >= 1024 || tiles > (K >= 128 ? 512 : 1024);
 }
 
 // Two workgroups of the split kernel fit a CU.

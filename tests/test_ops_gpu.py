@@ -65,8 +65,8 @@ def dot_tol(K):
     (64, 384, 1536, False, False, 1, True),     # skinny, K split over 3 workgroups
     (17, 40, 1000, True, False, 2, True),       # skinny split, scalar A loads, batched
     (64, 64, 4100, False, False, 1, False),     # K past the skinny range: tiled split-K
-    # >= 128 x 128 and >= 2^27 multiply-adds, with K >= 1024 or >= 256 tiles of
-    # 128 x 128: the bf16-split kernel in its default mode
+    # >= 128 x 128 and >= 2^27 multiply-adds, with K >= 1024 or > 512 tiles of
+    # 64 x 64 (1024 with K < 128): the bf16-split kernel in its default mode
     (256, 384, 1400, False, True, 1, True),     # ragged last k-tile, B contiguous along k
     (300, 260, 1111, True, True, 2, True),      # edge tiles on both sides, both operands transposed
     (4100, 1000, 33, False, False, 1, True),    # row strides of 33: no aligned vector loads
@@ -566,7 +566,7 @@ def test_gemm_gelu_epilogues(dev, gemm_mode, M, N, K):
     aux, act 2 = (A@B) * gelu'(aux), against NumPy float64 (the K = 8192 case
     takes the split-K path, whose reduce applies the epilogue; 2048 x 2048
     the split-bf16 kernel's own epilogue in its default mode, 512 x 1536 --
-    48 tiles of 128 x 128 with K < 1024 -- the fp32 kernel in both)."""
+    192 tiles of 64 x 64 with K < 1024 -- the fp32 kernel in both)."""
 
     from minitorch_amd import kernels as K_
 
@@ -782,7 +782,7 @@ def _split_tol(K, absprod):
 
 @pytest.mark.parametrize("ta,tb", [(False, False), (False, True), (True, False), (True, True)])
 @pytest.mark.parametrize("values", ["plain", "late", "far", "tiny", "zero_start", "sparse", "range"])
-@pytest.mark.parametrize("M,N,K", [(512, 4096, 256), (4101, 1003, 290), (391, 515, 2085)])
+@pytest.mark.parametrize("M,N,K", [(576, 4096, 256), (4101, 1003, 290), (391, 515, 2085)])
 def test_gemm_split_ranges(dev, M, N, K, values, ta, tb):
     """Split products hold every value to its own 24 bits, whatever the rest
     of its row or column is: single values 2^14 ("late") or 2^30 ("far") times
@@ -832,7 +832,7 @@ def test_gemm_unbalanced_features(dev, values, ta, tb):
     the last or one between."""
     from minitorch_amd import kernels as Kn
 
-    M, N, K = 1024, 1024, 384
+    M, N, K = 2048, 1280, 384
     for at in (0, K // 2 + 3, K - 1):
         _say(f"[gemm features] {values} at {at} ta={ta} tb={tb}")
         rng = np.random.default_rng(at)
