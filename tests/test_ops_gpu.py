@@ -857,6 +857,135 @@ def test_gemm_unbalanced_features(dev, values, ta, tb):
         assert np.all(err <= lim), (values, at, (err / lim).max())
 
 
+@pytest.mark.parametrize("M,N,K,batch,ta,tb", [
+    (8200, 2050, 50, 1, False, False),    # 65 x 17 tiles: up to three a workgroup; three k steps and a bit
+    (8200, 2050, 50, 1, True, True),
+    (8199, 2049, 48, 1, True, False),     # three whole k steps, the last one read by element
+    (4100, 4100, 33, 1, False, True),     # two whole k steps and one value
+    (9000, 2000, 20, 1, False, False),    # too short for the pipeline
+    (4100, 2050, 301, 1, True, False),
+    (1100, 1000, 70, 20, False, True),    # 9 x 8 tiles in each of 20 batches
+    (1030, 650, 130, 31, True, True),
+    (33001, 286, 70, 1, False, False),    # tiles of 128 x 96, 258 x 3
+    (11000, 288, 48, 4, False, True),
+])
+def test_gemm_split_many_tiles(dev, M, N, K, batch, ta, tb):
+    """Split products of more tiles than the 512 workgroups of a launch, which
+    take several each: the next tile's first k steps are staged during the
+    last ones of the tile before, across ragged rows, columns and k, and
+    batches."""
+    from minitorch_amd import kernels as Kn
+
+    _say(f"[gemm many tiles] M={M} N={N} K={K} batch={batch} ta={ta} tb={tb}")
+    rng = np.random.default_rng(M + N + K)
+    a = rng.standard_normal((batch, M, K), dtype=np.float32)
+    b = rng.standard_normal((batch, K, N), dtype=np.float32)
+    ta_ = T(np.swapaxes(a, 1, 2)).transpose(1, 2) if ta else T(a)
+    tb_ = T(np.swapaxes(b, 1, 2)).transpose(1, 2) if tb else T(b)
+    c = empty((batch, M, N))
+    Kn.gemm(ta_, tb_, c, batch=batch)
+    got = H(c)
+    for i in range(batch):
+        ad, bd = a[i].astype(np.float64), b[i].astype(np.float64)
+        err, lim = np.abs(got[i] - ad @ bd), _split_tol(K, np.abs(ad) @ np.abs(bd))
+        assert np.all(err <= lim), (i, err.max(), (err / lim).max())
+
+
+@pytest.mark.parametrize("M,N,K", [(8200, 2050, 130), (16384, 384, 384), (33001, 286, 70)])
+def test_gemm_split_many_tiles_epilogues(dev, M, N, K):
+    """The epilogues of the split kernel between a workgroup's tiles: bias and
+    beta C, GELU with the pre-activation stored, GELU' and a residual; rows of
+    C and aux wider than N keep what lies beyond it."""
+    from minitorch_amd import kernels as Kn
+
+    _say(f"[gemm many tiles, epilogues] M={M} N={N} K={K}")
+    rng = np.random.default_rng(M + N + K)
+    a = rng.standard_normal((M, K), dtype=np.float32) / np.float32(np.sqrt(K))
+    b = rng.standard_normal((K, N), dtype=np.float32)
+    bias, x = rng.standard_normal(N, dtype=np.float32), rng.standard_normal((M, N + 3), dtype=np.float32)
+    ta, tb, tbias = T(a), T(b), T(bias)
+    ad, bd = a.astype(np.float64), b.astype(np.float64)
+    prod, lim = ad @ bd, _split_tol(K, np.abs(ad) @ np.abs(bd))
+    xd = x[:, :N].astype(np.float64)
+    u = lambda v: 0.7978845834732056 * (v + 0.044714998453855515 * v ** 3)
+    gelu = lambda v: 0.5 * v * (1 + np.tanh(u(v)))
+    t = np.tanh(u(xd))
+    dgelu = 0.5 * (1 + t) + 0.5 * xd * (1 - t * t) * 0.7978845834732056 * (1 + 3 * 0.044714998453855515 * xd ** 2)
+
+    def check(got, ref, tol, keeps=True):
+        # two more rounded operations and the GELU's 2^-21
+        err = np.abs(got[:, :N] - ref)
+        assert np.all(err <= tol + 2.0 ** -21 * (np.abs(ref) + 1)), err.max()
+        if keeps:
+            np.testing.assert_array_equal(got[:, N:], x[:, N:])
+
+    c = T(x)
+    Kn.gemm(ta, tb, c[:, :N], beta=0.5, bias=tbias)
+    check(H(c), prod + bias + 0.5 * xd, lim)
+    c, h = T(x), T(x)
+    Kn.gemm(ta, tb, c[:, :N], bias=tbias, act=Kn.GEMM_ACT_GELU, aux=h[:, :N])
+    check(H(h), prod + bias, lim)
+    check(H(c), gelu(prod + bias), 2 * lim)
+    c = T(x)
+    Kn.gemm(ta, tb, c[:, :N], act=Kn.GEMM_ACT_GELU_BWD, aux=T(x)[:, :N])
+    check(H(c), prod * dgelu, 2 * lim + 2.0 ** -21 * np.abs(prod))
+    c = T(x)
+    Kn.gemm(ta, tb, c[:, :N], bias=tbias, act=Kn.GEMM_ACT_ADD, aux=T(x)[:, :N])
+    check(H(c), prod + bias + xd, lim)
+
+
+@pytest.mark.parametrize("M,N,K,ta,tb", [(4100, 2050, 300, True, False), (4100, 2050, 40, True, True),
+                                         (8200, 1030, 18, False, False), (5000, 2049, 129, False, True)])
+def test_gemm_split_many_tiles_colsum(dev, M, N, K, ta, tb):
+    """Column sums of B beside an unsplit product whose workgroups take
+    several tiles each: the sums change over to the next tile's while its
+    first k step is staged."""
+    from minitorch_amd import kernels as Kn
+
+    _say(f"[gemm many tiles, column sums] M={M} N={N} K={K} ta={ta} tb={tb}")
+    rng = np.random.default_rng(M + N + K)
+    a, b = rng.standard_normal((M, K), dtype=np.float32), rng.standard_normal((K, N), dtype=np.float32)
+    s0 = rng.standard_normal(N, dtype=np.float32)
+    ta_ = T(np.ascontiguousarray(a.T)).transpose(0, 1) if ta else T(a)
+    tb_ = T(np.ascontiguousarray(b.T)).transpose(0, 1) if tb else T(b)
+    c, s = empty((M, N)), T(s0)
+    Kn.gemm(ta_, tb_, c, colsum=s, colsum_accumulate=True)
+    ad, bd = a.astype(np.float64), b.astype(np.float64)
+    err = np.abs(H(c) - ad @ bd)
+    assert np.all(err <= _split_tol(K, np.abs(ad) @ np.abs(bd))), err.max()
+    # a thread's chain of K / 4 sums, eight threads and the old value
+    assert np.all(np.abs(H(s) - (s0 + bd.sum(0))) <= 2.0 ** -24 * (K / 4 + 12) * (np.abs(bd).sum(0) + np.abs(s0)))
+
+
+@pytest.mark.parametrize("sk", [0, 1, 2, 3])
+@pytest.mark.parametrize("side", ["a", "b"])
+def test_gemm_split_near_k_rows(dev, side, sk):
+    """An operand whose k rows lie 0 (one row for every k) to 3 values apart,
+    its row count no multiple of a load's four values: the loads that pass the
+    last row reach the operand's end in steps before the last."""
+    from minitorch_amd import kernels as Kn
+
+    _say(f"[gemm near k rows] {side} {sk}")
+    R, S, K = 1030, 2048, 300
+    rng = np.random.default_rng(sk)
+    base = rng.standard_normal(R + sk * (K - 1), dtype=np.float32)
+    x = base[np.arange(R)[:, None] + sk * np.arange(K)]
+    other = rng.standard_normal((S, K), dtype=np.float32)
+    # the near rows end with their allocation
+    tx = T(base)
+    if side == "a":
+        c = empty((R, S))
+        Kn.gemm(tx, T(np.ascontiguousarray(other.T)), c, M=R, N=S, K=K, sa=(1, sk, 0), sb=(S, 1, 0))
+        left, right = x, other.T
+    else:
+        c = empty((S, R))
+        Kn.gemm(T(other), tx, c, M=S, N=R, K=K, sa=(K, 1, 0), sb=(sk, 1, 0))
+        left, right = other, x.T
+    ld, rd = left.astype(np.float64), right.astype(np.float64)
+    err, lim = np.abs(H(c) - ld @ rd), _split_tol(K, np.abs(ld) @ np.abs(rd))
+    assert np.all(err <= lim), (err.max(), (err / lim).max())
+
+
 def test_gemm_rows_near_four_gib(dev):
     """A C of which 2^32 - 12 bytes follow its first row's second column tile
     (from 2^32 - 16 on, the columns past N are told apart by their offset):
