@@ -141,7 +141,9 @@ def test_reduce_sum(dev, shape, axes):
 def test_reduce_contiguous_runs(dev, rows, n, pad):
     """Sum and max over the last axis (runs of 256 and more take the kernel of
     their own), rows starting at any 4-byte address, accumulated into an
-    output; the sum twice gives the same bits."""
+    output; the sum twice gives the same bits.  Whole numbers small enough for
+    every partial sum to be exact have to come out exactly (each of them
+    counts once)."""
     from minitorch_amd import _lib as L
     from minitorch_amd import kernels as Kn
 
@@ -156,12 +158,63 @@ def test_reduce_contiguous_runs(dev, rows, n, pad):
         Kn.reduce(ta, [1], out, alpha=0.5, accumulate=True)
         got.append(H(out))
     x = a[:, pad:].astype(np.float64)
-    # every value passes through at most log2(n) + 48 rounded sums of a chunk
-    assert np.all(np.abs(got[0] - (base + 0.5 * x.sum(1))) <= 2.0 ** -24 * 70 * np.abs(x).sum(1))
+    ref = base + 0.5 * x.sum(1)
+    # a chunk is added in float64 and rounded once, the chunks likewise, then
+    # the product with 0.5 (exact) is added to the output
+    mask = (L.C.c_int * 2)(0, 1)
+    ws = L.lib().mtx_reduce_workspace_bytes(2, (L.C.c_int64 * 2)(rows, n), mask)
+    chunk = -(-n // max(1, min(ws // (4 * rows), n // 16384)))
+    parts = np.add.reduceat(x, np.arange(0, n, chunk), axis=1)
+    lim = 1.01 * 2.0 ** -24 * (0.5 * np.abs(parts).sum(1) + 0.5 * np.abs(x.sum(1)) + np.abs(ref))
+    assert np.all(np.abs(got[0] - ref) <= lim), (np.abs(got[0] - ref) / lim).max()
     assert np.array_equal(got[0], got[1])
+    whole = (rng.integers(1, 3, (rows, n + pad)) * rng.choice([-1, 1], (rows, n + pad))).astype(np.float32)
+    tw, out = T(whole)[:, pad:], T(np.arange(rows))
+    Kn.reduce(tw, [1], out, alpha=0.5, accumulate=True)
+    np.testing.assert_array_equal(H(out), np.arange(rows) + 0.5 * whole[:, pad:].astype(np.float64).sum(1))
     mx = empty((rows,))
     Kn.reduce(ta, [1], mx, op=L.RED_MAX)
     assert np.array_equal(H(mx), a[:, pad:].max(1))
+
+
+@pytest.mark.parametrize("n", [256, 1027, 40000])
+def test_reduce_runs_special_values(dev, n):
+    """Rows with NaN, infinities, -inf alone, fp32's lowest value alone and
+    signed zeros: the kernel for contiguous runs gives what the general one
+    gives of the same values in columns, and NumPy's fmax and sum."""
+    from minitorch_amd import _lib as L
+    from minitorch_amd import kernels as Kn
+
+    _say(f"[reduce runs, special values] {n}")
+    rng = np.random.default_rng(n)
+    low = np.finfo(np.float32).min
+    a = rng.standard_normal((9, n), dtype=np.float32)
+    a[0, n // 3] = np.nan
+    a[1] = np.nan
+    a[2, n - 1] = np.inf
+    a[3, 0], a[3, n // 2] = np.inf, -np.inf
+    a[4] = -np.inf
+    a[5] = low
+    a[6, n - 1] = -np.inf
+    a[7] = -0.0
+    a[8, :-1], a[8, -1] = low, np.nan
+    rows, cols = T(a), T(np.ascontiguousarray(a.T))
+    for op, f in ((L.RED_MAX, np.fmax.reduce), (L.RED_SUM, np.add.reduce)):
+        x, y = empty((9,)), empty((9,))
+        Kn.reduce(rows, [1], x, op=op)
+        Kn.reduce(cols, [0], y, op=op)
+        with np.errstate(invalid="ignore", over="ignore"):
+            ref = f(a.astype(np.float64), axis=1).astype(np.float32)
+        if op == L.RED_MAX:
+            ref[1] = -np.inf  # a row of NaN alone: where the maximum starts
+            np.testing.assert_array_equal(H(x), ref)
+            np.testing.assert_array_equal(H(y), ref)
+        else:
+            # (sums of ordinary values differ in their rounding)
+            odd = ~np.isfinite(ref)
+            odd[7] = True
+            np.testing.assert_array_equal(H(x)[odd], ref[odd])
+            np.testing.assert_array_equal(H(y)[odd], ref[odd])
 
 
 def test_reduce_runs_of_many_outputs(dev):
