@@ -100,8 +100,8 @@ __global__ __launch_bounds__(256) void reduce_kernel(const RedArgs g) {
 }
 
 // Reduced values that lie one after another in memory (sum of everything, of
-// the last axis): a workgroup per output and chunk, its 256 threads reading
-// float4 vectors side by side, four in flight each, and adding them in
+// the last axis): a workgroup or wave per output and chunk, its threads
+// reading float4 vectors side by side, four in flight each, and adding them in
 // float64 (free beside the reads: HBM bound), so a chunk's sum is rounded
 // once.  reduce_kernel gives an output four threads and a read four values:
 // the sum of 64 x 256 x 384 values took 142 + 8 us (512 chunks and their
@@ -111,49 +111,62 @@ struct __attribute__((packed, aligned(4))) unaligned4 {
 };
 __device__ __forceinline__ double red_op(bool is_max, double a, double b) { return is_max ? fmax(a, b) : a + b; }
 
-// the block's 256 values in a fixed order; the result in thread 0
-__device__ __forceinline__ double block_reduce(bool is_max, double v) {
-  __shared__ double part[4];
+// a wave's 64 values, and the block's 256 (the result in thread 0), in a fixed order
+__device__ __forceinline__ double wave_reduce(bool is_max, double v) {
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) v = red_op(is_max, v, __shfl_xor(v, m, 64));
+  return v;
+}
+__device__ __forceinline__ double block_reduce(bool is_max, double v) {
+  __shared__ double part[4];
+  v = wave_reduce(is_max, v);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
   __syncthreads();
   return red_op(is_max, red_op(is_max, part[0], part[1]), red_op(is_max, part[2], part[3]));
 }
 
+// W: the waves of an output, 4 (its workgroup) or 1.  A workgroup per run of a
+// few hundred values has a float4 or less per thread and costs its launch and
+// the exchange: 262144 x 256 127 us in reduce_kernel, 266 with four waves a run, 81
+// with one (3.3 TB/s); 16384 x 384 14.7, 20.2 and 8.3; 16384 x 2048 63.5, 27.6 and
+// 21.6; 16384 x 4096 125, 40.0 and 41.5; 16 x 8192 6.7, 3.5 and 4.7.
+template <int W>
 __global__ __launch_bounds__(256) void reduce_run_kernel(const RedArgs g) {
-  const int64_t o = blockIdx.x;
+  constexpr int T = 64 * W;
+  const int64_t o = W == 4 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int t = threadIdx.x % T;
   const int s = blockIdx.y;
+  if (o >= g.nout) return;
   const bool is_max = g.op == MTX_RED_MAX;
   const float* __restrict__ base = g.a + kept_offset(g, o);
   const int64_t r0 = (int64_t)s * g.chunk, r1 = min(g.nred, r0 + g.chunk);
   const double init = is_max ? -INFINITY : 0.0;
   double acc[4] = {init, init, init, init};
   const int64_t r4 = r0 + max((int64_t)0, (r1 - r0) / 4 * 4);
-  int64_t r = r0 + 4 * threadIdx.x;
-  for (; r + 3 * 1024 < r4; r += 4 * 1024) {
+  int64_t r = r0 + 4 * t;
+  for (; r + 3 * 4 * T < r4; r += 4 * 4 * T) {
     unaligned4 x[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const unaligned4*>(base + r + 1024 * u);
+    for (int u = 0; u < 4; ++u) x[u] = *reinterpret_cast<const unaligned4*>(base + r + 4 * T * u);
 #pragma unroll
     for (int u = 0; u < 4; ++u)
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[j] = red_op(is_max, acc[j], x[u].v[j]);
   }
-  for (; r < r4; r += 1024) {
+  for (; r < r4; r += 4 * T) {
     const unaligned4 x = *reinterpret_cast<const unaligned4*>(base + r);
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[j] = red_op(is_max, acc[j], x.v[j]);
   }
-  r = r4 + threadIdx.x;
+  r = r4 + t;
   if (r < r1) acc[0] = red_op(is_max, acc[0], base[r]);
-  const float t =
-      (float)block_reduce(is_max, red_op(is_max, red_op(is_max, acc[0], acc[1]), red_op(is_max, acc[2], acc[3])));
-  if (threadIdx.x != 0) return;
+  const double mine = red_op(is_max, red_op(is_max, acc[0], acc[1]), red_op(is_max, acc[2], acc[3]));
+  const float all = (float)(W == 4 ? block_reduce(is_max, mine) : wave_reduce(is_max, mine));
+  if (t != 0) return;
   if (g.nsplit > 1) {
-    g.ws[(int64_t)s * g.nout + o] = t;
+    g.ws[(int64_t)s * g.nout + o] = all;
   } else {
-    float v = g.alpha * t;
+    float v = g.alpha * all;
     if (g.accumulate) v += g.out[o];
     g.out[o] = v;
   }
@@ -270,15 +283,18 @@ extern "C" int mtx_reduce_f32(int op, int ndim, const int64_t* shape, const floa
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int bx = (int)((nout + 63) / 64);
   MTX_CHECK_SHAPE((nout + 63) / 64 < (1 << 30), "reduce: too many outputs");
-  // Runs of 256 values and more (shorter ones leave most of a workgroup's
-  // threads without a value), in chunks of 16384 and more: the mean of 16384
-  // row losses took 4.1 + 4.9 us in 256 chunks of reduce_kernel's, one
-  // workgroup 4.0.  (A launch has fewer than 2^32 threads.)
+  // Runs of 256 values and more (shorter ones leave lanes of a wave without a
+  // vector), in chunks of 16384 and more: the mean of 16384 row losses took 4.1 +
+  // 4.9 us in 256 chunks of reduce_kernel's, one workgroup 4.0.  (A launch has
+  // fewer than 2^32 threads.)
   if (g.nr == 1 && g.rstr[0] == 1 && nred >= 256 && nout < (1 << 24)) {
     s = (int)std::max<int64_t>(1, std::min<int64_t>(s, nred / 16384));
     g.nsplit = s;
     g.chunk = (nred + s - 1) / s;
-    hipLaunchKernelGGL(reduce_run_kernel, dim3((unsigned)nout, s), dim3(256), 0, st, g);
+    if (nred < 4096)  // a wave per run: fewer values than four waves' first loads
+      hipLaunchKernelGGL(reduce_run_kernel<1>, dim3((unsigned)((nout + 3) / 4)), dim3(256), 0, st, g);
+    else
+      hipLaunchKernelGGL(reduce_run_kernel<4>, dim3((unsigned)nout, s), dim3(256), 0, st, g);
     MTX_LAUNCHED();
     if (s > 1) {
       hipLaunchKernelGGL(reduce_run_combine_kernel, dim3((unsigned)nout), dim3(256), 0, st, g);

@@ -137,7 +137,8 @@ def test_reduce_sum(dev, shape, axes):
 
 
 @pytest.mark.parametrize("rows,n,pad", [(1, 256, 0), (1, 16384, 0), (1, 1000003, 1), (3, 70001, 3), (200, 257, 0),
-                                        (5, 4099, 2), (1, 6291456, 0)])
+                                        (5, 4099, 2), (1, 6291456, 0), (4099, 256, 1), (2050, 1027, 0), (7, 4095, 3),
+                                        (6, 4096, 0)])
 def test_reduce_contiguous_runs(dev, rows, n, pad):
     """Sum and max over the last axis (runs of 256 and more take the kernel of
     their own), rows starting at any 4-byte address, accumulated into an
