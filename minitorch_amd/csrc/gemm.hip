@@ -573,6 +573,10 @@ static_assert(row_bytes(((int64_t)1 << 32) - 12) <= kPastRow && row_bytes(((int6
                   row_bytes(-4) == 0 && row_bytes(kRowEnd - 4) == kRowEnd - 4,
               "stores past the last column are dropped");
 
+struct __attribute__((packed, aligned(4))) unaligned4 {
+  float v[4];
+};
+
 // a thread or lane number whose uses are computed where they stand: code that
 // runs once a tile or less otherwise keeps its addresses in registers across
 // the k loop, which needs them all
@@ -943,30 +947,66 @@ __global__ __launch_bounds__(kGT, 2) void gemm_x3_kernel(const GemmArgs g) {
         if (iq + kAhead < 4 * MI) aux(iq + kAhead);
       }
     } else {
+      // Other outputs (C transposed, rows that overlap) and aux arrays: an
+      // element's four rows 4 lh .. + 3 of a column together, as one vector
+      // where they lie side by side.  One element at a time took 168 us for 4096 x
+      // 4096 x 512 into a transposed C, this 119.
+      auto get = [](const float* p, int64_t step, int n, float (&x)[4]) {
+        if (step == 1 && n == 4) {
+          const unaligned4 f = *reinterpret_cast<const unaligned4*>(p);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) x[u] = f.v[u];
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) x[u] = u < n ? p[u * step] : 0.f;
+        }
+      };
+      auto set = [](float* p, int64_t step, int n, const float (&x)[4]) {
+        if (step == 1 && n == 4) {
+          *reinterpret_cast<unaligned4*>(p) = {x[0], x[1], x[2], x[3]};
+        } else {
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            if (u < n) p[u * step] = x[u];
+        }
+      };
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           float v[4][NI];
           values(i, q, v);
+          const int m = cur.m0 + wm + 32 * i + 8 * q + 4 * lh, nr = min(4, g.M - m);
 #pragma unroll
-          for (int u = 0; u < 4; ++u)
+          for (int j = 0; j < NI; ++j) {
+            const int n = n1 + 32 * j + lr;
+            if (nr <= 0 || n >= g.N) continue;
+            float* p = Out + (int64_t)m * so + (int64_t)n * (to_ws ? 1 : g.scn);
+            float* xp = X + (int64_t)m * g.sxm + (int64_t)n * g.sxn;
+            float w[4], o[4];
 #pragma unroll
-            for (int j = 0; j < NI; ++j) {
-              const int m = cur.m0 + wm + 32 * i + 8 * q + 4 * lh + u, n = n1 + 32 * j + lr;
-              if (m >= g.M || n >= g.N) continue;
-              float* p = Out + (int64_t)m * so + (int64_t)n * (to_ws ? 1 : g.scn);
-              float* xp = X + (int64_t)m * g.sxm + (int64_t)n * g.sxn;
-              float w = v[u][j];
-              if (rd_c) w += g.beta * *p;
-              if constexpr (ACT == 1) {
-                if (use_x) *xp = w;
-                w = to_ws ? w : gelu_tanh_fast(w);
-              }
-              if constexpr (ACT == 2) w = use_x ? w * gelu_grad_fast(*xp) : w;
-              if constexpr (ACT == 4) w = use_x ? w + *xp : w;
-              *p = w;
+            for (int u = 0; u < 4; ++u) w[u] = v[u][j];
+            if (rd_c) {
+              get(p, so, nr, o);
+#pragma unroll
+              for (int u = 0; u < 4; ++u) w[u] += g.beta * o[u];
             }
+            if constexpr (ACT == 1) {
+              if (use_x) set(xp, g.sxm, nr, w);
+              if (!to_ws) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) w[u] = gelu_tanh_fast(w[u]);
+              }
+            }
+            if constexpr (ACT == 2 || ACT == 4) {
+              if (use_x) {
+                get(xp, g.sxm, nr, o);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) w[u] = ACT == 2 ? w[u] * gelu_grad_fast(o[u]) : w[u] + o[u];
+              }
+            }
+            set(p, so, nr, w);
+          }
         }
     }
 
@@ -1567,7 +1607,8 @@ int gemm_impl(int M, int N, int K, int batch, float alpha, const float* a, int64
   g.fast = split3 && pipelined(g, ak, bn1);
   {
     const int64_t far = (int64_t)1 << 25;
-    const bool x_ok = !act || !aux || (sx_n == 1 && sx_m >= N && sx_m < far);
+    // aux rows that are only read may overlap (a row for all of them: stride 0)
+    const bool x_ok = !act || !aux || (sx_n == 1 && (act != 1 || sx_m >= N) && sx_m < far);
     g.rows_vec = p.ksplit > 1 ? N < far : sc_n == 1 && sc_m >= N && sc_m < far && x_ok;
   }
   int rc = split3 ? launch_x3(g, p.bn, ak, bn1, st)

@@ -1011,6 +1011,68 @@ def test_gemm_split_many_tiles_colsum(dev, M, N, K, ta, tb):
     assert np.all(np.abs(H(s) - (s0 + bd.sum(0))) <= 2.0 ** -24 * (K / 4 + 12) * (np.abs(bd).sum(0) + np.abs(s0)))
 
 
+@pytest.mark.parametrize("M,N,K", [(2050, 1283, 130), (2049, 1282, 50)])
+def test_gemm_split_output_forms(dev, M, N, K):
+    """Outputs and aux arrays of the split kernel other than plain rows: C
+    transposed (its rows' neighbours stored together, at the last rows one by
+    one) or with both strides wide, aux transposed, one row or one column of
+    it for all, with beta C, GELU and its pre-activation, GELU' and the
+    residual add."""
+    from minitorch_amd import kernels as Kn
+
+    _say(f"[gemm output forms] M={M} N={N} K={K}")
+    rng = np.random.default_rng(M)
+    a = rng.standard_normal((M, K), dtype=np.float32) / np.float32(np.sqrt(K))
+    b = rng.standard_normal((K, N), dtype=np.float32)
+    ta, tb = T(a), T(b)
+    ad, bd = a.astype(np.float64), b.astype(np.float64)
+    prod, lim = ad @ bd, _split_tol(K, np.abs(ad) @ np.abs(bd))
+    u = lambda v: 0.7978845834732056 * (v + 0.044714998453855515 * v ** 3)
+    gelu = lambda v: 0.5 * v * (1 + np.tanh(u(v)))
+
+    def dgelu(v):
+        t = np.tanh(u(v))
+        return 0.5 * (1 + t) + 0.5 * v * (1 - t * t) * 0.7978845834732056 * (1 + 3 * 0.044714998453855515 * v ** 2)
+
+    def view(x, form):
+        """A device array that reads as x (M, N) in one of the forms."""
+        if form == "rows":
+            return T(x)
+        if form == "columns":
+            return T(np.ascontiguousarray(x.T)).transpose(0, 1)
+        if form == "wide":
+            return T(np.repeat(np.repeat(x, 2, 0), 3, 1))[::2, ::3]
+        if form == "one row":
+            return T(x[:1].copy()).expand(M, N)
+        return T(x[:, :1].copy()).expand(M, N)
+
+    def check(got, ref, tol):
+        err = np.abs(H(got.contiguous()) - ref)
+        assert np.all(err <= tol + 2.0 ** -21 * (np.abs(ref) + 1)), err.max()
+
+    c0 = rng.standard_normal((M, N), dtype=np.float32)
+    for form in ("columns", "wide"):
+        c = view(c0, form)
+        Kn.gemm(ta, tb, c, beta=0.5)
+        check(c, prod + 0.5 * c0, lim)
+    for form in ("rows", "columns", "wide", "one row", "one column"):
+        x = rng.standard_normal((M, N), dtype=np.float32)
+        x = {"one row": np.broadcast_to(x[:1], (M, N)), "one column": np.broadcast_to(x[:, :1], (M, N))}.get(form, x)
+        xd = x.astype(np.float64)
+        for cform in ("rows", "columns"):
+            c = view(c0, cform)
+            Kn.gemm(ta, tb, c, act=Kn.GEMM_ACT_ADD, aux=view(x, form))
+            check(c, prod + xd, lim)
+            c = view(c0, cform)
+            Kn.gemm(ta, tb, c, act=Kn.GEMM_ACT_GELU_BWD, aux=view(x, form))
+            check(c, prod * dgelu(xd), 2 * lim + 2.0 ** -21 * np.abs(prod))
+            if not form.startswith("one"):
+                c, h = view(c0, cform), view(c0, form)
+                Kn.gemm(ta, tb, c, act=Kn.GEMM_ACT_GELU, aux=h)
+                check(h, prod, lim)
+                check(c, gelu(prod), 2 * lim)
+
+
 @pytest.mark.parametrize("sk", [0, 1, 2, 3])
 @pytest.mark.parametrize("side", ["a", "b"])
 def test_gemm_split_near_k_rows(dev, side, sk):
