@@ -33,7 +33,7 @@ HIPCC_FLAGS = [
     "-Wno-unused-function",
     "-Wno-unused-variable",
     # no packed-fp32 instructions: they have produced silent wrong results on
-    # this hardware pool
+    # this hardware
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     f"-I{INCLUDE}",
 ]

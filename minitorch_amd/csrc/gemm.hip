@@ -1443,7 +1443,9 @@ double x3_rounds(int64_t tiles, double w) {
 // 96.7, K = 1536 dX 133.7 -> 126.6; N = 1152 stays (94.7 against 106.8).
 // K is split only when the 128 x 128 tiles leave the CUs idle (weight
 // gradients, K = B*T): into as many ranges as keep one round of kX3Wgs
-// workgroups, each with >= MTX_SPLIT_MINK of K.
+// workgroups, each with >= MTX_SPLIT_MINK of K.  (With at most 64 ranges 128 x
+// 128 x 131072 took 109 us, in its 512, with 34 MB of partials, 58; 128 x 256 x
+// 65536 64 and 48 in 256; 384 x 384 x 131072, 56 ranges, 250 either way.)
 Plan plan_x3(int M, int N, int K, int batch, size_t ws_bytes, bool ak, bool colsum) {
   Plan p{128, 128, 1, K};
   const int64_t t = (int64_t)cdiv(M, 128) * cdiv(N, 128) * batch;

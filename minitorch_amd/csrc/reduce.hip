@@ -6,11 +6,13 @@
 // LayerNorm-parameter gradients, the positional-embedding gradient).
 //
 // The host splits the input's dimensions into kept ("outer", the output) and
-// reduced ones.  Each output element is reduced by one thread walking the
-// reduced index space in a fixed order; when there are few outputs and many
-// reduced elements the reduced range is split into S chunks whose partial
-// results go to the caller's workspace and are combined in chunk order by a
-// second kernel.  No atomics: results are bit-reproducible.
+// reduced ones.  In reduce_kernel four threads reduce an output element, each
+// walking its share of the reduced index space in a fixed order; contiguous
+// runs of 256 values and more have a kernel of their own, a wave or workgroup
+// each.  When there are few outputs and many reduced elements the reduced
+// range is split into S chunks whose partial results go to the caller's
+// workspace and are combined in a fixed order by a second kernel.  No atomics:
+// results are bit-reproducible.
 #include "mtx_common.h"
 
 #include <algorithm>

@@ -426,9 +426,10 @@ __global__ __launch_bounds__(256) void xent_bwd_kernel(const float* __restrict__
   }
 }
 
-// Long rows by workgroup from here on (wave and workgroup, us: 512 x 65536 rows
-// 53 and 57, 700 x 47934 52 and 44, 1024 x 32768 50 and 33, 5003 x 6706 59 and
-// 26, 8192 x 4096 77 and 24; 2048 rows: 5.1 and 4.5 at 512, 54 and 10 at 5003).
+// Long rows by workgroup from here on, where that is ahead for many rows and
+// few (wave and workgroup, us: 512 values x 65536 rows 53 and 57, though 5.1 and
+// 4.5 for 2048 rows; 700 x 47934 52 and 44, x 64 4.6 and 3.2; 1024 x 32768 50 and
+// 33; 5003 x 6706 59 and 26, x 2048 54 and 10; 8192 x 4096 77 and 24).
 constexpr int XENT_MIN = 700;
 int rows_grid(int64_t rows) { return (int)((rows + 3) / 4); }
 
